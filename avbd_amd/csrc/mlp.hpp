@@ -48,11 +48,25 @@ struct WarmIO {
 void launch_gemm_bf16(hipStream_t s, bool ta, bool tb, int epi, const uint16_t* a, int lda, const uint16_t* b,
                       int ldb, float* c32, uint16_t* c16, int ldc, const float* bias, const float* aux, int ldaux,
                       int M, int N, int K);
+// raw batch (rows x 24 features, rows x 3 targets or null) -> normalised x16 and t32
+void launch_stage_batch(hipStream_t s, const float* feat, const float* tgt, const float* norm, int rows, int rows_pad,
+                        uint16_t* x16, float* t32);
+// loss gradient at the output; one squared-error sum per block in loss_part (mlp_loss_parts of them)
 void launch_mse_grad(hipStream_t s, const float* y, const float* t, uint16_t* dy, int rows, int rows_pad, int ld,
-                     int outs, float* loss);
-void launch_colsum(hipStream_t s, const uint16_t* d, int rows, int ld, int cols, float* out);
+                     int outs, float* loss_part);
+int mlp_loss_parts(int rows_pad);
+// weight and bias gradients of every layer (flat parameter layout, layer l at
+// off[l]: W then b) and the loss sum behind them; part holds
+// mlp_grad_chunks(rows_pad) x n_params partial sums
+struct MlpGradIn {
+    const uint16_t* dz[kMlpLayers];
+    const uint16_t* h[kMlpLayers];
+    int off[kMlpLayers];
+};
+int mlp_grad_chunks(int rows_pad);
+void launch_grads(hipStream_t s, const MlpGradIn& in, int rows_pad, int n_params, float* part, const float* loss_part,
+                  float* grads);
 void launch_adam(hipStream_t s, float* w, uint16_t* w16, const float* gw, float* m1, float* m2, int n, float lr,
                  float b1, float b2, float eps, int t);
-void launch_f32_to_bf16(hipStream_t s, const float* x, uint16_t* y, int n);
 
 }  // namespace avbd

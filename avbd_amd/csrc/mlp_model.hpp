@@ -13,7 +13,7 @@ struct MlpModel {
         float* w = nullptr;        // FP32 master, out x in (row-major)
         uint16_t* w16 = nullptr;   // bf16 copy
         float* b = nullptr;
-        float *gw = nullptr, *gb = nullptr;
+        float *gw = nullptr, *gb = nullptr;   // inside `grads`
         float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;   // Adam moments
     };
 
@@ -44,7 +44,7 @@ struct MlpModel {
     hipStream_t stream;
     Layer layers[kMlpLayers];
     float* d_norm = nullptr;
-    float* d_loss = nullptr;
+    float* grads = nullptr;   // every layer's W and b gradient in the flat layout, then the loss sum
     std::vector<float> host_norm;
     bool loaded = false;
     int adam_t = 0;
@@ -56,14 +56,20 @@ struct MlpModel {
     uint16_t* h16[kMlpLayers] = {};
     uint16_t* d16[kMlpLayers] = {};
     float* t32 = nullptr;
+    float* raw_x = nullptr;      // staged raw features and targets
+    float* raw_t = nullptr;
+    float* part = nullptr;       // per row chunk: partial gradients
+    float* loss_part = nullptr;
+    int part_chunks = 0, loss_parts = 0;
 
 private:
     void upload_layer(int l, const float* w, const float* b);
     void zero_adam();
     void stage_batch(const float* feat, const float* tgt, int rows, int rows_pad);
+    void ensure_grad_parts(int rows_pad);
     void backward(int rows, int rows_pad, const uint16_t* x);
     void adam_step(float lr);
-    std::vector<void*> owned, batch_owned;
+    std::vector<void*> owned, batch_owned, part_owned;
 };
 
 }  // namespace avbd

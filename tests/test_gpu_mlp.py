@@ -279,3 +279,31 @@ def test_warm_start_on_the_32_cube_at_its_workload():
            f"prediction kept in {used} of {steps} steps; per step plain {ip} warm {iw}")
     assert np.abs(xw - xp).max() < 1e-3 * bbox(xp)
     assert sum(iw) < sum(ip)
+
+
+@pytest.mark.parametrize("rows", [1, 15, 17, 64, 65, 1000, 4097, 8200])
+def test_mlp_gradients_at_the_edges_of_the_row_chunks(rows):
+    """The gradient kernel stages 64 rows at a time and splits the rows over
+    at most 64 chunks: one row, around one padded strip, around one stage,
+    a ragged last chunk, and chunks of more than one stage (4,097 and 8,200).
+    The numpy restatement rounds the same operands to bf16; a value of dZ or H
+    that falls on a rounding boundary flips by one bf16 ulp (2^-8), which the
+    2 % bound per layer covers as in the test above."""
+    banner(f"gradients, {rows} rows")
+    from avbd_amd.sim import SimulationContext
+    ctx = SimulationContext(dt=1 / 60, solver_iters=1)
+    ctx.add_particles(np.zeros((1, 3)), mass=np.ones(1))
+    ctx.build_graph()
+    ctx.mlp_init(3)
+    rng = np.random.default_rng(rows)
+    X = rng.normal(size=(rows, IN)).astype(np.float32)
+    T = rng.normal(size=(rows, OUT)).astype(np.float32)
+    grads, loss = ctx.mlp_forward_backward(X, T)
+    want, want_loss = reference_grads(ctx.mlp_params(), X, T)
+    got, _ = unpack(np.concatenate([grads, np.zeros(2 * IN + 2 * OUT, np.float32)]))
+    assert abs(loss - want_loss) <= 5e-3 * want_loss
+    for (W, b), (gW, gb) in zip(got, want):
+        assert np.linalg.norm(W - gW) <= 0.02 * np.linalg.norm(gW) + 1e-12
+        assert np.linalg.norm(b - gb) <= 0.02 * np.linalg.norm(gb) + 1e-12
+    again, _ = ctx.mlp_forward_backward(X, T)
+    assert np.array_equal(grads, again)   # sums in a fixed order
