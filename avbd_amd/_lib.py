@@ -37,6 +37,7 @@ FLAG_PERSISTENT = 8
 FLAG_SEPARATE_CHEBYSHEV = 16
 FLAG_FP64_STATE = 32
 FLAG_HOST_COLORING = 64
+FLAG_RESIDENT_ALONE = 128
 
 
 class SceneDesc(C.Structure):

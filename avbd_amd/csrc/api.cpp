@@ -16,6 +16,7 @@
 #include "contacts.hpp"
 #include "internal.hpp"
 #include "mlp_model.hpp"
+#include "resident.hpp"
 #include "lbvh.hpp"
 
 using namespace avbd;
@@ -77,6 +78,11 @@ struct avbd_ctx {
     float4* x_alt = nullptr;
     uint32_t* cheb_list = nullptr;  // particles that are not work items of the last colour
     uint32_t n_cheb = 0;
+    // the resident solve: a whole stretch of iterations per launch from LDS
+    // (positional scenes without conflicts whose patches fit); one launch per
+    // colour phase otherwise
+    bool resident = false;
+    ResidentDev res;
 
     bool timing = false;
     std::vector<hipEvent_t> events;
@@ -180,6 +186,8 @@ void check_status(avbd_ctx* c) {
     uint32_t st = 0;
     hip_check(hipMemcpy(&st, c->d.status, sizeof st, hipMemcpyDeviceToHost), "D2H");
     if (st & 1u) c->nonfinite = true;
+    if (st & 2u)
+        throw CodeError(AVBD_E_HIP, "the resident solve waited too long for a neighbouring patch; the state is not valid");
     if (c->nonfinite) throw CodeError(AVBD_E_NONFINITE, nonfinite_message());
 }
 
@@ -341,6 +349,37 @@ JointRec to_dev(const HostJoint2& h) {
     r.p = h.p[0];
     r.p2 = h.p[1];
     return r;
+}
+
+// Edge constants of a tet (EdgeRec), in FP64 from Q, V lambda, V mu and alpha.
+TetEdges<double> edges_of(const double* Q, double VL, double VM, double alpha) {
+    double q[4][3];
+    for (int j = 0; j < 3; j++) {
+        for (int a = 0; a < 3; a++) q[a][j] = Q[3 * a + j];
+        q[3][j] = -(q[0][j] + q[1][j] + q[2][j]);
+    }
+    const double det = q[0][0] * (q[1][1] * q[2][2] - q[1][2] * q[2][1]) -
+                       q[0][1] * (q[1][0] * q[2][2] - q[1][2] * q[2][0]) +
+                       q[0][2] * (q[1][0] * q[2][1] - q[1][1] * q[2][0]);
+    auto w = [&](int a, int b) { return VM * (q[a][0] * q[b][0] + q[a][1] * q[b][1] + q[a][2] * q[b][2]); };
+    return TetEdges<double>{{w(0, 1), w(0, 2), w(0, 3), w(1, 2), w(1, 3), w(2, 3)}, VL * det * det, VL * det * alpha};
+}
+
+// FP32 state: rounded once from the staged FP64 material.
+TetEdges<float> tet_edges(const HostNH& t) {
+    const TetEdges<double> e = edges_of(t.Q, t.V * t.lambda, t.V * t.mu, t.mu / t.lambda + 1.0);
+    TetEdges<float> f;
+    for (int k = 0; k < 6; k++) f.w[k] = (float)e.w[k];
+    f.h = (float)e.h;
+    f.b = (float)e.b;
+    return f;
+}
+
+// FP64 state: from the device's FP32 record, which defines the model there.
+TetEdges<double> tet_edges(const TetRec& r) {
+    double Q[9];
+    for (int k = 0; k < 9; k++) Q[k] = r.q[k];
+    return edges_of(Q, r.VL, r.VM, r.alpha);
 }
 
 // Append one particle to the FP64 staging pools (ParticlePool::addParticle).
@@ -546,6 +585,10 @@ F64State f64_state(const avbd_ctx* c) {
     return f;
 }
 
+// The step's iterations run in the resident launches: the scene was
+// partitioned at set-up, and with dynamic contacts the step is the static one.
+bool uses_resident(const avbd_ctx* c) { return c->resident && (!c->dynamic || dyn_quiet(c)); }
+
 void enqueue_head(avbd_ctx* c, bool with_events) {
     const float dt = (float)c->desc.dt, g = (float)c->desc.g_accel;
     hipStream_t s = c->stream;
@@ -629,7 +672,15 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
         dz.dyn_off = f0.dyn_off = nullptr;
         dz.dyn_ent = f0.dyn_ent = nullptr;
     }
-    for (uint32_t i = i0; i < i1; i++) {
+    const bool resident = uses_resident(c) && !with_events;
+    if (resident) {
+        double* rr = check ? c->res_rr : nullptr;
+        if (c->fp64)
+            launch_resident_f64(s, c->res, f0, c->damping, c->desc.dt, rc, c->omega_tab + i0, i1 - i0, rr);
+        else
+            launch_resident(s, c->res, dz, c->damping, dt, rc, c->omega_tab + i0, i1 - i0, rr);
+    }
+    for (uint32_t i = i0; i < i1 && !resident; i++) {
         const float omega = c->omega_seq[i];
         const uint32_t j = i - i0;
         const bool odd = (i & 1u) != 0;
@@ -684,7 +735,9 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
     if (check) {
         // an interval has an even number of iterations whenever the step is
         // fused (see avbd_build_graph), so the iterate is back in x
-        if (c->fp64) launch_residual_f64(s, f0, c->cfg, c->damping, c->desc.dt, c->f.x, c->res_rr, c->rc);
+        if (resident) {
+            // |r_v|^2 was left by the launch
+        } else if (c->fp64) launch_residual_f64(s, f0, c->cfg, c->damping, c->desc.dt, c->f.x, c->res_rr, c->rc);
         else launch_residual_pass(s, dz, c->cfg, c->damping, dt, c->rc, c->res_rr);
         launch_residual_decide(s, c->rc, c->res_rr, c->res_scene_off, c->n_res_scenes, c->res_acc_scene,
                                c->res_mg2_scene, c->res_tol * c->res_tol, c->res_check_every, fz);
@@ -692,7 +745,7 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
     hip_check(hipGetLastError(), "kernel launch");
 }
 
-void enqueue_tail(avbd_ctx* c) {
+void enqueue_tail(avbd_ctx* c, bool with_events) {
     const float dt = (float)c->desc.dt, g = (float)c->desc.g_accel;
     hipStream_t s = c->stream;
     const uint32_t iters = c->iters();
@@ -700,7 +753,8 @@ void enqueue_tail(avbd_ctx* c) {
         launch_residual_finish(s, c->rc, scene_freeze(c), c->n_res_scenes, c->d.n_items + c->d.n_oitems);
     // fused: the final positions are in x_alt after an odd number of
     // iterations (never in residual mode, whose intervals are even)
-    if (c->fuse_cheb && (!c->dynamic || dyn_quiet(c)) && !c->rc && (iters & 1u)) {
+    if (c->fuse_cheb && (!c->dynamic || dyn_quiet(c)) && !c->rc && (iters & 1u) &&
+        (with_events || !uses_resident(c))) {
         if (c->fp64) launch_settle_f64(s, c->f.x, c->f.x_alt, c->d.n, nullptr, iters);
         else launch_settle(s, c->d.x, c->x_alt, c->d.n, nullptr, iters);
     }
@@ -728,7 +782,7 @@ void enqueue_step(avbd_ctx* c, bool with_events) {
     } else {
         enqueue_iters(c, with_events, 0, c->iters(), false);
     }
-    enqueue_tail(c);
+    enqueue_tail(c, with_events);
     join_broadphase(c);
 }
 
@@ -779,7 +833,7 @@ void capture_graph(avbd_ctx* c) {
             join_broadphase(c);
         });
         c->interval_exec = capture(c, [&] { enqueue_iters(c, false, 0, every, true); });
-        c->tail_exec = capture(c, [&] { enqueue_tail(c); });
+        c->tail_exec = capture(c, [&] { enqueue_tail(c, false); });
         return;
     }
     c->graph_exec = capture(c, [&] { enqueue_step(c, false); });
@@ -809,7 +863,7 @@ void dyn_residual_graphs(avbd_ctx* c) {
         enqueue_iters(c, false, 0, every, true);
     });
     c->interval_exec = capture(c, [&] { enqueue_iters(c, false, 0, every, true); });
-    c->tail_exec = capture(c, [&] { enqueue_tail(c); });
+    c->tail_exec = capture(c, [&] { enqueue_tail(c, false); });
     c->dyn_graph_key = std::move(key);
 }
 
@@ -845,7 +899,7 @@ void run_residual_step(avbd_ctx* c, bool graphs) {
         hip_check(hipEventRecord(c->part_ev[k], s), "hipEventRecord");
     }
     if (graphs) hip_check(hipGraphLaunch(c->tail_exec, s), "hipGraphLaunch");
-    else enqueue_tail(c);
+    else enqueue_tail(c, false);
 }
 
 // Pinned staging of a detection round's host arrays: reserve the round's
@@ -1146,6 +1200,77 @@ void tune_fusion(avbd_ctx* c) {
     h2d(pll, save.data() + 2 * nx, nx);
     h2d(c->d.ground, save.data() + 3 * nx, ng);
     c->fuse_cheb = t_fused < t_sep;
+}
+
+// Partition the scenes for the resident solve and put the plan on the device.
+// A scene takes it when every patch fits a workgroup's LDS and, since the
+// patches of a scene have to run at once, there are at most as many as CUs
+// (a single tet mesh up to about 36^3 cells in FP64); otherwise, and with
+// AVBD_FLAG_NO_PERSISTENT or AVBD_FLAG_SEPARATE_CHEBYSHEV, every colour phase is
+// a launch of its own.
+void setup_resident(avbd_ctx* c) {
+    if (c->desc.flags & AVBD_FLAG_NO_PERSISTENT) return;
+    hipDeviceProp_t prop;
+    hip_check(hipGetDeviceProperties(&prop, c->device), "hipGetDeviceProperties");
+    std::vector<uint32_t> so = c->scene_offsets;
+    if (so.empty()) so = {0u, c->d.n};
+    HostModel m;
+    m.n = c->d.n;
+    m.nh = &c->nh;
+    m.scene_offsets = &so;
+    uint64_t inc = 0;
+    for (const VItem& it : c->plan.items) inc += it.inc_count;
+    ResidentLimits lim;
+    lim.real_bytes = c->fp64 ? 8u : 4u;
+    lim.damp = c->damping;
+    lim.ground = c->d.n_ground != 0;
+    lim.max_cluster = (uint32_t)prop.multiProcessorCount;
+    lim.lds_bytes = (uint32_t)prop.maxSharedMemoryPerMultiProcessor - 1024u;
+    // a patch below 1000 (about 42 free vertices) costs more in exchange than it
+    // saves in arithmetic: 8^3 and 15^3 steps of 20 iterations take 326 us and 2.27
+    // ms with 1000, 352 us and 2.37 ms with 500
+    lim.target = (uint32_t)std::max<uint64_t>(1000, (inc + lim.max_cluster - 1) / lim.max_cluster);
+    ResidentPlan plan;
+    if (!build_resident(m, c->plan, c->x.data(), lim, plan)) return;
+    ResidentDev& r = c->res;
+    auto put = [&](auto& dst, const auto& src) {
+        using T = std::remove_const_t<std::remove_pointer_t<std::remove_reference_t<decltype(dst)>>>;
+        T* p = dev_alloc<T>(c, src.size() * sizeof(src[0]) / sizeof(T) + 1);
+        if (!src.empty())
+            hip_check(hipMemcpyAsync(p, src.data(), src.size() * sizeof(src[0]), hipMemcpyHostToDevice, c->stream),
+                      "hipMemcpyAsync H2D");
+        dst = p;
+    };
+    put(r.patches, plan.patches);
+    put(r.gid, plan.gid);
+    put(r.tet, plan.tet);
+    put(r.tix, plan.tix);
+    put(r.inc, plan.inc);
+    put(r.item, plan.item);
+    put(r.target, plan.target);
+    put(r.col, plan.col);
+    const size_t words = (size_t)plan.slots * (c->fp64 ? 6 : 3) + 1;
+    const size_t np = plan.patches.size();
+    r.xch = dev_alloc<unsigned long long>(c, words);
+    r.epoch = dev_alloc<uint32_t>(c, np);
+    r.launches = dev_alloc<uint32_t>(c, np);
+    r.sync = dev_alloc<uint32_t>(c, 2 * np);
+    hip_check(hipMemsetAsync(r.xch, 0, words * sizeof(unsigned long long), c->stream), "hipMemsetAsync");
+    hip_check(hipMemsetAsync(r.epoch, 0, np * sizeof(uint32_t), c->stream), "hipMemsetAsync");
+    hip_check(hipMemsetAsync(r.launches, 0, np * sizeof(uint32_t), c->stream), "hipMemsetAsync");
+    hip_check(hipMemsetAsync(r.sync, 0, 2 * np * sizeof(uint32_t), c->stream), "hipMemsetAsync");
+    r.status = c->d.status;
+    r.n_patches = (uint32_t)np;
+    r.n_colors = c->plan.num_colors;
+    r.lds_bytes = plan.lds_bytes;
+    r.max_cluster = plan.max_cluster;
+    resident_shape(plan, c->plan.num_colors, lim, c->desc.lanes_per_vertex, r.lanes, r.block);
+    // 10 ms: what the scene costs alone, so that waiting at most doubles a launch
+    // that another stream's work keeps from being resident
+    r.gather_ticks = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 1000000u;
+    r.has_ground = lim.ground;
+    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    c->resident = true;
 }
 
 }  // namespace
@@ -1916,15 +2041,48 @@ int avbd_build_graph(avbd_ctx* c) {
         upload(c, d.fixed, c->fixed);
         upload(c, d.inc, c->plan.inc);
         {
-            // per-incidence record copies (work-item order) for the vertex solve
+            // per-incidence records (work-item order) for the vertex solve
             if (n >= (1u << 30)) throw std::runtime_error("more than 2^30 particles");
-            std::vector<TetRec> ir(c->plan.inc.size());
-            for (size_t k = 0; k < ir.size(); k++) {
-                ir[k] = tr[c->plan.inc[k] >> 2];
-                ir[k].idx[3] |= (c->plan.inc[k] & 3u) << 30;
+            const std::vector<uint32_t>& inc = c->plan.inc;
+            auto put = [&](auto& rec, const auto& e, size_t k) {
+                const uint32_t t = inc[k] >> 2, a = inc[k] & 3u;
+                for (int j = 0; j < 3; j++) {
+                    rec.w[j] = e.w[kEdgeWeight[a][j]];
+                    rec.i[j] = tr[t].idx[kEdgeCorner[a][j]];
+                }
+                rec.h = e.h;
+                rec.b = e.b;
+            };
+            if (c->damping) {
+                std::vector<TetRec> ir(inc.size());
+                for (size_t k = 0; k < ir.size(); k++) {
+                    ir[k] = tr[inc[k] >> 2];
+                    ir[k].idx[3] |= (inc[k] & 3u) << 30;
+                }
+                d.irec = dev_alloc<TetRec>(c, ir.size());
+                upload(c, d.irec, ir);
+            } else if (c->fp64) {
+                std::vector<TetEdges<double>> te(d.n_tets);
+                for (uint32_t t = 0; t < d.n_tets; t++) te[t] = tet_edges(tr[t]);
+                std::vector<EdgeRec64> er(inc.size());
+                for (size_t k = 0; k < er.size(); k++) put(er[k], te[inc[k] >> 2], k);
+                EdgeRec64* p = dev_alloc<EdgeRec64>(c, er.size());
+                upload(c, p, er);
+                c->f.erec = p;
+                TetEdges<double>* pe = dev_alloc<TetEdges<double>>(c, te.size());
+                upload(c, pe, te);
+                c->res.edges = pe;
+            } else {
+                std::vector<TetEdges<float>> te(d.n_tets);
+                for (uint32_t t = 0; t < d.n_tets; t++) te[t] = tet_edges(c->nh[t]);
+                std::vector<EdgeRec> er(inc.size());
+                for (size_t k = 0; k < er.size(); k++) put(er[k], te[inc[k] >> 2], k);
+                d.erec = dev_alloc<EdgeRec>(c, er.size());
+                upload(c, d.erec, er);
+                TetEdges<float>* pe = dev_alloc<TetEdges<float>>(c, te.size());
+                upload(c, pe, te);
+                c->res.edges = pe;
             }
-            d.irec = dev_alloc<TetRec>(c, ir.size());
-            upload(c, d.irec, ir);
         }
         upload(c, d.items, c->plan.items);
         upload(c, c->d_conflicts, c->plan.conflict_list);
@@ -1975,6 +2133,8 @@ int avbd_build_graph(avbd_ctx* c) {
             double w = 1;
             for (uint32_t i = 0; i < c->iters(); i++) om[i] = (float)(w = omega_at(i, c->desc.iter_acceleration, w));
             c->omega_seq = om;
+            c->omega_tab = dev_alloc<float>(c, om.size());
+            upload(c, c->omega_tab, om);
         }
         d.status = dev_alloc<uint32_t>(c, 1);
         hip_check(hipMemsetAsync(d.status, 0, sizeof(uint32_t), c->stream), "hipMemsetAsync");
@@ -1999,10 +2159,8 @@ int avbd_build_graph(avbd_ctx* c) {
             c->res_scene_off = dev_alloc<uint32_t>(c, so.size());
             c->res_mg2_scene = dev_alloc<double>(c, c->n_res_scenes);
             c->res_acc_scene = dev_alloc<double>(c, c->n_res_scenes);
-            c->omega_tab = dev_alloc<float>(c, c->omega_seq.size());
             upload(c, c->res_scene_off, so);
             upload(c, c->res_mg2_scene, mg2);
-            upload(c, c->omega_tab, c->omega_seq);
             if (c->n_res_scenes > 1) {
                 std::vector<uint32_t> scene_of(n, 0), items(c->n_res_scenes, 0);
                 for (uint32_t sc = 0; sc < c->n_res_scenes; sc++)
@@ -2053,6 +2211,7 @@ int avbd_build_graph(avbd_ctx* c) {
             c->cheb_list = dev_alloc<uint32_t>(c, std::max<size_t>(1, rest.size()));
             if (!rest.empty()) upload(c, c->cheb_list, rest);
             c->fuse_cheb = true;
+            setup_resident(c);
         }
         c->built = true;
 

@@ -1,0 +1,142 @@
+// resident.hpp -- the resident solve: data shared by the host partitioner
+// (resident_host.cpp) and the kernel (resident_kernels.hip).
+//
+// Every scene is cut into patches of neighbouring particles; one workgroup
+// owns a patch, keeps its tets, its particles and a copy of the neighbouring
+// particles (the halo) in LDS, and runs a whole stretch of iterations (every
+// colour phase, Chebyshev step and dual update) in one launch.  The patches of
+// one scene (a cluster) exchange the positions of boundary vertices after
+// each colour through tagged words in device memory.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <vector>
+
+#include "internal.hpp"
+
+namespace avbd {
+
+struct alignas(16) ResidentPatch {
+    uint32_t own, items, local, tets;   // particles owned (the first `items` are work items), own + halo, tets
+    uint32_t inc, targets;              // tet incidences of the items; halo slots they are sent to
+    uint32_t gid_off, tet_off, inc_off, item_off, col_off, target_off;   // into the arrays below
+    uint32_t slot;                      // exchange slot of the first halo particle
+    uint32_t scene;
+    uint32_t first, count;              // the cluster's patches [first, first + count)
+};
+
+// Contact state of an own particle as the iterations need it (GroundRec
+// without k_start, which only the start of a step reads).
+struct alignas(16) ResidentGround {
+    float k_n, k_t, k_b, lambda_n, lambda_t, lambda_b, C_n_prev, mu_s, mu_k, cp_x, cp_z;
+    uint32_t flags;
+};
+
+// LDS layout of a patch, in bytes (the same function sizes the launch and
+// carves the array in the kernel).  Undamped tets: eight arrays of their edge
+// constants (TetEdges; arrays and not records, whose 16- or 32-word stride would
+// put every lane on the same few banks) and 8 bytes per incidence; damped
+// tets: rest shape, E_prev and corners, 2 bytes per incidence.
+struct ResidentLds {
+    uint32_t edge, quad, damp, tix, x, last, lastlast, ym, ground, force, gof, item, target, col, inc, total;
+};
+__host__ __device__ inline ResidentLds resident_lds(uint32_t own, uint32_t items, uint32_t local, uint32_t tets,
+                                                    uint32_t inc, uint32_t targets, uint32_t colors, uint32_t real,
+                                                    bool damp, bool ground) {
+    ResidentLds l;
+    uint32_t at = 0;
+    auto take = [&](uint32_t bytes) {
+        const uint32_t o = at;
+        at += (bytes + 15u) & ~15u;
+        return o;
+    };
+    l.edge = take(damp ? 0u : 8u * real * tets);
+    l.quad = take(damp ? 48u * tets : 0u);
+    l.damp = take(damp ? 32u * tets : 0u);
+    l.tix = take(damp ? 8u * tets : 0u);
+    l.inc = take((damp ? 2u : 8u) * inc);
+    l.x = take(3u * real * local);
+    l.last = take(3u * real * local);
+    l.lastlast = take(3u * real * local);
+    l.ym = take(4u * real * own);
+    l.ground = take(ground ? (uint32_t)sizeof(ResidentGround) * own : 0u);
+    l.force = take(ground ? 3u * real * own : 0u);
+    l.gof = take(ground ? 4u * own : 0u);
+    l.item = take(8u * items);
+    l.target = take(4u * targets);
+    l.col = take(8u * (colors + 1u));
+    l.total = at;
+    return l;
+}
+
+struct ResidentPlan {
+    std::vector<ResidentPatch> patches;
+    std::vector<uint32_t> gid;     // per local particle its global index: own items by colour, other own, then the
+                                   // halo by colour (fixed particles last)
+    std::vector<uint32_t> tet;     // global tet of every patch tet
+    std::vector<uint16_t> tix;     // its four local particles
+    std::vector<uint16_t> inc;     // per incidence, by item in pool order: the three other local particles
+                                   // (kEdgeCorner order) and (patch tet << 2) | corner
+    std::vector<uint32_t> item;    // per item: first incidence | count << 16, first target | count << 16
+    std::vector<uint32_t> target;  // first exchange word of each halo slot that an item's position is sent to
+    std::vector<uint32_t> col;     // per patch: colours + 1 item offsets, colours + 1 halo offsets (local indices)
+    uint32_t slots = 0, lds_bytes = 0, max_cluster = 0;
+};
+
+struct ResidentLimits {
+    uint32_t real_bytes;      // 4 or 8
+    bool damp, ground;
+    uint32_t lds_bytes;       // LDS a workgroup may use
+    uint32_t max_cluster;     // patches of one scene (all must be resident at once)
+    uint32_t target;          // tet incidences per patch aimed at
+};
+
+// Partition every scene (recursive coordinate bisection of `pos`, 3 doubles
+// per particle); false when some scene does not fit the limits.
+bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos, const ResidentLimits& lim,
+                    ResidentPlan& out);
+
+// Lanes per vertex (when not given) and threads of a patch's workgroup.  A phase
+// is one chain of latencies per item, so the lanes grow while the largest phase
+// still has a group for each item in 512 threads: 16 for an undamped vertex (24
+// incidences, then two reads per lane; 32 only adds a reduction step), 32 for a
+// damped one, whose incidence is twice the work.  Step of 20 iterations at 8 / 16 /
+// 32 lanes: 14^3 particles damped 6.2 / 3.9 / 3.2 ms, 15^3 undamped 2.41 / 2.27 /
+// 2.33 ms; 32^3 (35 items per phase, two passes at 16) 2.37 / 2.40 / 2.73 ms.
+// 1024 threads where one phase has more items than 512 threads hold groups
+// (512 scenes: 38.0 -> 34.4 ms; idle wavefronts cost 2.4 -> 3.3 ms at 32^3); FP64
+// stays at 512, where its registers fit.
+void resident_shape(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t given,
+                    uint32_t& lanes, uint32_t& block);
+
+// Device side of the plan plus the state the kernel works on.
+struct ResidentDev {
+    const ResidentPatch* patches = nullptr;
+    const uint32_t* gid = nullptr;
+    const uint32_t* tet = nullptr;
+    const uint2* tix = nullptr;
+    const uint2* inc = nullptr;
+    const uint2* item = nullptr;
+    const uint32_t* target = nullptr;
+    const uint32_t* col = nullptr;
+    const void* edges = nullptr;         // TetEdges of the state's precision per tet (no damping)
+    unsigned long long* xch = nullptr;   // per halo slot 3 (FP32) or 6 (FP64) tagged words
+    uint32_t* epoch = nullptr;           // per patch: exchanges per colour so far (the tag base)
+    uint32_t* launches = nullptr;        // per patch: launches so far
+    uint32_t* sync = nullptr;            // per patch (the cluster's first one): arrivals, decision word
+    uint32_t* status = nullptr;          // = DevState::status
+    uint32_t n_patches = 0, n_colors = 0, lds_bytes = 0, max_cluster = 0, lanes = 8, block = 512;
+    uint32_t gather_ticks = 0;           // 100 MHz ticks a patch waits for its cluster to be resident
+    bool has_ground = false;
+};
+
+// Iterations [iter0, iter0 + iters) of a step (in residual mode iter0 is the
+// control word's counter); rr: |r_v|^2 per particle after the last one, or null.
+void launch_resident(hipStream_t s, const ResidentDev& r, const DevState& d, bool damping, float dt, const ResCtl* rc,
+                     const float* omega_tab, uint32_t iters, double* rr);
+void launch_resident_f64(hipStream_t s, const ResidentDev& r, const F64State& f, bool damping, double dt,
+                         const ResCtl* rc, const float* omega_tab, uint32_t iters, double* rr);
+
+}  // namespace avbd

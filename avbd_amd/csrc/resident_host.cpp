@@ -1,0 +1,263 @@
+// resident_host.cpp -- partition of the scenes into patches for the resident
+// solve (resident.hpp).
+#include <algorithm>
+#include <atomic>
+#include <numeric>
+#include <thread>
+
+#include "resident.hpp"
+
+namespace avbd {
+
+namespace {
+
+constexpr uint32_t NONE = 0xFFFFFFFFu;
+
+// Recursive coordinate bisection: parts [0, parts) of the particles in
+// idx[lo, hi), each cut along the longest side of the box so that the weight
+// divides in proportion to the parts of the two sides.
+void bisect(uint32_t* idx, uint32_t lo, uint32_t hi, uint32_t first, uint32_t parts, const double* pos,
+            const uint32_t* weight, uint32_t base, uint32_t* part) {
+    if (parts <= 1 || hi - lo <= 1) {
+        for (uint32_t k = lo; k < hi; k++) part[idx[k]] = first;
+        return;
+    }
+    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
+    uint64_t total = 0;
+    for (uint32_t k = lo; k < hi; k++) {
+        const double* p = pos + 3 * (size_t)(base + idx[k]);
+        for (int a = 0; a < 3; a++) {
+            mn[a] = std::min(mn[a], p[a]);
+            mx[a] = std::max(mx[a], p[a]);
+        }
+        total += weight[idx[k]];
+    }
+    int axis = 0;
+    for (int a = 1; a < 3; a++)
+        if (mx[a] - mn[a] > mx[axis] - mn[axis]) axis = a;
+    // ties by index, so that the cut does not depend on the sort
+    std::sort(idx + lo, idx + hi, [&](uint32_t a, uint32_t b) {
+        const double pa = pos[3 * (size_t)(base + a) + axis], pb = pos[3 * (size_t)(base + b) + axis];
+        return pa < pb || (pa == pb && a < b);
+    });
+    const uint32_t left = parts / 2;
+    const uint64_t want = total * left / parts;
+    uint64_t sum = 0;
+    uint32_t cut = lo;
+    while (cut < hi && sum + weight[idx[cut]] <= want) sum += weight[idx[cut++]];
+    bisect(idx, lo, cut, first, left, pos, weight, base, part);
+    bisect(idx, cut, hi, first + left, parts - left, pos, weight, base, part);
+}
+
+// One scene's patches (offsets relative to the scene's own arrays).
+bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, const ResidentLimits& lim,
+                 uint32_t scene, ResidentPlan& out) {
+    const uint32_t lo = (*m.scene_offsets)[scene], hi = (*m.scene_offsets)[scene + 1], n = hi - lo;
+    if (n == 0) return true;
+    const uint32_t colors = plan.num_colors;
+    std::vector<uint32_t> weight(n), part(n), order(n);
+    uint64_t total = 0;
+    for (uint32_t v = 0; v < n; v++) {
+        // an item costs its incidences and about eight more (reduction, solve)
+        weight[v] = plan.item_kind[lo + v] == 1 ? plan.item_of[lo + v].inc_count + 8u : 1u;
+        total += weight[v];
+    }
+    uint32_t parts = (uint32_t)std::min<uint64_t>((total + lim.target - 1) / lim.target, lim.max_cluster);
+    parts = std::max(parts, 1u);
+    std::vector<uint32_t> local(n, NONE), stamp(n, NONE);
+    std::vector<uint32_t> tet_stamp, tet_local;
+    std::vector<std::vector<uint32_t>> readers(n);   // halo slots holding a copy of the particle
+    const auto& nh = *m.nh;
+    uint32_t t0 = NONE, t1 = 0;   // the scene's tets lie in [t0, t1]
+    for (uint32_t v = 0; v < n; v++)
+        if (plan.item_kind[lo + v] == 1) {
+            const VItem& it = plan.item_of[lo + v];
+            for (uint32_t k = 0; k < it.inc_count; k++) {
+                const uint32_t t = plan.inc[it.inc_begin + k] >> 2;
+                t0 = std::min(t0, t);
+                t1 = std::max(t1, t);
+            }
+        }
+    const uint32_t n_tets = t0 == NONE ? 0 : t1 - t0 + 1;
+    while (true) {
+        std::iota(order.begin(), order.end(), 0u);
+        bisect(order.data(), 0, n, 0, parts, pos, weight.data(), lo, part.data());
+        out = ResidentPlan{};
+        std::vector<std::vector<uint32_t>> own(parts);
+        for (uint32_t v = 0; v < n; v++) own[part[v]].push_back(v);
+        tet_stamp.assign(n_tets, NONE);
+        tet_local.assign(n_tets, 0);
+        std::fill(stamp.begin(), stamp.end(), NONE);
+        for (auto& r : readers) r.clear();
+        bool fits = true;
+        for (uint32_t q = 0; q < parts; q++) {
+            if (own[q].empty()) continue;
+            auto colour_of = [&](uint32_t v) { return plan.item_kind[lo + v] == 1 ? plan.color[lo + v] : colors; };
+            std::stable_sort(own[q].begin(), own[q].end(),
+                             [&](uint32_t a, uint32_t b) { return colour_of(a) < colour_of(b); });
+            ResidentPatch p{};
+            p.scene = scene;
+            p.own = (uint32_t)own[q].size();
+            p.gid_off = (uint32_t)out.gid.size();
+            p.tet_off = (uint32_t)out.tet.size();
+            p.inc_off = (uint32_t)out.inc.size() / 4;
+            p.item_off = (uint32_t)out.item.size() / 2;
+            p.slot = out.slots;
+            p.col_off = (uint32_t)out.col.size();
+            std::vector<uint32_t> tets, halo;
+            for (uint32_t k = 0; k < p.own; k++) {
+                stamp[own[q][k]] = q;
+                local[own[q][k]] = k;
+            }
+            for (uint32_t v : own[q]) {
+                if (plan.item_kind[lo + v] != 1) break;
+                const VItem& it = plan.item_of[lo + v];
+                const uint32_t begin = (uint32_t)out.inc.size() / 4 - p.inc_off;
+                if (begin + it.inc_count > 0xFFFFu) return false;
+                out.item.push_back(begin | it.inc_count << 16);
+                out.item.push_back(0);
+                p.items++;
+                for (uint32_t k = 0; k < it.inc_count; k++) {
+                    const uint32_t code = plan.inc[it.inc_begin + k], t = code >> 2;
+                    if (tet_stamp[t - t0] != q) {
+                        tet_stamp[t - t0] = q;
+                        tet_local[t - t0] = (uint32_t)tets.size();
+                        tets.push_back(t);
+                        for (uint32_t g : nh[t].idx) {
+                            const uint32_t u = g - lo;
+                            if (stamp[u] == q) continue;
+                            stamp[u] = q;
+                            halo.push_back(u);
+                        }
+                    }
+                    if (tet_local[t - t0] > 0x3FFFu) return false;
+                    // the particles' local indices are known once the halo is complete
+                    for (int j = 0; j < 3; j++) out.inc.push_back(0);
+                    out.inc.push_back((uint16_t)(tet_local[t - t0] << 2 | (code & 3u)));
+                }
+            }
+            std::sort(halo.begin(), halo.end(), [&](uint32_t a, uint32_t b) {
+                const uint32_t ca = colour_of(a), cb = colour_of(b);
+                return ca < cb || (ca == cb && a < b);
+            });
+            p.local = p.own + (uint32_t)halo.size();
+            p.tets = (uint32_t)tets.size();
+            p.inc = (uint32_t)out.inc.size() / 4 - p.inc_off;
+            if (p.local > 0xFFFFu) return false;
+            for (uint32_t k = 0; k < halo.size(); k++) {
+                local[halo[k]] = p.own + k;
+                if (colour_of(halo[k]) < colors) readers[halo[k]].push_back(p.slot + k);
+            }
+            out.slots += (uint32_t)halo.size();
+            for (uint32_t e = p.inc_off; e < p.inc_off + p.inc; e++) {
+                const uint32_t code = out.inc[4 * (size_t)e + 3];
+                for (int j = 0; j < 3; j++)
+                    out.inc[4 * (size_t)e + j] = (uint16_t)local[nh[tets[code >> 2]].idx[kEdgeCorner[code & 3u][j]] - lo];
+            }
+            for (uint32_t v : own[q]) out.gid.push_back(lo + v);
+            for (uint32_t v : halo) out.gid.push_back(lo + v);
+            for (uint32_t t : tets) {
+                out.tet.push_back(t);
+                for (uint32_t g : nh[t].idx) out.tix.push_back((uint16_t)local[g - lo]);
+            }
+            // item and halo ranges per colour
+            uint32_t k = 0;
+            for (uint32_t c = 0; c <= colors; c++) {
+                while (k < p.items && colour_of(own[q][k]) < c) k++;
+                out.col.push_back(k);
+            }
+            k = 0;
+            for (uint32_t c = 0; c <= colors; c++) {
+                while (k < halo.size() && colour_of(halo[k]) < c) k++;
+                out.col.push_back(p.own + k);
+            }
+            out.patches.push_back(p);
+        }
+        for (ResidentPatch& p : out.patches) {
+            p.target_off = (uint32_t)out.target.size();
+            for (uint32_t k = 0; k < p.items; k++) {
+                const auto& r = readers[out.gid[p.gid_off + k] - lo];
+                const uint32_t begin = (uint32_t)out.target.size() - p.target_off;
+                if (begin + r.size() > 0xFFFFu) return false;
+                out.item[2 * (size_t)(p.item_off + k) + 1] = begin | (uint32_t)r.size() << 16;
+                out.target.insert(out.target.end(), r.begin(), r.end());
+            }
+            p.targets = (uint32_t)out.target.size() - p.target_off;
+            const uint32_t bytes = resident_lds(p.own, p.items, p.local, p.tets, p.inc, p.targets, colors,
+                                                lim.real_bytes, lim.damp, lim.ground)
+                                       .total;
+            out.lds_bytes = std::max(out.lds_bytes, bytes);
+            if (bytes > lim.lds_bytes) fits = false;
+        }
+        if (fits) return true;
+        if (parts >= lim.max_cluster || parts >= n) return false;
+        parts = std::min(lim.max_cluster, std::max(parts + 1, parts + parts / 5));
+    }
+}
+
+}  // namespace
+
+bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos, const ResidentLimits& lim,
+                    ResidentPlan& out) {
+    const uint32_t n_scenes = (uint32_t)m.scene_offsets->size() - 1;
+    std::vector<ResidentPlan> scenes(n_scenes);
+    std::atomic<uint32_t> next{0};
+    std::atomic<bool> ok{true};
+    const uint32_t workers = std::min(n_scenes, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+    auto work = [&] {
+        for (uint32_t s; ok && (s = next++) < n_scenes;)
+            if (!build_scene(m, plan, pos, lim, s, scenes[s])) ok = false;
+    };
+    if (workers <= 1) {
+        work();
+    } else {
+        std::vector<std::thread> pool;
+        for (uint32_t w = 0; w < workers; w++) pool.emplace_back(work);
+        for (auto& t : pool) t.join();
+    }
+    if (!ok) return false;
+    out = ResidentPlan{};
+    const uint32_t words = lim.real_bytes == 8 ? 6u : 3u;   // per slot
+    for (const ResidentPlan& s : scenes) {
+        const uint32_t first = (uint32_t)out.patches.size(), count = (uint32_t)s.patches.size();
+        for (ResidentPatch p : s.patches) {
+            p.gid_off += (uint32_t)out.gid.size();
+            p.tet_off += (uint32_t)out.tet.size();
+            p.inc_off += (uint32_t)out.inc.size() / 4;
+            p.item_off += (uint32_t)out.item.size() / 2;
+            p.target_off += (uint32_t)out.target.size();
+            p.slot += out.slots;
+            p.col_off += (uint32_t)out.col.size();
+            p.first = first;
+            p.count = count;
+            out.patches.push_back(p);
+        }
+        out.gid.insert(out.gid.end(), s.gid.begin(), s.gid.end());
+        out.tet.insert(out.tet.end(), s.tet.begin(), s.tet.end());
+        out.tix.insert(out.tix.end(), s.tix.begin(), s.tix.end());
+        out.inc.insert(out.inc.end(), s.inc.begin(), s.inc.end());
+        out.item.insert(out.item.end(), s.item.begin(), s.item.end());
+        out.col.insert(out.col.end(), s.col.begin(), s.col.end());
+        for (uint32_t t : s.target) out.target.push_back((t + out.slots) * words);
+        out.slots += s.slots;
+        out.lds_bytes = std::max(out.lds_bytes, s.lds_bytes);
+        out.max_cluster = std::max(out.max_cluster, count);
+    }
+    return !out.patches.empty() && (uint64_t)out.slots * words < (1u << 28);
+}
+
+void resident_shape(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t given,
+                    uint32_t& lanes, uint32_t& block) {
+    uint32_t most = 0;   // items of one colour in one patch
+    for (const ResidentPatch& p : plan.patches)
+        for (uint32_t c = 0; c < colors; c++)
+            most = std::max(most, plan.col[p.col_off + c + 1] - plan.col[p.col_off + c]);
+    lanes = given;
+    if (!lanes) {
+        lanes = 8;
+        while (lanes < (lim.damp ? 32u : 16u) && 2 * lanes * most <= 512) lanes *= 2;
+    }
+    block = lim.real_bytes == 4 && lanes * most > 512 ? 1024u : 512u;
+}
+
+}  // namespace avbd

@@ -24,26 +24,11 @@
 #include "dyn_device.hpp"
 #include "internal.hpp"
 #include "kernarg.hpp"
+#include "tet_device_f64.hpp"
 #include "warm_device.hpp"
 
 namespace avbd {
 namespace {
-
-struct D3 {
-    double x, y, z;
-};
-__device__ __forceinline__ D3 dd3(double4 v) { return D3{v.x, v.y, v.z}; }
-__device__ __forceinline__ D3 operator-(D3 a, D3 b) { return D3{a.x - b.x, a.y - b.y, a.z - b.z}; }
-__device__ __forceinline__ D3 operator+(D3 a, D3 b) { return D3{a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ D3 operator*(double s, D3 a) { return D3{s * a.x, s * a.y, s * a.z}; }
-__device__ __forceinline__ double dot3(D3 a, D3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ D3 cross3(D3 a, D3 b) {
-    return D3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
-}
-
-struct SymD {
-    double a00, a11, a22, a01, a02, a12;
-};
 
 __device__ __forceinline__ float4 mirror(double4 p) {
     return make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
@@ -57,132 +42,6 @@ __device__ __forceinline__ void load_rec(const TetRec* __restrict__ recs, uint32
     r1 = f[1];
     r2 = f[2];
     r3 = f[3];
-}
-
-// Deformation gradient columns f_c = sum_r d_r Q[r][c] of a record
-// (r1 = q00 q01 q02 q10, r2 = q11 q12 q20 q21, r3 = q22 VL VM alpha).
-__device__ __forceinline__ void deform(D3 p0, D3 p1, D3 p2, D3 p3, float4 r1, float4 r2, float4 r3, D3& f0, D3& f1,
-                                       D3& f2) {
-    const D3 d0 = p0 - p3, d1 = p1 - p3, d2 = p2 - p3;
-    f0 = (double)r1.x * d0 + (double)r1.w * d1 + (double)r2.z * d2;
-    f1 = (double)r1.y * d0 + (double)r2.x * d1 + (double)r2.w * d2;
-    f2 = (double)r1.z * d0 + (double)r2.y * d1 + (double)r3.x * d2;
-}
-
-// One tet incidence of the stable Neo-Hookean energy in FP64
-// (NeoHookeanEnergySolver::accumulate, energy/elastic/NeoHookeanEnergySolver.hpp:121-227):
-// Gauss-Newton hydrostatic term, exact deviatoric term, strain-rate damping.
-template <bool DAMP>
-__device__ __forceinline__ void nh_incidence(D3 p0, D3 p1, D3 p2, D3 p3, float4 r1, float4 r2, float4 r3,
-                                             uint32_t local, const TetDamp* __restrict__ damp, uint32_t t,
-                                             double inv_dt, D3& g, SymD& h) {
-    D3 f0, f1, f2;
-    deform(p0, p1, p2, p3, r1, r2, r3, f0, f1, f2);
-    const double q00 = r1.x, q01 = r1.y, q02 = r1.z, q10 = r1.w, q11 = r2.x, q12 = r2.y, q20 = r2.z, q21 = r2.w,
-                 q22 = r3.x;
-    const double VL = r3.y, VM = r3.z, alpha = r3.w;
-    const D3 c0 = cross3(f1, f2), c1 = cross3(f2, f0), c2 = cross3(f0, f1);
-    const double J = dot3(f0, c0);
-    D3 q;
-    if (local == 0) q = D3{q00, q01, q02};
-    else if (local == 1) q = D3{q10, q11, q12};
-    else if (local == 2) q = D3{q20, q21, q22};
-    else q = D3{-(q00 + q10 + q20), -(q01 + q11 + q21), -(q02 + q12 + q22)};
-    const D3 Fq = q.x * f0 + q.y * f1 + q.z * f2;
-    const D3 Fc = q.x * c0 + q.y * c1 + q.z * c2;
-    const double hyd = VL * (J - alpha);
-    const double q2 = dot3(q, q);
-    g = g + (hyd * Fc + VM * Fq);
-    const double dev = VM * q2;
-    h.a00 += VL * Fc.x * Fc.x + dev;
-    h.a11 += VL * Fc.y * Fc.y + dev;
-    h.a22 += VL * Fc.z * Fc.z + dev;
-    h.a01 += VL * Fc.x * Fc.y;
-    h.a02 += VL * Fc.x * Fc.z;
-    h.a12 += VL * Fc.y * Fc.z;
-    if constexpr (DAMP) {
-        const TetDamp dr = damp[t];
-        const double dm = dr.damp;
-        const double e00 = (0.5 * dot3(f0, f0) - 0.5 - dr.e00) * inv_dt;
-        const double e11 = (0.5 * dot3(f1, f1) - 0.5 - dr.e11) * inv_dt;
-        const double e22 = (0.5 * dot3(f2, f2) - 0.5 - dr.e22) * inv_dt;
-        const double e01 = (0.5 * dot3(f0, f1) - dr.e01) * inv_dt;
-        const double e02 = (0.5 * dot3(f0, f2) - dr.e02) * inv_dt;
-        const double e12 = (0.5 * dot3(f1, f2) - dr.e12) * inv_dt;
-        const D3 Eq = D3{e00 * q.x + e01 * q.y + e02 * q.z, e01 * q.x + e11 * q.y + e12 * q.z,
-                         e02 * q.x + e12 * q.y + e22 * q.z};
-        const D3 FEq = Eq.x * f0 + Eq.y * f1 + Eq.z * f2;
-        g = g + dm * FEq;
-        const double diag = dm * dot3(q, Eq);
-        const double a = 0.5 * dm * inv_dt;
-        const double ff00 = f0.x * f0.x + f1.x * f1.x + f2.x * f2.x;
-        const double ff11 = f0.y * f0.y + f1.y * f1.y + f2.y * f2.y;
-        const double ff22 = f0.z * f0.z + f1.z * f1.z + f2.z * f2.z;
-        const double ff01 = f0.x * f0.y + f1.x * f1.y + f2.x * f2.y;
-        const double ff02 = f0.x * f0.z + f1.x * f1.z + f2.x * f2.z;
-        const double ff12 = f0.y * f0.z + f1.y * f1.z + f2.y * f2.z;
-        h.a00 += diag + a * (q2 * ff00 + Fq.x * Fq.x);
-        h.a11 += diag + a * (q2 * ff11 + Fq.y * Fq.y);
-        h.a22 += diag + a * (q2 * ff22 + Fq.z * Fq.z);
-        h.a01 += a * (q2 * ff01 + Fq.x * Fq.y);
-        h.a02 += a * (q2 * ff02 + Fq.x * Fq.z);
-        h.a12 += a * (q2 * ff12 + Fq.y * Fq.z);
-    }
-}
-
-// Ground AL contact (CollisionConstraintEnergySolver::accumulate<3> with the
-// ground constraint, energy/collision/GroundCollisionEnergySolver.hpp:27-60).
-__device__ __forceinline__ void ground_accumulate(const GroundRec& c, D3 p, D3& g, SymD& h) {
-    const double Cn = -p.y, Ct = p.x - (double)c.cp_x, Cb = p.z - (double)c.cp_z;
-    const double Ccorr = Cn - (double)kAlpha * c.C_n_prev;
-    const double lnp = fmax(0.0, (double)c.k_n * Ccorr + c.lambda_n);
-    double lt = (double)c.k_t * Ct + c.lambda_t;
-    double lb = (double)c.k_b * Cb + c.lambda_b;
-    const double mag = sqrt(lt * lt + lb * lb);
-    const double mu = (c.flags & GF_USE_STATIC) ? c.mu_s : c.mu_k;
-    const double lmax = mu * lnp;
-    if (mag > lmax) {
-        const double nrm = mag + 1e-8;
-        lt = lt / nrm * lmax;
-        lb = lb / nrm * lmax;
-    }
-    g.x += lt;
-    g.y += -lnp;
-    g.z += lb;
-    h.a00 += c.k_t;
-    h.a11 += c.k_n;
-    h.a22 += c.k_b;
-}
-
-// Dual + stiffness-ramp update of one ground record at the extrapolated
-// position (CollisionConstraintEnergySolver::updateAfterIteration,
-// energy/collision/CollisionConstraintEnergySolver.hpp:60-134).
-__device__ __forceinline__ void ground_dual_update(GroundRec& c, D3 xp) {
-    const double Cn = -xp.y, Ct = xp.x - (double)c.cp_x, Cb = xp.z - (double)c.cp_z;
-    const double Ccorr = Cn - (double)kAlpha * c.C_n_prev;
-    const double lnp = (double)c.k_n * Ccorr + c.lambda_n;
-    const double ltp = (double)c.k_t * Ct + c.lambda_t;
-    const double lbp = (double)c.k_b * Cb + c.lambda_b;
-    if (lnp > 0.0) c.k_n = (float)(c.k_n + (double)kBeta * fabs(Ccorr));
-    const double ln = fmax(0.0, lnp);
-    c.lambda_n = (float)ln;
-    const double mag = sqrt(ltp * ltp + lbp * lbp);
-    double lmax = ((c.flags & GF_USE_STATIC) ? c.mu_s : c.mu_k) * ln;
-    if (mag < lmax) {
-        c.k_t = (float)(c.k_t + (double)kBeta * fabs(Ct));
-        c.k_b = (float)(c.k_b + (double)kBeta * fabs(Cb));
-        c.lambda_t = (float)ltp;
-        c.lambda_b = (float)lbp;
-        c.flags |= GF_UNCLAMPED;
-    } else {
-        if (c.flags & GF_USE_STATIC) {
-            c.flags &= ~GF_USE_STATIC;
-            lmax = c.mu_k * lnp;
-        }
-        c.lambda_t = (float)(ltp / (mag + 1e-8) * lmax);
-        c.lambda_b = (float)(lbp / (mag + 1e-8) * lmax);
-        c.flags &= ~GF_UNCLAMPED;
-    }
 }
 
 // Vertex-triangle contact (the only dynamic kind with the FP64 state, where
@@ -237,76 +96,49 @@ __device__ __forceinline__ void dyn_terms(const uint32_t* __restrict__ off, cons
     }
 }
 
-__device__ __forceinline__ D3 ldlt3(const SymD& A, D3 b) {
-    const double d0 = A.a00;
-    const double l10 = A.a01 / d0, l20 = A.a02 / d0;
-    const double d1 = A.a11 - l10 * A.a01;
-    const double l21 = (A.a12 - l20 * A.a01) / d1;
-    const double d2 = A.a22 - l20 * A.a02 - l21 * l21 * d1;
-    const double z0 = b.x;
-    const double z1 = b.y - l10 * z0;
-    const double z2 = b.z - l20 * z0 - l21 * z1;
-    const double x2 = z2 / d2;
-    const double x1 = z1 / d1 - l21 * x2;
-    const double x0 = z0 / d0 - l10 * x1 - l20 * x2;
-    return D3{x0, x1, x2};
-}
-
-template <int L>
-__device__ __forceinline__ double group_sum(double v) {
-#pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
 __device__ __forceinline__ uint32_t xcd_logical_block() {
     const uint32_t b = blockIdx.x, G = gridDim.x;
     const uint32_t x = b % 8u, q = b / 8u;
     return x * (G / 8u) + min(x, G % 8u) + q;
 }
 
+template <bool DAMP>
+__host__ __device__ __forceinline__ const typename Inc64<DAMP>::Rec* inc_records(const F64State& f) {
+    if constexpr (DAMP) return f.irec;
+    else return f.erec;
+}
+
 // Sum of the tet incidences of one work item over its L lanes (every lane
 // gets the sums); U incidences per lane are gathered at once (records, then
 // positions with the next records in flight), summed in incidence order.
+// xa: the item's own position.
 template <int L, int U, bool DAMP, bool HESS>
 __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, const uint32_t* __restrict__ inc,
-                                              const TetRec* __restrict__ irec, const TetDamp* __restrict__ damp,
-                                              const double4* x, double inv_dt, D3& g, SymD& h) {
-    const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT;
+                                              const typename Inc64<DAMP>::Rec* __restrict__ irec,
+                                              const TetDamp* __restrict__ damp, const double4* x, D3 xa,
+                                              double inv_dt, D3& g, SymD& h) {
+    using Inc = Inc64<DAMP>;
+    const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT, base = it.inc_begin;
     g = D3{0.0, 0.0, 0.0};
     h = SymD{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    uint4 idx[U];
-    float4 r1[U], r2[U], r3[U];
+    Inc cur[U];
 #pragma unroll
     for (int u = 0; u < U; u++)
-        if (lane + u * L < cnt) load_rec(irec, it.inc_begin + lane + u * L, idx[u], r1[u], r2[u], r3[u]);
+        if (lane + u * L < cnt) cur[u].load(irec, base + lane + u * L);
     for (uint32_t j0 = lane; j0 < cnt; j0 += U * L) {
-        D3 P[U][4];
+        typename Inc::Pos P[U];
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (j0 + u * L < cnt) {
-                P[u][0] = dd3(x[idx[u].x]);
-                P[u][1] = dd3(x[idx[u].y]);
-                P[u][2] = dd3(x[idx[u].z]);
-                P[u][3] = dd3(x[idx[u].w & 0x3fffffffu]);
-            }
-        uint4 nidx[U];
-        float4 n1[U], n2[U], n3[U];
+            if (j0 + u * L < cnt) P[u] = cur[u].gather(x);
+        Inc next[U];
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (j0 + (U + u) * L < cnt) load_rec(irec, it.inc_begin + j0 + (U + u) * L, nidx[u], n1[u], n2[u], n3[u]);
+            if (j0 + (U + u) * L < cnt) next[u].load(irec, base + j0 + (U + u) * L);
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (j0 + u * L < cnt)
-                nh_incidence<DAMP>(P[u][0], P[u][1], P[u][2], P[u][3], r1[u], r2[u], r3[u], idx[u].w >> 30, damp,
-                                   DAMP ? (inc[it.inc_begin + j0 + u * L] >> 2) : 0u, inv_dt, g, h);
+            if (j0 + u * L < cnt) cur[u].add(P[u], xa, damp, DAMP ? (inc[base + j0 + u * L] >> 2) : 0u, inv_dt, g, h);
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            idx[u] = nidx[u];
-            r1[u] = n1[u];
-            r2[u] = n2[u];
-            r3[u] = n3[u];
-        }
+        for (int u = 0; u < U; u++) cur[u] = next[u];
     }
     g.x = group_sum<L>(g.x);
     g.y = group_sum<L>(g.y);
@@ -327,13 +159,7 @@ __device__ __forceinline__ double4 item_solve(const VItem& it, double4 xv, doubl
                                               SymD h, double inv_dt2) {
     const D3 p = dd3(xv);
     if (it.ground >= 0) ground_accumulate(gr, p, g, h);
-    const double md = xv.w * inv_dt2;
-    h.a00 += md;
-    h.a11 += md;
-    h.a22 += md;
-    const D3 b = D3{-md * (p.x - yv.x) - g.x, -md * (p.y - yv.y) - g.y, -md * (p.z - yv.z) - g.z};
-    const D3 dx = ldlt3(h, b);
-    return make_double4(p.x + dx.x, p.y + dx.y, p.z + dx.z, xv.w);
+    return block_step(xv, yv, g, h, inv_dt2);
 }
 
 // One colour phase (_solveParticle<3>, simulation/VBDSolver.hpp:285-449,487-510).
@@ -350,7 +176,7 @@ struct DynF64 {
 template <int L, bool DAMP, int U, bool DYN = false>
 __global__ __launch_bounds__(256) void solve_color_f64_kernel(const VItem* __restrict__ items, uint32_t n_items,
                                                               const uint32_t* __restrict__ inc,
-                                                              const TetRec* __restrict__ irec,
+                                                              const typename Inc64<DAMP>::Rec* __restrict__ irec,
                                                               const TetDamp* __restrict__ damp, double4* x,
                                                               const double4* __restrict__ y,
                                                               const GroundRec* __restrict__ ground, double4* x_out,
@@ -367,17 +193,17 @@ __global__ __launch_bounds__(256) void solve_color_f64_kernel(const VItem* __res
     const VItem it = items[item];   // in flight with the converged flag's load
     if (done && *done) return;      // residual target reached earlier in this step
     if (frozen && frozen[scene_of[it.v]]) return;   // the item's scene has converged in this step
-    double4 xv = make_double4(0.0, 0.0, 0.0, 0.0), yv = xv;
+    const double4 xv = x[it.v];
+    double4 yv = make_double4(0.0, 0.0, 0.0, 0.0);
     GroundRec gr{};
     const bool lead = lane == 0;
     if (lead) {
-        xv = x[it.v];
         yv = y[it.v];
         if (it.ground >= 0) gr = ground[it.ground];
     }
     D3 g;
     SymD h;
-    item_gradient<L, U, DAMP, true>(it, lane, inc, irec, damp, x, inv_dt, g, h);
+    item_gradient<L, U, DAMP, true>(it, lane, inc, irec, damp, x, dd3(xv), inv_dt, g, h);
     if (!lead) return;
     if constexpr (DYN) {
         // static energies (tets, ground) first, then the dynamic contacts
@@ -409,7 +235,7 @@ __global__ __launch_bounds__(256) void solve_cheb_f64_kernel(F64State f, const V
                                                              const double4* __restrict__ x_cur, double4* x_next,
                                                              float omega, const ResCtl* rc, const float* omega_tab,
                                                              uint32_t j, double inv_dt, double inv_dt2) {
-    kernarg_prefetch(f.inc, f.irec, f.damp, f.y, f.ground, f.x_last, f.x_lastlast, f.ground_of, f.frozen, f.scene_of,
+    kernarg_prefetch(f.inc, f.irec, f.erec, f.damp, f.y, f.ground, f.x_last, f.x_lastlast, f.ground_of, f.frozen, f.scene_of,
                      items, n_items, sx, cx, cheb_list, n_cheb, x_cur, x_next, rc, inv_dt, inv_dt2, blockDim.x);
     const uint32_t xcd = blockIdx.x % 8u, q = blockIdx.x / 8u;
     if (q < sx) {
@@ -424,18 +250,18 @@ __global__ __launch_bounds__(256) void solve_cheb_f64_kernel(F64State f, const V
             if (lane == 0) x_next[v] = x_cur[v];
             return;
         }
-        double4 xv = make_double4(0.0, 0.0, 0.0, 0.0), yv = xv, xll = xv;
+        const double4 xv = x_cur[v];
+        double4 yv = make_double4(0.0, 0.0, 0.0, 0.0), xll = yv;
         GroundRec gr{};
         const bool lead = lane == 0;
         if (lead) {
-            xv = x_cur[v];
             yv = f.y[v];
             xll = f.x_lastlast[v];
             if (it.ground >= 0) gr = f.ground[it.ground];
         }
         D3 g;
         SymD h;
-        item_gradient<L, U, DAMP, true>(it, lane, f.inc, f.irec, f.damp, x_cur, inv_dt, g, h);
+        item_gradient<L, U, DAMP, true>(it, lane, f.inc, inc_records<DAMP>(f), f.damp, x_cur, dd3(xv), inv_dt, g, h);
         if (!lead) return;
         const double4 xs = item_solve(it, xv, yv, gr, g, h, inv_dt2);
         const double4 xp = make_double4(w * (xs.x - xll.x) + xll.x, w * (xs.y - xll.y) + xll.y,
@@ -607,7 +433,7 @@ __global__ __launch_bounds__(256) void residual_f64_kernel(F64State f, const VIt
                                                            uint32_t n_items, const double4* __restrict__ x,
                                                            double* __restrict__ rr, const ResCtl* rc, double inv_dt,
                                                            double inv_dt2) {
-    kernarg_prefetch(f.inc, f.irec, f.damp, f.y, f.ground, f.frozen, f.scene_of, f.dyn_off, items, n_items, x, rr, rc,
+    kernarg_prefetch(f.inc, f.irec, f.erec, f.damp, f.y, f.ground, f.frozen, f.scene_of, f.dyn_off, items, n_items, x, rr, rc,
                      inv_dt, inv_dt2, blockDim.x);
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t item = tid / L, lane = tid % L;
@@ -617,9 +443,10 @@ __global__ __launch_bounds__(256) void residual_f64_kernel(F64State f, const VIt
     if (f.frozen && f.frozen[f.scene_of[it.v]]) return;   // keeps the residual it converged with
     D3 g;
     SymD h;
-    item_gradient<L, 1, DAMP, false>(it, lane, f.inc, f.irec, f.damp, x, inv_dt, g, h);
+    const double4 xv = x[it.v];
+    item_gradient<L, 1, DAMP, false>(it, lane, f.inc, inc_records<DAMP>(f), f.damp, x, dd3(xv), inv_dt, g, h);
     if (lane != 0) return;
-    const double4 xv = x[it.v], yv = f.y[it.v];
+    const double4 yv = f.y[it.v];
     if (it.ground >= 0) ground_accumulate(f.ground[it.ground], dd3(xv), g, h);
     if (f.dyn_off) dyn_terms(f.dyn_off, f.dyn_ent, f.dyn, x, it.v, g, h);
     const double md = xv.w * inv_dt2;
@@ -678,9 +505,10 @@ __global__ __launch_bounds__(256) void stats_f64_kernel(F64State f, const VItem*
         const VItem it = items[item];
         D3 g;
         SymD h;
-        item_gradient<L, 1, DAMP, false>(it, lane, f.inc, f.irec, f.damp, f.x, inv_dt, g, h);
+        const double4 xv = f.x[it.v];
+        item_gradient<L, 1, DAMP, false>(it, lane, f.inc, inc_records<DAMP>(f), f.damp, f.x, dd3(xv), inv_dt, g, h);
         if (lane == 0) {
-            const double4 xv = f.x[it.v], yv = f.y[it.v];
+            const double4 yv = f.y[it.v];
             if (it.ground >= 0) ground_accumulate(f.ground[it.ground], dd3(xv), g, h);
             if (f.dyn_off) dyn_terms(f.dyn_off, f.dyn_ent, f.dyn, f.x, it.v, g, h);
             const double md = xv.w * inv_dt2;
@@ -890,13 +718,13 @@ void launch_solve_color_f64(hipStream_t s, const F64State& f, const LaunchCfg& c
     const dim3 grid(blocks_for(count * L, block)), blk(block);
     const double inv_dt = 1.0 / dt, inv_dt2 = inv_dt * inv_dt;
 #define AVBD_F64_LAUNCH(LL, DD, UU)                                                                                  \
-    hipLaunchKernelGGL((solve_color_f64_kernel<LL, DD, UU>), grid, blk, 0, s, f.items + begin, count, f.inc, f.irec, \
+    hipLaunchKernelGGL((solve_color_f64_kernel<LL, DD, UU>), grid, blk, 0, s, f.items + begin, count, f.inc, inc_records<DD>(f), \
                        f.damp, f.x, f.y, f.ground, x_out, inv_dt, inv_dt2, done, f.frozen, f.scene_of, DynF64{})
     // with dynamic contacts: one incidence gathered per lane at a time
 #define AVBD_F64_U(LL, DD)                                                                                         \
     if (f.dyn_off)                                                                                                 \
         hipLaunchKernelGGL((solve_color_f64_kernel<LL, DD, 1, true>), grid, blk, 0, s, f.items + begin, count,    \
-                           f.inc, f.irec, f.damp, f.x, f.y, f.ground, x_out, inv_dt, inv_dt2, done, f.frozen,      \
+                           f.inc, inc_records<DD>(f), f.damp, f.x, f.y, f.ground, x_out, inv_dt, inv_dt2, done, f.frozen,      \
                            f.scene_of, DynF64{f.dyn_off, f.dyn_ent, f.dyn, f.x_buf});                               \
     else if (cfg.batch >= 4) AVBD_F64_LAUNCH(LL, DD, 4);                                                           \
     else if (cfg.batch >= 2) AVBD_F64_LAUNCH(LL, DD, 2);                                                           \

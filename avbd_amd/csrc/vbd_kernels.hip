@@ -22,105 +22,12 @@
 #include "kernarg.hpp"
 #include "dyn_device.hpp"
 #include "rigid_device.hpp"
+#include "tet_device.hpp"
 #include "warm_device.hpp"
 
 namespace avbd {
 
 namespace {
-
-struct Sym3 {
-    float a00, a11, a22, a01, a02, a12;
-};
-
-__device__ __forceinline__ float3 f3(float4 v) { return make_float3(v.x, v.y, v.z); }
-__device__ __forceinline__ float3 operator-(float3 a, float3 b) { return make_float3(a.x - b.x, a.y - b.y, a.z - b.z); }
-__device__ __forceinline__ float3 operator+(float3 a, float3 b) { return make_float3(a.x + b.x, a.y + b.y, a.z + b.z); }
-__device__ __forceinline__ float3 operator*(float s, float3 a) { return make_float3(s * a.x, s * a.y, s * a.z); }
-__device__ __forceinline__ float dot3(float3 a, float3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ float3 cross3(float3 a, float3 b) {
-    return make_float3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
-}
-
-// Load a 64-byte tet record with four 16-byte loads.
-__device__ __forceinline__ void load_tet(const TetRec* __restrict__ tets, uint32_t t, uint4& idx, float4& r1,
-                                         float4& r2, float4& r3) {
-    const uint4* p = reinterpret_cast<const uint4*>(tets + t);
-    idx = p[0];
-    const float4* f = reinterpret_cast<const float4*>(p);
-    r1 = f[1];
-    r2 = f[2];
-    r3 = f[3];
-}
-
-// One tet incidence of the stable Neo-Hookean energy
-// (NeoHookeanEnergySolver::accumulate, energy/elastic/NeoHookeanEnergySolver.hpp:121-227).
-// q = Q.row(local) for local < 3, -(Q.row0 + Q.row1 + Q.row2) for local 3 (the
-// reference's sign = -1 folded into q; every term is linear in q or quadratic).
-// The record (idx, r1..r3) is already loaded; t indexes the damping record.
-// nh_incidence_pos takes the four vertex positions already gathered.
-template <bool DAMP>
-__device__ __forceinline__ void nh_incidence_pos(float3 p0, float3 p1, float3 p2, float3 p3, float4 r1, float4 r2,
-                                                 float4 r3, uint32_t local, const TetDamp* __restrict__ damp,
-                                                 uint32_t t, float inv_dt, float3& g, Sym3& h) {
-    // r1 = q00 q01 q02 q10 ; r2 = q11 q12 q20 q21 ; r3 = q22 VL VM alpha
-    const float3 d0 = p0 - p3, d1 = p1 - p3, d2 = p2 - p3;
-    const float q00 = r1.x, q01 = r1.y, q02 = r1.z, q10 = r1.w, q11 = r2.x, q12 = r2.y, q20 = r2.z, q21 = r2.w,
-                q22 = r3.x;
-    const float VL = r3.y, VM = r3.z, alpha = r3.w;
-    // F = D Q: column c of F = d0 Q[0][c] + d1 Q[1][c] + d2 Q[2][c]
-    const float3 f0 = q00 * d0 + q10 * d1 + q20 * d2;
-    const float3 f1 = q01 * d0 + q11 * d1 + q21 * d2;
-    const float3 f2 = q02 * d0 + q12 * d1 + q22 * d2;
-    const float3 c0 = cross3(f1, f2), c1 = cross3(f2, f0), c2 = cross3(f0, f1);
-    const float J = dot3(f0, c0);
-    float3 q;
-    if (local == 0) q = make_float3(q00, q01, q02);
-    else if (local == 1) q = make_float3(q10, q11, q12);
-    else if (local == 2) q = make_float3(q20, q21, q22);
-    else q = make_float3(-(q00 + q10 + q20), -(q01 + q11 + q21), -(q02 + q12 + q22));
-    const float3 Fq = q.x * f0 + q.y * f1 + q.z * f2;
-    const float3 Fc = q.x * c0 + q.y * c1 + q.z * c2;
-    const float hyd = VL * (J - alpha);
-    const float q2 = dot3(q, q);
-    g = g + (hyd * Fc + VM * Fq);
-    const float dev = VM * q2;
-    h.a00 += VL * Fc.x * Fc.x + dev;
-    h.a11 += VL * Fc.y * Fc.y + dev;
-    h.a22 += VL * Fc.z * Fc.z + dev;
-    h.a01 += VL * Fc.x * Fc.y;
-    h.a02 += VL * Fc.x * Fc.z;
-    h.a12 += VL * Fc.y * Fc.z;
-    if constexpr (DAMP) {
-        const TetDamp dr = damp[t];
-        const float dm = dr.damp;
-        // Edot = (0.5 F^T F - 0.5 I - E_prev) / dt, symmetric
-        const float e00 = (0.5f * dot3(f0, f0) - 0.5f - dr.e00) * inv_dt;
-        const float e11 = (0.5f * dot3(f1, f1) - 0.5f - dr.e11) * inv_dt;
-        const float e22 = (0.5f * dot3(f2, f2) - 0.5f - dr.e22) * inv_dt;
-        const float e01 = (0.5f * dot3(f0, f1) - dr.e01) * inv_dt;
-        const float e02 = (0.5f * dot3(f0, f2) - dr.e02) * inv_dt;
-        const float e12 = (0.5f * dot3(f1, f2) - dr.e12) * inv_dt;
-        const float3 Eq = make_float3(e00 * q.x + e01 * q.y + e02 * q.z, e01 * q.x + e11 * q.y + e12 * q.z,
-                                      e02 * q.x + e12 * q.y + e22 * q.z);
-        const float3 FEq = Eq.x * f0 + Eq.y * f1 + Eq.z * f2;
-        g = g + dm * FEq;
-        const float diag = dm * dot3(q, Eq);
-        const float a = 0.5f * dm * inv_dt;
-        // F F^T rows: (F F^T)_ij = sum_c F_ic F_jc
-        const float ff00 = f0.x * f0.x + f1.x * f1.x + f2.x * f2.x;
-        const float ff11 = f0.y * f0.y + f1.y * f1.y + f2.y * f2.y;
-        const float ff22 = f0.z * f0.z + f1.z * f1.z + f2.z * f2.z;
-        const float ff01 = f0.x * f0.y + f1.x * f1.y + f2.x * f2.y;
-        const float ff02 = f0.x * f0.z + f1.x * f1.z + f2.x * f2.z;
-        const float ff12 = f0.y * f0.z + f1.y * f1.z + f2.y * f2.z;
-        h.a00 += diag + a * (q2 * ff00 + Fq.x * Fq.x);
-        h.a11 += diag + a * (q2 * ff11 + Fq.y * Fq.y);
-        h.a22 += diag + a * (q2 * ff22 + Fq.z * Fq.z);
-        h.a01 += a * (q2 * ff01 + Fq.x * Fq.y);
-        h.a02 += a * (q2 * ff02 + Fq.x * Fq.z);
-        h.a12 += a * (q2 * ff12 + Fq.y * Fq.z);
-    }
-}
 
 template <bool DAMP>
 __device__ __forceinline__ void nh_incidence_rec(const float4* x, uint4 idx, float4 r1, float4 r2, float4 r3,
@@ -138,46 +45,6 @@ __device__ __forceinline__ void nh_incidence(const float4* x, const TetRec* __re
     float4 r1, r2, r3;
     load_tet(tets, e >> 2, idx, r1, r2, r3);
     nh_incidence_rec<DAMP>(x, idx, r1, r2, r3, e & 3u, damp, e >> 2, inv_dt, g, h);
-}
-
-// Incidence k of the work-item order, read from the per-incidence copy of
-// the tet records (contiguous for an item's lanes, no index indirection);
-// the local vertex index sits in the top two bits of idx.w.
-template <bool DAMP>
-__device__ __forceinline__ void nh_incidence_k(const float4* x, const TetRec* __restrict__ irec,
-                                               const uint32_t* __restrict__ inc, const TetDamp* __restrict__ damp,
-                                               uint32_t k, float inv_dt, float3& g, Sym3& h) {
-    uint4 idx;
-    float4 r1, r2, r3;
-    load_tet(irec, k, idx, r1, r2, r3);
-    const uint32_t local = idx.w >> 30;
-    idx.w &= 0x3fffffffu;
-    nh_incidence_rec<DAMP>(x, idx, r1, r2, r3, local, damp, DAMP ? (inc[k] >> 2) : 0u, inv_dt, g, h);
-}
-
-// Ground AL contact contribution (CollisionConstraintEnergySolver::accumulate<3>,
-// energy/collision/CollisionConstraintEnergySolver.hpp:180-285 with the ground
-// constraint of energy/collision/GroundCollisionEnergySolver.hpp:27-60).
-__device__ __forceinline__ void ground_accumulate(const GroundRec& c, float3 p, float3& g, Sym3& h) {
-    const float Cn = -p.y, Ct = p.x - c.cp_x, Cb = p.z - c.cp_z;
-    const float Ccorr = Cn - kAlpha * c.C_n_prev;
-    const float lnp = fmaxf(0.0f, c.k_n * Ccorr + c.lambda_n);
-    float lt = c.k_t * Ct + c.lambda_t;
-    float lb = c.k_b * Cb + c.lambda_b;
-    const float mag = sqrtf(lt * lt + lb * lb);
-    const float mu = (c.flags & GF_USE_STATIC) ? c.mu_s : c.mu_k;
-    const float lmax = mu * lnp;
-    if (mag > lmax) {
-        const float nrm = mag + 1e-8f;
-        lt = lt / nrm * lmax;
-        lb = lb / nrm * lmax;
-    }
-    g.x += lt;
-    g.y += -lnp;
-    g.z += lb;
-    h.a00 += c.k_t;
-    h.a11 += c.k_n;
-    h.a22 += c.k_b;
 }
 
 // Dynamic contacts incident to one positional particle (the reference
@@ -203,29 +70,6 @@ __device__ __forceinline__ void dyn_add3(const DynArgs& a, const float4* x, uint
     }
 }
 
-// Solve (m/dt^2 I + H) dx = b for symmetric positive definite H by LDL^T.
-__device__ __forceinline__ float3 ldlt3(const Sym3& A, float3 b) {
-    const float d0 = A.a00;
-    const float l10 = A.a01 / d0, l20 = A.a02 / d0;
-    const float d1 = A.a11 - l10 * A.a01;
-    const float l21 = (A.a12 - l20 * A.a01) / d1;
-    const float d2 = A.a22 - l20 * A.a02 - l21 * l21 * d1;
-    const float z0 = b.x;
-    const float z1 = b.y - l10 * z0;
-    const float z2 = b.z - l20 * z0 - l21 * z1;
-    const float x2 = z2 / d2;
-    const float x1 = z1 / d1 - l21 * x2;
-    const float x0 = z0 / d0 - l10 * x1 - l20 * x2;
-    return make_float3(x0, x1, x2);
-}
-
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
-}
-
 // Workgroups are dispatched round-robin over the 8 XCDs (block b -> XCD b % 8),
 // each with its own L2.  Remap so that XCD x runs a contiguous range of
 // logical blocks: work items are ordered by vertex index, i.e. spatially, so
@@ -237,71 +81,40 @@ __device__ __forceinline__ uint32_t xcd_logical_block() {
     return x * (G / 8u) + min(x, G % 8u) + q;
 }
 
-// A lane's incidences in batches of U (j0, j0 + L, ..., j0 + (U-1) L, those
-// < cnt): a batch's records are loaded together, then its vertex positions
-// together with the next batch's records, then its terms are accumulated in
-// incidence order -- the same order and arithmetic as one incidence at a
-// time, with fewer dependent memory round trips and the next records in
-// flight during the arithmetic.
-template <int U>
-struct IncBatch {
-    uint4 idx[U];
-    float4 r1[U], r2[U], r3[U];
-};
-
-template <int L, int U>
-__device__ __forceinline__ void load_inc_batch(const TetRec* __restrict__ irec, uint32_t base, uint32_t j0,
-                                               uint32_t cnt, IncBatch<U>& b) {
-#pragma unroll
-    for (int u = 0; u < U; u++)
-        if (j0 + u * L < cnt) load_tet(irec, base + j0 + u * L, b.idx[u], b.r1[u], b.r2[u], b.r3[u]);
-}
-
-template <int L, int U, bool DAMP>
-__device__ __forceinline__ void nh_incidences_batch(const float4* x, const TetRec* __restrict__ irec,
-                                                    const uint32_t* __restrict__ inc,
-                                                    const TetDamp* __restrict__ damp, uint32_t base, uint32_t j0,
-                                                    uint32_t cnt, float inv_dt, float3& g, Sym3& h,
-                                                    IncBatch<U>& cur) {
-    const uint4* idx = cur.idx;
-    const float4 *r1 = cur.r1, *r2 = cur.r2, *r3 = cur.r3;
-    float3 P[U][4];
-#pragma unroll
-    for (int u = 0; u < U; u++)
-        if (j0 + u * L < cnt) {
-            P[u][0] = f3(x[idx[u].x]);
-            P[u][1] = f3(x[idx[u].y]);
-            P[u][2] = f3(x[idx[u].z]);
-            P[u][3] = f3(x[idx[u].w & 0x3fffffffu]);
-        }
-    IncBatch<U> next;
-    if (j0 + U * L < cnt) load_inc_batch<L, U>(irec, base, j0 + U * L, cnt, next);
-#pragma unroll
-    for (int u = 0; u < U; u++)
-        if (j0 + u * L < cnt)
-            nh_incidence_pos<DAMP>(P[u][0], P[u][1], P[u][2], P[u][3], r1[u], r2[u], r3[u], idx[u].w >> 30, damp,
-                                   DAMP ? (inc[base + j0 + u * L] >> 2) : 0u, inv_dt, g, h);
-    cur = next;
-}
-
 // The tet incidences of one work item summed over the L lanes of its group
-// (every lane gets the sums; every lane of the group must call it).  U > 1
-// gathers U incidences of a lane at once (nh_incidences_batch).
+// (every lane gets the sums; every lane of the group must call it).  A lane
+// takes its incidences (lane, lane + L, ...) in batches of U: a batch's records
+// are loaded together, then its vertex positions together with the next
+// batch's records, then its terms are added in incidence order -- the same
+// order and arithmetic as one at a time, with fewer dependent memory round trips.
+// xa: the item's own position.
 template <int L, bool DAMP, int U>
 __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, const uint32_t* __restrict__ inc,
-                                              const TetRec* __restrict__ irec, const TetDamp* __restrict__ damp,
-                                              const float4* x, float inv_dt, float3& g, Sym3& h) {
-    const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT;
+                                              const typename Inc32<DAMP>::Rec* __restrict__ irec,
+                                              const TetDamp* __restrict__ damp, const float4* x, float3 xa,
+                                              float inv_dt, float3& g, Sym3& h) {
+    using Inc = Inc32<DAMP>;
+    const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT, base = it.inc_begin;
     g = make_float3(0.f, 0.f, 0.f);
     h = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if constexpr (U > 1) {
-        IncBatch<U> cur;
-        if (lane < cnt) load_inc_batch<L, U>(irec, it.inc_begin, lane, cnt, cur);
-        for (uint32_t j0 = lane; j0 < cnt; j0 += U * L)
-            nh_incidences_batch<L, U, DAMP>(x, irec, inc, damp, it.inc_begin, j0, cnt, inv_dt, g, h, cur);
-    } else {
-        for (uint32_t j = lane; j < cnt; j += L)
-            nh_incidence_k<DAMP>(x, irec, inc, damp, it.inc_begin + j, inv_dt, g, h);
+    Inc cur[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (lane + u * L < cnt) cur[u].load(irec, base + lane + u * L);
+    for (uint32_t j0 = lane; j0 < cnt; j0 += U * L) {
+        typename Inc::Pos P[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (j0 + u * L < cnt) P[u] = cur[u].gather(x);
+        Inc next[U];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (j0 + (U + u) * L < cnt) next[u].load(irec, base + j0 + (U + u) * L);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (j0 + u * L < cnt) cur[u].add(P[u], xa, damp, DAMP ? (inc[base + j0 + u * L] >> 2) : 0u, inv_dt, g, h);
+#pragma unroll
+        for (int u = 0; u < U; u++) cur[u] = next[u];
     }
     g.x = group_sum<L>(g.x);
     g.y = group_sum<L>(g.y);
@@ -316,42 +129,42 @@ __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, co
 
 // The group leader's part of the vertex block solve: ground AL terms,
 // dynamic contacts, inertia, and the 3x3 solve; returns the new position.
+template <bool DAMP>
+__host__ __device__ __forceinline__ const typename Inc32<DAMP>::Rec* inc_records(const DevState& d) {
+    if constexpr (DAMP) return d.irec;
+    else return d.erec;
+}
+
 template <bool DYN>
 __device__ __forceinline__ float4 item_solve(const VItem& it, float4 xv, float4 yv, const GroundRec& gr, float3 g,
                                              Sym3 h, const float4* x, const DynArgs& da, float inv_dt2) {
     const float3 p = f3(xv);
     if (it.ground >= 0) ground_accumulate(gr, p, g, h);
     if constexpr (DYN) dyn_add3(da, x, it.v, g, h);
-    const float md = xv.w * inv_dt2;   // m / dt^2
-    h.a00 += md;
-    h.a11 += md;
-    h.a22 += md;
-    const float3 b = make_float3(-md * (p.x - yv.x) - g.x, -md * (p.y - yv.y) - g.y, -md * (p.z - yv.z) - g.z);
-    const float3 dx = ldlt3(h, b);
-    return make_float4(p.x + dx.x, p.y + dx.y, p.z + dx.z, xv.w);
+    return block_step(xv, yv, g, h, inv_dt2);
 }
 
 // One vertex block solve (_solveParticle<3>, simulation/VBDSolver.hpp:285-449,487-510)
 // by the L lanes of a group; every lane of the group must call it.
 template <int L, bool DAMP, bool DYN = false, int U = 1>
 __device__ __forceinline__ void solve_item(const VItem& it, uint32_t lane, const uint32_t* __restrict__ inc,
-                                           const TetRec* __restrict__ irec, const TetDamp* __restrict__ damp,
-                                           float4* x, const float4* __restrict__ y,
+                                           const typename Inc32<DAMP>::Rec* __restrict__ irec,
+                                           const TetDamp* __restrict__ damp, float4* x, const float4* __restrict__ y,
                                            const GroundRec* __restrict__ ground, float4* x_out, float4* x_buf,
                                            float inv_dt, float inv_dt2, const DynArgs& da) {
     // the group leader's own state is loaded first, so that its latency
     // overlaps the incidence gathers instead of following the reduction
-    float4 xv = make_float4(0.f, 0.f, 0.f, 0.f), yv = xv;
+    const float4 xv = x[it.v];
+    float4 yv = make_float4(0.f, 0.f, 0.f, 0.f);
     GroundRec gr{};
     const bool lead = lane == 0;
     if (lead) {
-        xv = x[it.v];
         yv = y[it.v];
         if (it.ground >= 0) gr = ground[it.ground];
     }
     float3 g;
     Sym3 h;
-    item_gradient<L, DAMP, U>(it, lane, inc, irec, damp, x, inv_dt, g, h);
+    item_gradient<L, DAMP, U>(it, lane, inc, irec, damp, x, f3(xv), inv_dt, g, h);
     if (!lead) return;
     const float4 nx = item_solve<DYN>(it, xv, yv, gr, g, h, x, da, inv_dt2);
     if (it.inc_count & VITEM_CONFLICT) x_buf[it.v] = nx;
@@ -361,7 +174,7 @@ __device__ __forceinline__ void solve_item(const VItem& it, uint32_t lane, const
 template <int L, bool DAMP, bool DYN, int U>
 __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_color_kernel(const VItem* __restrict__ items, uint32_t n_items,
                                                            const uint32_t* __restrict__ inc,
-                                                           const TetRec* __restrict__ irec,
+                                                           const typename Inc32<DAMP>::Rec* __restrict__ irec,
                                                            const TetDamp* __restrict__ damp, float4* x,
                                                            const float4* __restrict__ y,
                                                            const GroundRec* __restrict__ ground, float4* x_out,
@@ -531,43 +344,6 @@ __global__ void commit_kernel(DevState d, const uint32_t* __restrict__ list, uin
     if (k < count) commit_one(d, list[k]);
 }
 
-// _particleChebyshevAcceleration (VBDSolver.hpp:513-536) of one position.
-__device__ __forceinline__ float4 cheb_apply(float4 xp, float4 xll, float omega) {
-    xp.x = omega * (xp.x - xll.x) + xll.x;
-    xp.y = omega * (xp.y - xll.y) + xll.y;
-    xp.z = omega * (xp.z - xll.z) + xll.z;
-    return xp;
-}
-
-// CollisionConstraintEnergySolver::updateAfterIteration (CollisionConstraintEnergySolver.hpp:60-134)
-// of one ground record at the extrapolated position xp.
-__device__ __forceinline__ void ground_dual_update(GroundRec& c, float4 xp) {
-    const float Cn = -xp.y, Ct = xp.x - c.cp_x, Cb = xp.z - c.cp_z;
-    const float Ccorr = Cn - kAlpha * c.C_n_prev;
-    const float lnp = c.k_n * Ccorr + c.lambda_n;
-    const float ltp = c.k_t * Ct + c.lambda_t;
-    const float lbp = c.k_b * Cb + c.lambda_b;
-    if (lnp > 0.f) c.k_n += kBeta * fabsf(Ccorr);
-    c.lambda_n = fmaxf(0.f, lnp);
-    const float mag = sqrtf(ltp * ltp + lbp * lbp);
-    float lmax = ((c.flags & GF_USE_STATIC) ? c.mu_s : c.mu_k) * c.lambda_n;
-    if (mag < lmax) {
-        c.k_t += kBeta * fabsf(Ct);
-        c.k_b += kBeta * fabsf(Cb);
-        c.lambda_t = ltp;
-        c.lambda_b = lbp;
-        c.flags |= GF_UNCLAMPED;
-    } else {
-        if (c.flags & GF_USE_STATIC) {
-            c.flags &= ~GF_USE_STATIC;
-            lmax = c.mu_k * lnp;
-        }
-        c.lambda_t = ltp / (mag + 1e-8f) * lmax;
-        c.lambda_b = lbp / (mag + 1e-8f) * lmax;
-        c.flags &= ~GF_UNCLAMPED;
-    }
-}
-
 // Chebyshev step (positions and orientations) and the dual / stiffness update
 // of the particle's contact and joint records; the position is read from
 // x_in and written to x_out (the same buffer unless the step is fused into
@@ -629,7 +405,7 @@ __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_cheb_kernel(
     DevState d, const VItem* __restrict__ items, uint32_t n_items, uint32_t sx, uint32_t cx,
     const uint32_t* __restrict__ cheb_list, uint32_t n_cheb, float4* __restrict__ x_next, float omega_fixed,
     const ResCtl* rc, const float* __restrict__ omega_tab, uint32_t j, float inv_dt, float inv_dt2) {
-    kernarg_prefetch(d.x, d.y, d.x_last, d.x_lastlast, d.ground, d.ground_of, d.inc, d.irec, d.damp, d.frozen,
+    kernarg_prefetch(d.x, d.y, d.x_last, d.x_lastlast, d.ground, d.ground_of, d.inc, d.irec, d.erec, d.damp, d.frozen,
                      d.scene_of, items, n_items, sx, cx, cheb_list, n_cheb, x_next, rc, inv_dt, inv_dt2, blockDim.x);
     const uint32_t xcd = blockIdx.x % 8u, q = blockIdx.x / 8u;
     if (q < sx) {
@@ -644,11 +420,11 @@ __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_cheb_kernel(
             if (lane == 0) x_next[v] = d.x[v];
             return;
         }
-        float4 xv = make_float4(0.f, 0.f, 0.f, 0.f), yv = xv, xl = xv, xll = xv;
+        const float4 xv = d.x[v];
+        float4 yv = make_float4(0.f, 0.f, 0.f, 0.f), xl = yv, xll = yv;
         GroundRec gr{};
         const bool lead = lane == 0;
         if (lead) {
-            xv = d.x[v];
             yv = d.y[v];
             xl = d.x_last[v];
             xll = d.x_lastlast[v];
@@ -656,7 +432,7 @@ __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_cheb_kernel(
         }
         float3 g;
         Sym3 h;
-        item_gradient<L, DAMP, U>(it, lane, d.inc, d.irec, d.damp, d.x, inv_dt, g, h);
+        item_gradient<L, DAMP, U>(it, lane, d.inc, inc_records<DAMP>(d), d.damp, d.x, f3(xv), inv_dt, g, h);
         if (!lead) return;
         const float4 xp = cheb_apply(item_solve<false>(it, xv, yv, gr, g, h, d.x, DynArgs{}, inv_dt2), xll, omega);
         x_next[v] = xp;
@@ -809,15 +585,12 @@ __global__ __launch_bounds__(256) void solve_ocolor_kernel(DevState d, uint32_t 
 template <int L, bool DAMP>
 __device__ __forceinline__ float residual_item(const VItem& it, uint32_t lane, const DevState& d, float inv_dt,
                                                float inv_dt2) {
-    const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT;
-    float3 g = make_float3(0.f, 0.f, 0.f);
-    Sym3 h = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (uint32_t j = lane; j < cnt; j += L) nh_incidence_k<DAMP>(d.x, d.irec, d.inc, d.damp, it.inc_begin + j, inv_dt, g, h);
-    g.x = group_sum<L>(g.x);
-    g.y = group_sum<L>(g.y);
-    g.z = group_sum<L>(g.z);
+    const float4 xv = d.x[it.v];
+    float3 g;
+    Sym3 h;
+    item_gradient<L, DAMP, 1>(it, lane, d.inc, inc_records<DAMP>(d), d.damp, d.x, f3(xv), inv_dt, g, h);
     if (lane != 0) return 0.f;
-    const float4 xv = d.x[it.v], yv = d.y[it.v];
+    const float4 yv = d.y[it.v];
     if (it.ground >= 0) ground_accumulate(d.ground[it.ground], f3(xv), g, h);
     const float md = xv.w * inv_dt2;
     const float rx = md * (xv.x - yv.x) + g.x, ry = md * (xv.y - yv.y) + g.y, rz = md * (xv.z - yv.z) + g.z;
@@ -1392,7 +1165,7 @@ void solve_dispatch(hipStream_t s, const DevState& d, uint32_t block, uint32_t b
     const uint32_t threads = count * L;
     const dim3 grid(blocks_for(threads, block)), blk(block);
 #define AVBD_SOLVE_ARGS \
-    d.items + begin, count, d.inc, d.irec, d.damp, d.x, d.y, d.ground, x_out, d.x_buf, 1.0f / dt, 1.0f / (dt * dt), \
+    d.items + begin, count, d.inc, inc_records<DAMP>(d), d.damp, d.x, d.y, d.ground, x_out, d.x_buf, 1.0f / dt, 1.0f / (dt * dt), \
         done, dyn_args(d), d.frozen, d.scene_of
     if (block > 256) batch = 1;   // the batched variants are built for blocks of <= 256 threads
     if (d.dyn_off) hipLaunchKernelGGL((solve_color_kernel<L, DAMP, true, 1>), grid, blk, 0, s, AVBD_SOLVE_ARGS);

@@ -56,7 +56,7 @@ class SimulationContext:
                  iter_acceleration: float = 0.95, particle_capacity: int = 0, energy_capacity: int = 0,
                  device: int = 0, lanes_per_vertex: int = 0, block_size: int = 0, use_graph: bool = True,
                  serial_broadphase: bool = False, separate_chebyshev: bool = False, gather_batch: int = 0,
-                 fp64_state: bool = False, host_coloring: bool = False):
+                 fp64_state: bool = False, host_coloring: bool = False, flags: int = 0):
         desc = _lib.SceneDesc()
         desc.particle_capacity = particle_capacity
         desc.energy_capacity = energy_capacity
@@ -67,7 +67,8 @@ class SimulationContext:
         desc.flags = ((0 if use_graph else _lib.FLAG_NO_GRAPH) | (_lib.FLAG_SERIAL_BROADPHASE if serial_broadphase else 0)
                       | (_lib.FLAG_SEPARATE_CHEBYSHEV if separate_chebyshev else 0)
                       | (_lib.FLAG_FP64_STATE if fp64_state else 0)
-                      | (_lib.FLAG_HOST_COLORING if host_coloring else 0))
+                      | (_lib.FLAG_HOST_COLORING if host_coloring else 0)
+                      | flags)
         desc.device = device
         desc.lanes_per_vertex = lanes_per_vertex
         desc.block_size = block_size
@@ -582,14 +583,14 @@ class Simulation:
     def __init__(self, scene: Scene, device: int = 0, lanes_per_vertex: int = 0, block_size: int = 0,
                  use_graph: bool = True, serial_broadphase: bool = False,
                  residual_target: Optional[tuple] = None, separate_chebyshev: bool = False, gather_batch: int = 0,
-                 fp64_state: bool = False, host_coloring: bool = False):
+                 fp64_state: bool = False, host_coloring: bool = False, flags: int = 0):
         self.scene = scene
         self.ctx = SimulationContext(dt=scene.dt, g_accel=scene.g, solver_iters=scene.iters,
                                      iter_acceleration=scene.rho, device=device,
                                      lanes_per_vertex=lanes_per_vertex, block_size=block_size,
                                      use_graph=use_graph, serial_broadphase=serial_broadphase,
                                      separate_chebyshev=separate_chebyshev, gather_batch=gather_batch,
-                                     fp64_state=fp64_state, host_coloring=host_coloring)
+                                     fp64_state=fp64_state, host_coloring=host_coloring, flags=flags)
         self.solver = VBDSolver(self.ctx, scene.iters, scene.rho)
         if residual_target is not None:
             self.ctx.set_residual_target(*residual_target)

@@ -61,9 +61,15 @@ typedef enum {
 
 /* ---- context creation flags ---- */
 #define AVBD_FLAG_NO_GRAPH 1u    /* launch kernels eagerly instead of replaying a hipGraph */
-#define AVBD_FLAG_NO_PERSISTENT 4u  /* one kernel launch per solver phase (the default) */
-#define AVBD_FLAG_PERSISTENT 8u     /* rejected by avbd_create (AVBD_E_ARG): the persistent step
-                                       kernel was removed.  Every grid barrier needed agent-scope
+#define AVBD_FLAG_NO_PERSISTENT 4u  /* one kernel launch per solver phase also where the resident solve
+                                       (all iterations of a stretch in one launch, each patch of the mesh
+                                       in one workgroup's LDS) would run; the results are identical for the
+                                       same lanes_per_vertex */
+#define AVBD_FLAG_RESIDENT_ALONE 128u /* for tests: the resident solve takes its path for a device that
+                                         cannot hold all patches of a scene at once (one workgroup per
+                                         scene runs all of its patches; identical results) */
+#define AVBD_FLAG_PERSISTENT 8u     /* rejected by avbd_create (AVBD_E_ARG): a step kernel
+                                       with grid barriers was removed.  Every barrier needed agent-scope
                                        release / acquire fences, which write back and invalidate
                                        the L2 of every XCD, so on MI355X one launch per phase
                                        replayed from a hipGraph was 25x faster */

@@ -1,0 +1,80 @@
+"""The resident solve (every iteration of a stretch in one launch, the patches
+of a scene in the LDS of workgroups that exchange boundary positions) equals
+one launch per phase bit for bit at the same lanes per vertex, whatever the
+partition: scenes of one patch and of many, patches of odd sizes, particles
+without a free neighbour, damping, ground contacts, batches of scenes of
+different sizes, odd iteration counts, and the path for a device that cannot
+hold a scene's patches at once."""
+import numpy as np
+import pytest
+
+from avbd_amd import _lib, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def scene_of(kind, n):
+    if kind == "hang":
+        sc = scenes.hanging_cube(n=n)
+    elif kind == "damped":
+        sc = scenes.dropped_cube(n=n, height=0.01)
+        for m in sc.meshes:
+            m.kd = 1e-3
+    elif kind == "batch":
+        sc = scenes.cube_batch(n_scenes=n, n_min=1, n_max=9)
+        for m in sc.meshes:
+            m.rest[:, 1] += 0.01 - m.rest[:, 1].min()
+    else:
+        sc = scenes.dropped_cube(n=n, height=0.01)
+    return sc
+
+
+# a single cell, a cube below one patch, just above it, tens of patches, ragged
+# ones; lanes below and above the number of 32-bit pieces of a position
+CASES = [("hang", 1, 8), ("hang", 2, 4), ("drop", 5, 16), ("drop", 6, 32), ("drop", 13, 8), ("damped", 3, 8),
+         ("damped", 9, 32), ("batch", 7, 8), ("batch", 40, 4)]
+
+
+@pytest.mark.parametrize("fp64", [False, True])
+@pytest.mark.parametrize("kind,n,lanes", CASES)
+def test_resident_equals_one_launch_per_phase(kind, n, lanes, fp64):
+    from avbd_amd.sim import Simulation
+    print(f"[gpu-test] resident {kind} {n} lanes {lanes} fp64 {fp64}", flush=True)
+    sc = scene_of(kind, n)
+    sc.iters = 7
+    kw = dict(fp64_state=fp64, lanes_per_vertex=lanes, block_size=128)
+    runs = [Simulation(sc, flags=f, **kw)
+            for f in (_lib.FLAG_NO_PERSISTENT, 0, _lib.FLAG_RESIDENT_ALONE, _lib.FLAG_NO_GRAPH)]
+    for r in runs:
+        r.setup()
+    for k in range(3):
+        for r in runs:
+            r.update(3)
+        x0, v0 = runs[0].ctx.state()
+        assert np.isfinite(x0).all()
+        for j, r in enumerate(runs[1:]):
+            x, v = r.ctx.state()
+            assert np.array_equal(x, x0) and np.array_equal(v, v0), (k, j)
+    if kind != "hang":
+        ref = bytes(runs[0].ctx.ground_records())
+        assert all(bytes(r.ctx.ground_records()) == ref for r in runs[1:])
+
+
+@pytest.mark.parametrize("kind,n,check", [("drop", 6, 1), ("drop", 7, 5), ("batch", 9, 3)])
+def test_resident_stops_where_one_launch_per_phase_stops(kind, n, check):
+    """Residual target: the same iteration counts, residuals and positions,
+    with scenes of a batch that stop at different checks."""
+    from avbd_amd.sim import Simulation
+    print(f"[gpu-test] resident residual {kind} {n} every {check}", flush=True)
+    sc = scene_of(kind, n)
+    kw = dict(fp64_state=True, lanes_per_vertex=8, block_size=128, residual_target=(1e-4, 203, check))
+    runs = [Simulation(sc, flags=f, **kw) for f in (_lib.FLAG_NO_PERSISTENT, 0, _lib.FLAG_RESIDENT_ALONE)]
+    for r in runs:
+        r.setup()
+        r.update(4)
+    s0, h0 = runs[0].ctx.stats(), runs[0].ctx.residual_history()
+    for r in runs[1:]:
+        s = r.ctx.stats()
+        assert (s.iterations_total, s.last_step_iterations) == (s0.iterations_total, s0.last_step_iterations)
+        assert np.array_equal(r.ctx.residual_history(), h0)
+        assert np.array_equal(r.positions(), runs[0].positions())
