@@ -83,6 +83,7 @@ struct avbd_ctx {
     // colour phase otherwise
     bool resident = false;
     ResidentDev res;
+    ResidentCheck res_check;   // residual mode: the check intervals of a resident launch
 
     bool timing = false;
     std::vector<hipEvent_t> events;
@@ -648,7 +649,8 @@ void enqueue_head(avbd_ctx* c, bool with_events) {
 
 // Iterations [i0, i1) of a step.  With `check` (residual mode: i0 = 0,
 // i1 = res_check_every) the Chebyshev weights come from the device table and
-// a residual check follows the last iteration.
+// a residual check follows the last iteration; a resident launch runs up to
+// intervals_per_launch() such intervals.
 void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool check) {
     const float dt = (float)c->desc.dt;
     hipStream_t s = c->stream;
@@ -674,11 +676,12 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
     }
     const bool resident = uses_resident(c) && !with_events;
     if (resident) {
-        double* rr = check ? c->res_rr : nullptr;
-        if (c->fp64)
-            launch_resident_f64(s, c->res, f0, c->damping, c->desc.dt, rc, c->omega_tab + i0, i1 - i0, rr);
-        else
-            launch_resident(s, c->res, dz, c->damping, dt, rc, c->omega_tab + i0, i1 - i0, rr);
+        ResidentCheck chk;
+        if (check) chk = c->res_check;
+        chk.every = i1 - i0;
+        if (c->fp64) launch_resident_f64(s, c->res, f0, c->damping, c->desc.dt, rc, c->omega_tab + i0, chk);
+        else launch_resident(s, c->res, dz, c->damping, dt, rc, c->omega_tab + i0, chk);
+        if (check) launch_residual_collect(s, c->rc, chk, c->res_acc_scene, c->n_res_scenes, fz);
     }
     for (uint32_t i = i0; i < i1 && !resident; i++) {
         const float omega = c->omega_seq[i];
@@ -732,12 +735,10 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
         launch_joint2_dual(s, dz, done);   // oriented particles: never fused
         if (n_active) launch_dyn_dual(s, c->d, d_active, n_active, done);
     }
-    if (check) {
+    if (check && !resident) {
         // an interval has an even number of iterations whenever the step is
         // fused (see avbd_build_graph), so the iterate is back in x
-        if (resident) {
-            // |r_v|^2 was left by the launch
-        } else if (c->fp64) launch_residual_f64(s, f0, c->cfg, c->damping, c->desc.dt, c->f.x, c->res_rr, c->rc);
+        if (c->fp64) launch_residual_f64(s, f0, c->cfg, c->damping, c->desc.dt, c->f.x, c->res_rr, c->rc);
         else launch_residual_pass(s, dz, c->cfg, c->damping, dt, c->rc, c->res_rr);
         launch_residual_decide(s, c->rc, c->res_rr, c->res_scene_off, c->n_res_scenes, c->res_acc_scene,
                                c->res_mg2_scene, c->res_tol * c->res_tol, c->res_check_every, fz);
@@ -771,14 +772,19 @@ void enqueue_tail(avbd_ctx* c, bool with_events) {
     hip_check(hipGetLastError(), "kernel launch");
 }
 
+// Launches of check intervals that the budget of a step takes.
+uint32_t interval_launches(avbd_ctx* c) {
+    const uint32_t intervals = c->iters() / c->res_check_every, per = uses_resident(c) ? c->res_check.per_launch : 1u;
+    return (intervals + per - 1) / per;
+}
+
 // One whole step at the fixed iteration count (or, in residual mode, the
 // eager form: every interval with its check, the done flag turning the rest
 // into no-ops).
 void enqueue_step(avbd_ctx* c, bool with_events) {
     enqueue_head(c, with_events);
     if (c->rc) {
-        for (uint32_t k = 0; k < c->iters() / c->res_check_every; k++)
-            enqueue_iters(c, false, 0, c->res_check_every, true);
+        for (uint32_t k = 0; k < interval_launches(c); k++) enqueue_iters(c, false, 0, c->res_check_every, true);
     } else {
         enqueue_iters(c, with_events, 0, c->iters(), false);
     }
@@ -876,7 +882,7 @@ void dyn_residual_graphs(avbd_ctx* c) {
 // sequence is launched eagerly.
 void run_residual_step(avbd_ctx* c, bool graphs) {
     constexpr uint32_t kAhead = 2;
-    const uint32_t intervals = c->iters() / c->res_check_every;
+    const uint32_t intervals = interval_launches(c);
     hipStream_t s = c->stream;
     for (uint32_t k = 0; k < intervals; k++) {
         if (k >= kAhead) {
@@ -1255,6 +1261,24 @@ void setup_resident(avbd_ctx* c) {
     r.epoch = dev_alloc<uint32_t>(c, np);
     r.launches = dev_alloc<uint32_t>(c, np);
     r.sync = dev_alloc<uint32_t>(c, 2 * np);
+    r.sums = dev_alloc<unsigned long long>(c, 4 * np);
+    hip_check(hipMemsetAsync(r.sums, 0, 4 * np * sizeof(unsigned long long), c->stream), "hipMemsetAsync");
+    if (c->rc) {
+        // About 100 iterations per launch: a launch costs some 50 us (loading the
+        // patches, the handshake, recording the checks, the gap) against 1.4 ms for
+        // 100 iterations at 32^3, and one that runs much longer keeps other streams'
+        // work off the CUs.
+        ResidentCheck& k = c->res_check;
+        k.total = c->res_max_iters / c->res_check_every;
+        k.per_launch = std::max(1u, std::min(k.total, 100u / c->res_check_every));
+        k.per_scene = c->n_res_scenes > 1;
+        k.tol2 = c->res_tol * c->res_tol;
+        k.mg2 = c->res_mg2_scene;
+        k.hist = dev_alloc<double>(c, (size_t)k.per_launch * c->n_res_scenes);
+        k.ran = dev_alloc<uint32_t>(c, c->n_res_scenes);
+        hip_check(hipMemsetAsync(k.ran, 0, c->n_res_scenes * sizeof(uint32_t), c->stream), "hipMemsetAsync");
+        hip_check(hipMemsetAsync(c->res_acc_scene, 0, c->n_res_scenes * sizeof(double), c->stream), "hipMemsetAsync");
+    }
     hip_check(hipMemsetAsync(r.xch, 0, words * sizeof(unsigned long long), c->stream), "hipMemsetAsync");
     hip_check(hipMemsetAsync(r.epoch, 0, np * sizeof(uint32_t), c->stream), "hipMemsetAsync");
     hip_check(hipMemsetAsync(r.launches, 0, np * sizeof(uint32_t), c->stream), "hipMemsetAsync");
@@ -2196,8 +2220,9 @@ int avbd_build_graph(avbd_ctx* c) {
         // without oriented particles or conflicted vertices)
         // (residual mode: with an even check interval, so that every interval
         // starts on the same buffer and one interval graph serves them all)
-        if (!(c->desc.flags & AVBD_FLAG_SEPARATE_CHEBYSHEV) && c->d.n_rot == 0 && c->d.n_oitems == 0 &&
-            c->plan.num_colors > 0 && c->plan.conflict_list.empty() && (!c->rc || c->res_check_every % 2 == 0)) {
+        const bool positional = !(c->desc.flags & AVBD_FLAG_SEPARATE_CHEBYSHEV) && c->d.n_rot == 0 &&
+                                c->d.n_oitems == 0 && c->plan.num_colors > 0 && c->plan.conflict_list.empty();
+        if (positional && (!c->rc || c->res_check_every % 2 == 0)) {
             const uint32_t last = c->plan.num_colors - 1;
             std::vector<uint8_t> in_last(n, 0);
             for (uint32_t k = c->plan.item_offsets[last]; k < c->plan.item_offsets[last + 1]; k++)
@@ -2211,8 +2236,8 @@ int avbd_build_graph(avbd_ctx* c) {
             c->cheb_list = dev_alloc<uint32_t>(c, std::max<size_t>(1, rest.size()));
             if (!rest.empty()) upload(c, c->cheb_list, rest);
             c->fuse_cheb = true;
-            setup_resident(c);
         }
+        if (positional) setup_resident(c);
         c->built = true;
 
         // timing events bracket the solve launches of a fixed-count step

@@ -111,6 +111,18 @@ bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos
 void resident_shape(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t given,
                     uint32_t& lanes, uint32_t& block);
 
+// What a launch runs: check intervals of `every` iterations until the scene has
+// converged, per_launch of them at most and `total` in a step (hist set), or
+// just `every` iterations (hist null).
+struct ResidentCheck {
+    uint32_t every = 0, per_launch = 0, total = 0;
+    uint32_t per_scene = 0;       // the scenes of a batch stop on their own
+    double tol2 = 0;
+    const double* mg2 = nullptr;  // per scene: ||M g||^2 over its free particles
+    double* hist = nullptr;       // per scene per_launch residual sums
+    uint32_t* ran = nullptr;      // per scene: checks of this launch (0 again once recorded)
+};
+
 // Device side of the plan plus the state the kernel works on.
 struct ResidentDev {
     const ResidentPatch* patches = nullptr;
@@ -123,6 +135,7 @@ struct ResidentDev {
     const uint32_t* col = nullptr;
     const void* edges = nullptr;         // TetEdges of the state's precision per tet (no damping)
     unsigned long long* xch = nullptr;   // per halo slot 3 (FP32) or 6 (FP64) tagged words
+    unsigned long long* sums = nullptr;  // two sets of two tagged words per patch: its residual sum
     uint32_t* epoch = nullptr;           // per patch: exchanges per colour so far (the tag base)
     uint32_t* launches = nullptr;        // per patch: launches so far
     uint32_t* sync = nullptr;            // per patch (the cluster's first one): arrivals, decision word
@@ -132,11 +145,13 @@ struct ResidentDev {
     bool has_ground = false;
 };
 
-// Iterations [iter0, iter0 + iters) of a step (in residual mode iter0 is the
-// control word's counter); rr: |r_v|^2 per particle after the last one, or null.
+// The iterations of `chk` from omega_tab[0] (in residual mode omega_tab[rc->iter]).
 void launch_resident(hipStream_t s, const ResidentDev& r, const DevState& d, bool damping, float dt, const ResCtl* rc,
-                     const float* omega_tab, uint32_t iters, double* rr);
+                     const float* omega_tab, const ResidentCheck& chk);
 void launch_resident_f64(hipStream_t s, const ResidentDev& r, const F64State& f, bool damping, double dt,
-                         const ResCtl* rc, const float* omega_tab, uint32_t iters, double* rr);
+                         const ResCtl* rc, const float* omega_tab, const ResidentCheck& chk);
+// After a launch with checks: the step's residual record, counters and frozen scenes.
+void launch_residual_collect(hipStream_t s, ResCtl* rc, const ResidentCheck& chk, double* acc_scene, uint32_t n_scenes,
+                             const SceneFreeze& fz);
 
 }  // namespace avbd

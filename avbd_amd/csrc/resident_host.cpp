@@ -17,7 +17,7 @@ constexpr uint32_t NONE = 0xFFFFFFFFu;
 // idx[lo, hi), each cut along the longest side of the box so that the weight
 // divides in proportion to the parts of the two sides.
 void bisect(uint32_t* idx, uint32_t lo, uint32_t hi, uint32_t first, uint32_t parts, const double* pos,
-            const uint32_t* weight, uint32_t base, uint32_t* part) {
+            const uint32_t* weight, uint32_t base, uint32_t* part, uint32_t threads) {
     if (parts <= 1 || hi - lo <= 1) {
         for (uint32_t k = lo; k < hi; k++) part[idx[k]] = first;
         return;
@@ -36,22 +36,27 @@ void bisect(uint32_t* idx, uint32_t lo, uint32_t hi, uint32_t first, uint32_t pa
     for (int a = 1; a < 3; a++)
         if (mx[a] - mn[a] > mx[axis] - mn[axis]) axis = a;
     // ties by index, so that the cut does not depend on the sort
-    std::sort(idx + lo, idx + hi, [&](uint32_t a, uint32_t b) {
-        const double pa = pos[3 * (size_t)(base + a) + axis], pb = pos[3 * (size_t)(base + b) + axis];
-        return pa < pb || (pa == pb && a < b);
-    });
+    std::vector<std::pair<double, uint32_t>> key(hi - lo);
+    for (uint32_t k = lo; k < hi; k++) key[k - lo] = {pos[3 * (size_t)(base + idx[k]) + axis], idx[k]};
+    std::sort(key.begin(), key.end());
+    for (uint32_t k = lo; k < hi; k++) idx[k] = key[k - lo].second;
     const uint32_t left = parts / 2;
     const uint64_t want = total * left / parts;
     uint64_t sum = 0;
     uint32_t cut = lo;
     while (cut < hi && sum + weight[idx[cut]] <= want) sum += weight[idx[cut++]];
-    bisect(idx, lo, cut, first, left, pos, weight, base, part);
-    bisect(idx, cut, hi, first + left, parts - left, pos, weight, base, part);
+    // the two sides touch different particles
+    std::thread side;
+    if (hi - lo > 4096 && threads > 1)
+        side = std::thread(bisect, idx, lo, cut, first, left, pos, weight, base, part, threads / 2);
+    else bisect(idx, lo, cut, first, left, pos, weight, base, part, 1);
+    bisect(idx, cut, hi, first + left, parts - left, pos, weight, base, part, threads - threads / 2);
+    if (side.joinable()) side.join();
 }
 
 // One scene's patches (offsets relative to the scene's own arrays).
 bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, const ResidentLimits& lim,
-                 uint32_t scene, ResidentPlan& out) {
+                 uint32_t scene, uint32_t threads, ResidentPlan& out) {
     const uint32_t lo = (*m.scene_offsets)[scene], hi = (*m.scene_offsets)[scene + 1], n = hi - lo;
     if (n == 0) return true;
     const uint32_t colors = plan.num_colors;
@@ -81,7 +86,7 @@ bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, c
     const uint32_t n_tets = t0 == NONE ? 0 : t1 - t0 + 1;
     while (true) {
         std::iota(order.begin(), order.end(), 0u);
-        bisect(order.data(), 0, n, 0, parts, pos, weight.data(), lo, part.data());
+        bisect(order.data(), 0, n, 0, parts, pos, weight.data(), lo, part.data(), threads);
         out = ResidentPlan{};
         std::vector<std::vector<uint32_t>> own(parts);
         for (uint32_t v = 0; v < n; v++) own[part[v]].push_back(v);
@@ -203,10 +208,11 @@ bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos
     std::vector<ResidentPlan> scenes(n_scenes);
     std::atomic<uint32_t> next{0};
     std::atomic<bool> ok{true};
-    const uint32_t workers = std::min(n_scenes, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+    const uint32_t cpus = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+    const uint32_t workers = std::min(n_scenes, cpus);
     auto work = [&] {
         for (uint32_t s; ok && (s = next++) < n_scenes;)
-            if (!build_scene(m, plan, pos, lim, s, scenes[s])) ok = false;
+            if (!build_scene(m, plan, pos, lim, s, std::max(1u, cpus / workers), scenes[s])) ok = false;
     };
     if (workers <= 1) {
         work();

@@ -17,14 +17,16 @@
 // on the same values as its owner's.
 //
 // What bounds it now is the chain of one phase: LDS reads of a lane's two or
-// three incidences, their sum over the lanes, the 3x3 solve (4,400 cycles in
-// FP64, 3,900 in FP32 at 8 lanes), then the neighbours' words through the caches
-// (2,400), 4 times per iteration; about 25 us per launch go into loading the patch
-// and the handshake.  Iterations of one scene, one launch per phase before ->
-// now: FP64 32^3 to a residual target 36.6 -> 18.8 us each (6350 of them, checks
-// every 10 included); FP32 32^3 step of 10 iterations 365 -> 240 us (then bound
-// by the broad phase beside it), 15^3 of 20 440 -> 237 us, 512 cubes of 4 to 16
-// cells and 10 iterations 49.1 -> 33.9 ms per 10 steps with the read-back.
+// three incidences (2,400 cycles for wavefront 0 in FP64 at 8 lanes: nine
+// positions and five constants each, by all wavefronts of the CU), their sum over
+// the lanes and the 3x3 solve (600), sending (1,000), then waiting for the
+// neighbours' words (2,100); 4 times per iteration.  Loading the patch and the
+// handshake take 45,000 cycles per launch, a residual check 17,000.
+// One launch per phase before -> now: FP64 32^3 to a residual target 36.6 ->
+// 14.4 us per iteration, checks every 10 included (18.8 with one launch per
+// check); 64 FP64 cubes 48.5 -> 25.4 ms; FP32 32^3 step of 10 iterations 365 ->
+// 240 us (then bound by the broad phase beside it), 15^3 of 20 440 -> 237 us, 512
+// cubes of 4 to 16 cells 49.1 -> 33.9 ms per 10 steps with the read-back.
 //
 // Exchange: every 32-bit piece of a position travels in an 8-byte word next
 // to a 32-bit tag (the number of the exchange), written and read with relaxed
@@ -34,6 +36,13 @@
 // overwritten before it has been read: its owner solves the vertex again only
 // after it has received, in the same iteration, the results that its readers
 // computed from it.
+//
+// Residual checks (ResidentCheck): a launch covers several check intervals.
+// After each one every patch publishes the sum of its |r_v|^2 the same way,
+// takes those of all patches of its cluster and adds them in one order, so all
+// of them reach the same decision without a further exchange.  Two sets of
+// words, used in turn: a patch that sends its sum for check k has read those of
+// check k - 1, so the words of k - 1 are free once every sum of k has arrived.
 //
 // Waits end: the patches of a scene depend on each other, so they must all be
 // running.  Each announces itself after loading its patch and waits until
@@ -110,8 +119,7 @@ struct Args {
     const ResCtl* rc;
     const float* omega_tab;
     const uint32_t* frozen;
-    double* rr;
-    uint32_t iters;
+    ResidentCheck chk;   // every: iterations of the launch when it has no checks
     R inv_dt, inv_dt2;
 };
 
@@ -146,6 +154,27 @@ __device__ __forceinline__ R chebyshev(R w, R x, R xll) {
     return w * (x - xll) + xll;
 }
 
+// The converged test of a scene with residual sum r2 (that of the launch which
+// records the checks: residual_collect_kernel).
+__device__ __forceinline__ bool converged(const ResidentCheck& k, uint32_t scene, double r2) {
+    const double m = k.mg2[scene];
+    return k.per_scene ? r2 <= k.tol2 * m : !(m > 0) || r2 / m <= k.tol2;
+}
+
+// Sum over the workgroup in a fixed order, the same value in every thread.
+template <int B>
+__device__ __forceinline__ double block_sum(double v, double* red) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    __syncthreads();   // red is free
+    if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0;
+#pragma unroll
+    for (int w = 0; w < B / 64; w++) t += red[w];
+    return t;
+}
+
 // Edge constants of a tet as corner a sees them.
 __device__ __forceinline__ uint32_t weight_index(uint32_t a, uint32_t j) {
     // kEdgeWeight[a][j] in nibble a
@@ -177,12 +206,13 @@ __device__ __forceinline__ GroundRec to_rec(const ResidentGround& l) {
 // A scene whose patches could not all run at once: its first patch runs the
 // stretch alone on the state in device memory, patch by patch (a workgroup's
 // own global writes are visible to it after a barrier).
-template <class R, int L, bool DAMP>
-__device__ __forceinline__ void run_alone(const Args<R>& a, uint32_t first, uint32_t count) {
+template <class R, int L, bool DAMP, int B>
+__device__ __forceinline__ void run_alone(const Args<R>& a, uint32_t first, uint32_t count, uint32_t scene,
+                                          uint32_t checks, double* red) {
     using K = Kind<R>;
     using V3 = typename K::V3;
     using V4 = typename K::V4;
-    const uint32_t lane = threadIdx.x % L, group = threadIdx.x / L, groups = blockDim.x / L;
+    const uint32_t lane = threadIdx.x % L, group = threadIdx.x / L, groups = B / L;
     const uint32_t nc = a.r.n_colors;
     const float* omega = a.omega_tab + (a.rc ? a.rc->iter : 0u);
     auto pos = [&](uint32_t v) {
@@ -213,7 +243,8 @@ __device__ __forceinline__ void run_alone(const Args<R>& a, uint32_t first, uint
             }
         }
     };
-    for (uint32_t i = 0; i < a.iters; i++) {
+    for (uint32_t n = 0; n < checks; n++) {
+    for (uint32_t i = 0; i < a.chk.every; i++) {
         for (uint32_t c = 0; c < nc; c++) {
             for (uint32_t q = first; q < first + count; q++) {
                 const ResidentPatch p = a.r.patches[q];
@@ -233,10 +264,10 @@ __device__ __forceinline__ void run_alone(const Args<R>& a, uint32_t first, uint
             }
             __syncthreads();
         }
-        const R w = omega[i];
+        const R w = *omega++;
         for (uint32_t q = first; q < first + count; q++) {
             const ResidentPatch p = a.r.patches[q];
-            for (uint32_t k = threadIdx.x; k < p.own; k += blockDim.x) {
+            for (uint32_t k = threadIdx.x; k < p.own; k += B) {
                 const uint32_t v = a.r.gid[p.gid_off + k];
                 const V4 xc = a.x[v], xl = a.last[v], xll = a.lastlast[v];
                 const V4 xp = K::v4(chebyshev(w, xc.x, xll.x), chebyshev(w, xc.y, xll.y), chebyshev(w, xc.z, xll.z),
@@ -254,22 +285,43 @@ __device__ __forceinline__ void run_alone(const Args<R>& a, uint32_t first, uint
         }
         __syncthreads();
     }
-    if (a.rr)
-        for (uint32_t q = first; q < first + count; q++) {
-            const ResidentPatch p = a.r.patches[q];
-            for (uint32_t k = group; k < p.items; k += groups) {
-                const uint32_t v = a.r.gid[p.gid_off + k];
-                const V4 xv = a.x[v];
-                V3 g;
-                typename K::Sym h;
-                item(p, k, K::v3(xv.x, xv.y, xv.z), g, h);
-                sum_group<L, false>(g, h);
-                if (lane != 0) continue;
-                const int32_t gi = a.ground_of[v];
-                if (gi >= 0) ground_accumulate(a.ground[gi], K::v3(xv.x, xv.y, xv.z), g, h);
-                a.rr[v] = residual2(xv, a.y[v], g, a.inv_dt2);
-            }
+    if (!a.chk.hist) return;
+    for (uint32_t q = first; q < first + count; q++) {
+        const ResidentPatch p = a.r.patches[q];
+        double r2 = 0;
+        for (uint32_t k = group; k < p.items; k += groups) {
+            const uint32_t v = a.r.gid[p.gid_off + k];
+            const V4 xv = a.x[v];
+            V3 g;
+            typename K::Sym h;
+            item(p, k, K::v3(xv.x, xv.y, xv.z), g, h);
+            sum_group<L, false>(g, h);
+            if (lane != 0) continue;
+            const int32_t gi = a.ground_of[v];
+            if (gi >= 0) ground_accumulate(a.ground[gi], K::v3(xv.x, xv.y, xv.z), g, h);
+            r2 += residual2(xv, a.y[v], g, a.inv_dt2);
         }
+        r2 = block_sum<B>(r2, red);
+        // under tag 0, which no exchange waits for
+        if (threadIdx.x < 2)
+            __hip_atomic_store(a.r.sums + 2 * q + threadIdx.x, (word_t)Kind<double>::word(make_double4(r2, 0, 0, 0), threadIdx.x),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    double sum = 0;
+    for (uint32_t q = threadIdx.x; q < count; q += B) {
+        const word_t* w = a.r.sums + 2 * (first + q);
+        const word_t lo = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                     hi = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sum += __longlong_as_double((long long)(hi << 32 | lo));
+    }
+    sum = block_sum<B>(sum, red);
+    if (threadIdx.x == 0) {
+        a.chk.hist[scene * a.chk.per_launch + n] = sum;
+        a.chk.ran[scene] = n + 1;
+    }
+    if (converged(a.chk, scene, sum)) return;
+    }
 }
 
 // A lane's incidence, read from LDS in two steps: what does not change
@@ -350,10 +402,13 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
     constexpr uint32_t W = K::kWords;
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ uint32_t decision, dead;
+    __shared__ double red[B / 64];
     if (a.rc && a.rc->done) return;
     const ResidentPatch p = a.r.patches[blockIdx.x];
     if (a.frozen && a.frozen[p.scene]) return;
     const uint32_t tid = threadIdx.x, nc = a.r.n_colors;
+    // check intervals of this launch (the step's budget is chk.total of them)
+    const uint32_t checks = a.chk.hist ? min(a.chk.per_launch, a.chk.total - min(a.chk.total, a.rc->checks)) : 1u;
     const bool has_ground = a.r.has_ground;
     const ResidentLds o =
         resident_lds(p.own, p.items, p.local, p.tets, p.inc, p.targets, nc, sizeof(R), DAMP, has_ground);
@@ -475,13 +530,27 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
         }
         __syncthreads();
         if (decision) {
-            if (blockIdx.x == p.first) run_alone<R, L, DAMP>(a, p.first, p.count);
+            if (blockIdx.x == p.first) run_alone<R, L, DAMP, B>(a, p.first, p.count, p.scene, checks, red);
             return;   // the exchange did not run: the epochs stay
         }
     }
 
     const uint32_t lane = tid % L, group = tid / L;
     constexpr uint32_t groups = B / L;
+    // the payload of an exchange word, once it carries `tag`
+    auto wait_word = [&](const word_t* src, uint32_t tag) {
+        uint64_t t0 = 0;
+        while (true) {
+            const word_t u = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((uint32_t)(u >> 32) == tag) return (uint32_t)u;
+            if (t0 == 0) t0 = wall_clock64();
+            if (*(volatile uint32_t*)&dead || wall_clock64() - t0 > kWaitTicks) {
+                *(volatile uint32_t*)&dead = 1;
+                atomicOr(a.r.status, 2u);
+                return 0u;
+            }
+        }
+    };
     // takes the halo of colour c at exchange `tag`: the slots of a colour are
     // contiguous, and so are their places in x, so a thread moves one 32-bit piece
     // (threads from the top: the low ones have the items)
@@ -489,22 +558,23 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
         const uint32_t h0 = col[nc + 1 + c], h1 = col[nc + 2 + c];
         const word_t* src = a.r.xch + (size_t)(p.slot + (h0 - p.own)) * W;
         uint32_t* dst = reinterpret_cast<uint32_t*>(x) + h0 * W;
-        for (uint32_t k = B - 1 - tid; k < (h1 - h0) * W; k += B) {
-            uint64_t t0 = 0;
-            while (true) {
-                const word_t u = __hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((uint32_t)(u >> 32) == tag) {
-                    dst[k] = (uint32_t)u;
-                    break;
-                }
-                if (t0 == 0) t0 = wall_clock64();
-                if (*(volatile uint32_t*)&dead || wall_clock64() - t0 > kWaitTicks) {
-                    *(volatile uint32_t*)&dead = 1;
-                    atomicOr(a.r.status, 2u);
-                    break;
-                }
-            }
+        for (uint32_t k = B - 1 - tid; k < (h1 - h0) * W; k += B) dst[k] = wait_word(src + k, tag);
+    };
+    // the scene's sum of the patches' v after exchange `tag`
+    auto scene_sum = [&](double v, uint32_t tag, uint32_t turn) {
+        v = block_sum<B>(v, red);
+        if (p.count == 1) return v;
+        word_t* set = a.r.sums + 2 * (size_t)(turn * a.r.n_patches + p.first);
+        if (tid < 2)
+            __hip_atomic_store(set + 2 * (blockIdx.x - p.first) + tid,
+                               (word_t)tag << 32 | Kind<double>::word(make_double4(v, 0, 0, 0), tid), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        double sum = 0;
+        for (uint32_t q = tid; q < p.count; q += B) {
+            const word_t lo = wait_word(set + 2 * q, tag), hi = wait_word(set + 2 * q + 1, tag);
+            sum += __longlong_as_double((long long)(hi << 32 | lo));
         }
+        return block_sum<B>(sum, red);
     };
 
     // A lane's first incidence of a colour phase is read ahead: indices and
@@ -545,7 +615,6 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
         read_item(k);
         if (own) read_own(k);
     };
-    read_ahead(0, false);
     auto gather = [&](V3 xa, V3& g, typename K::Sym& h) {
         const uint32_t begin = it.x & 0xffffu, cnt = it.x >> 16;
         g = K::v3(0, 0, 0);
@@ -575,61 +644,62 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
 
     // ---- the iterations
     const float* omega = a.omega_tab + (a.rc ? a.rc->iter : 0u);
-    read_ahead_own(0);
-    for (uint32_t i = 0; i < a.iters; i++) {
-        const uint32_t tag = base + i + 1u;
-        const R w = omega[i];
-        for (uint32_t c = 0; c < nc; c++) {
-            const uint32_t end = col[c + 1], begin = col[c] + group;
-            for (uint32_t k = begin; k < end; k += groups) {
-                if (k != begin) {
-                    read_item(k);
-                    read_own(k);
+    uint32_t tag = base;
+    for (uint32_t n = 0; n < checks; n++) {
+        read_ahead(0, true);
+        for (uint32_t i = 0; i < a.chk.every; i++) {
+            tag++;
+            const R w = *omega++;
+            for (uint32_t c = 0; c < nc; c++) {
+                const uint32_t end = col[c + 1], begin = col[c] + group;
+                for (uint32_t k = begin; k < end; k += groups) {
+                    if (k != begin) {
+                        read_item(k);
+                        read_own(k);
+                    }
+                    V3 g;
+                    typename K::Sym h;
+                    gather(K::v3(xv.x, xv.y, xv.z), g, h);
+                    sum_group<L, true>(g, h);
+                    // every lane of the group solves the block: the same instructions
+                    // as one lane would issue, and each can then send a piece of the result
+                    if (touches) ground_add(gk, gf, g, h);
+                    const V4 nx = block_step(xv, yv, g, h, a.inv_dt2);
+                    send(nx, tag);
+                    if (lane == 0) {
+                        x[3 * k] = nx.x;
+                        x[3 * k + 1] = nx.y;
+                        x[3 * k + 2] = nx.z;
+                    }
                 }
-                V3 g;
-                typename K::Sym h;
-                gather(K::v3(xv.x, xv.y, xv.z), g, h);
-                sum_group<L, true>(g, h);
-                // every lane of the group solves the block: the same instructions
-                // as one lane would issue, and each can then send a piece of the result
-                if (touches) ground_add(gk, gf, g, h);
-                const V4 nx = block_step(xv, yv, g, h, a.inv_dt2);
-                send(nx, tag);
-                if (lane == 0) {
-                    x[3 * k] = nx.x;
-                    x[3 * k + 1] = nx.y;
-                    x[3 * k + 2] = nx.z;
+                read_ahead(c + 1 < nc ? c + 1 : 0u, c + 1 < nc);
+                // a vertex of colour c has no neighbour of colour c, so the halo of
+                // this colour can change while other wavefronts still solve it
+                refresh(c, tag);
+                lds_barrier();
+            }
+            for (uint32_t k = tid; k < p.local; k += B) {
+                R q[3];
+    #pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const R xll = lastlast[3 * k + j];
+                    q[j] = chebyshev(w, x[3 * k + j], xll);
+                    lastlast[3 * k + j] = last[3 * k + j];
+                    last[3 * k + j] = q[j];
+                    x[3 * k + j] = q[j];
+                }
+                if (has_ground && k < p.own && gof[k] >= 0) {
+                    GroundRec rec = to_rec(ground[k]);
+                    dual(rec, K::v3(q[0], q[1], q[2]));
+                    ground[k] = to_lds(rec);
+                    ground_terms(k, rec, K::v3(q[0], q[1], q[2]));
                 }
             }
-            read_ahead(c + 1 < nc ? c + 1 : 0u, c + 1 < nc);
-            // a vertex of colour c has no neighbour of colour c, so the halo of
-            // this colour can change while other wavefronts still solve it
-            refresh(c, tag);
             lds_barrier();
+            read_ahead_own(0);
         }
-        for (uint32_t k = tid; k < p.local; k += B) {
-            R q[3];
-#pragma unroll
-            for (int j = 0; j < 3; j++) {
-                const R xll = lastlast[3 * k + j];
-                q[j] = chebyshev(w, x[3 * k + j], xll);
-                lastlast[3 * k + j] = last[3 * k + j];
-                last[3 * k + j] = q[j];
-                x[3 * k + j] = q[j];
-            }
-            if (has_ground && k < p.own && gof[k] >= 0) {
-                GroundRec rec = to_rec(ground[k]);
-                dual(rec, K::v3(q[0], q[1], q[2]));
-                ground[k] = to_lds(rec);
-                ground_terms(k, rec, K::v3(q[0], q[1], q[2]));
-            }
-        }
-        lds_barrier();
-        read_ahead_own(0);
-    }
-
-    // ---- residual, then the state back
-    if (a.rr)
+        if (!a.chk.hist) break;
+        double r2 = 0;
         for (uint32_t k = group; k < p.items; k += groups) {
             read_item(k);
             read_own(k);
@@ -639,9 +709,18 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
             sum_group<L, false>(g, h);
             if (lane == 0) {
                 if (touches) ground_add(gk, gf, g, h);
-                a.rr[a.r.gid[p.gid_off + k]] = residual2(xv, yv, g, a.inv_dt2);
+                r2 += residual2(xv, yv, g, a.inv_dt2);
             }
         }
+        r2 = scene_sum(r2, tag, n & 1u);
+        if (tid == 0 && blockIdx.x == p.first) {
+            a.chk.hist[p.scene * a.chk.per_launch + n] = r2;
+            a.chk.ran[p.scene] = n + 1;
+        }
+        if (converged(a.chk, p.scene, r2)) break;   // the same in every patch of the scene
+    }
+
+    // ---- the state back
     for (uint32_t k = tid; k < p.own; k += B) {
         const uint32_t v = a.r.gid[p.gid_off + k];
         const R m = ym[4 * k + 3];
@@ -660,7 +739,7 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
             rec.flags = l.flags;
         }
     }
-    if (tid == 0 && p.count > 1) a.r.epoch[blockIdx.x] = base + a.iters;
+    if (tid == 0 && p.count > 1) a.r.epoch[blockIdx.x] = tag;
 }
 
 template <class R, int L, bool DAMP, int B>
@@ -673,9 +752,9 @@ void dispatch_block(hipStream_t s, const Args<R>& a) {
 
 template <class R, int L, bool DAMP>
 void dispatch(hipStream_t s, const Args<R>& a) {
-    if (a.r.block >= 1024) dispatch_block<R, L, DAMP, 1024>(s, a);
-    else if (a.r.block >= 512) dispatch_block<R, L, DAMP, 512>(s, a);
-    else dispatch_block<R, L, DAMP, 256>(s, a);
+    if constexpr (sizeof(R) == 4)
+        if (a.r.block == 1024) return dispatch_block<R, L, DAMP, 1024>(s, a);
+    dispatch_block<R, L, DAMP, 512>(s, a);
 }
 
 template <class R>
@@ -698,22 +777,95 @@ void launch(hipStream_t s, const Args<R>& a, bool damping) {
 }  // namespace
 
 void launch_resident(hipStream_t s, const ResidentDev& r, const DevState& d, bool damping, float dt, const ResCtl* rc,
-                     const float* omega_tab, uint32_t iters, double* rr) {
-    if (iters == 0) return;
+                     const float* omega_tab, const ResidentCheck& chk) {
+    if (chk.every == 0) return;
     Args<float> a{r,      d.x,       d.y,      d.x_last, d.x_lastlast, d.ground,
                   d.ground_of, d.tets, d.damp, static_cast<const TetEdges<float>*>(r.edges), rc, omega_tab,
-                  d.frozen, rr, iters, 1.0f / dt, 1.0f / (dt * dt)};
+                  d.frozen, chk, 1.0f / dt, 1.0f / (dt * dt)};
     launch<float>(s, a, damping);
 }
 
 void launch_resident_f64(hipStream_t s, const ResidentDev& r, const F64State& f, bool damping, double dt,
-                         const ResCtl* rc, const float* omega_tab, uint32_t iters, double* rr) {
-    if (iters == 0) return;
+                         const ResCtl* rc, const float* omega_tab, const ResidentCheck& chk) {
+    if (chk.every == 0) return;
     const double inv_dt = 1.0 / dt;
     Args<double> a{r,      f.x,       f.y,      f.x_last, f.x_lastlast, f.ground,
                    f.ground_of, f.tets, f.damp, static_cast<const TetEdges<double>*>(r.edges), rc, omega_tab,
-                   f.frozen, rr, iters, inv_dt, inv_dt * inv_dt};
+                   f.frozen, chk, inv_dt, inv_dt * inv_dt};
     launch<double>(s, a, damping);
+}
+
+// Records the checks of a resident launch.  Per check: the sums over all
+// scenes (a scene that had stopped counts with the residual it stopped at), in
+// the order of residual_decide_kernel, one wavefront per check; then the step's
+// counters, and the scenes that stopped are frozen.  One workgroup; it runs once
+// per launch of about a hundred iterations.
+__global__ __launch_bounds__(1024) void residual_collect_kernel(ResCtl* rc, ResidentCheck k, double* acc_scene,
+                                                                uint32_t n_scenes, SceneFreeze fz) {
+    __shared__ uint32_t most, reached;
+    if (rc->done) return;
+    if (threadIdx.x == 0) {
+        most = 0;
+        reached = 0xFFFFFFFFu;
+    }
+    __syncthreads();
+    const uint32_t iter = rc->iter, checks = rc->checks;
+    for (uint32_t s = threadIdx.x; s < n_scenes; s += 1024) {
+        uint32_t ran = k.ran[s];
+        const bool stopped = fz.frozen && fz.frozen[s];
+        if (stopped) ran = k.ran[s] = 0;
+        if (ran) acc_scene[s] = k.hist[s * k.per_launch + ran - 1];
+        atomicMax(&most, ran);
+        if (!fz.frozen || stopped) continue;
+        const uint32_t n = ran ? ran : 1u;   // a scene without particles has no patch
+        if (converged(k, s, ran ? acc_scene[s] : 0.0)) {
+            fz.frozen[s] = 1;
+            fz.iters[s] = iter + n * k.every;
+        }
+    }
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t n = threadIdx.x >> 6; n < most; n += 16) {
+        double r[4] = {0, 0, 0, 0}, m[4] = {0, 0, 0, 0}, w = 0;
+        for (uint32_t s0 = 0; s0 < n_scenes; s0 += 256)
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                const uint32_t s = s0 + 64 * j + lane;
+                if (s >= n_scenes) break;
+                const double v = n < k.ran[s] ? k.hist[s * k.per_launch + n] : acc_scene[s], mg = k.mg2[s];
+                r[j] += v;
+                m[j] += mg;
+                if (mg > 0) w = fmax(w, v / mg);
+            }
+        double rs = (r[0] + r[2]) + (r[1] + r[3]), ms = (m[0] + m[2]) + (m[1] + m[3]);
+        for (int off = 32; off > 0; off >>= 1) {
+            rs += __shfl_down(rs, off);
+            ms += __shfl_down(ms, off);
+            w = fmax(w, __shfl_xor(w, off));
+        }
+        if (lane == 0) {
+            if (checks + n < kMaxResidualChecks) {
+                rc->rel[checks + n] = ms > 0 ? sqrt(rs / ms) : 0.0;
+                rc->worst[checks + n] = sqrt(w);
+            }
+            if (w <= k.tol2) atomicMin(&reached, n);
+        }
+    }
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s < n_scenes; s += 1024) k.ran[s] = 0;
+    if (threadIdx.x == 0) {
+        rc->checks = checks + most;
+        rc->iter = iter + most * k.every;
+        if (reached < most || (most == 0 && checks < k.total)) {   // (no check run: every scene is frozen)
+            rc->done = 1;
+            rc->last_iters = rc->iter;
+        }
+    }
+}
+
+void launch_residual_collect(hipStream_t s, ResCtl* rc, const ResidentCheck& chk, double* acc_scene, uint32_t n_scenes,
+                             const SceneFreeze& fz) {
+    hipLaunchKernelGGL(residual_collect_kernel, dim3(1), dim3(1024), 0, s, rc, chk, acc_scene, n_scenes, fz);
 }
 
 }  // namespace avbd
