@@ -83,6 +83,8 @@ struct avbd_ctx {
     // colour phase otherwise
     bool resident = false;
     ResidentDev res;
+    bool bundled = false;      // static scenes of oriented particles only, each component small enough
+    BundleDev bundles;
     ResidentCheck res_check;   // residual mode: the check intervals of a resident launch
 
     bool timing = false;
@@ -683,7 +685,9 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
         else launch_resident(s, c->res, dz, c->damping, dt, rc, c->omega_tab + i0, chk);
         if (check) launch_residual_collect(s, c->rc, chk, c->res_acc_scene, c->n_res_scenes, fz);
     }
-    for (uint32_t i = i0; i < i1 && !resident; i++) {
+    const bool bundled = c->bundled && !c->dynamic && !with_events;
+    if (bundled) launch_bundles(s, dz, c->bundles, dt, rc, c->omega_tab + i0, i1 - i0);
+    for (uint32_t i = i0; i < i1 && !resident && !bundled; i++) {
         const float omega = c->omega_seq[i];
         const uint32_t j = i - i0;
         const bool odd = (i & 1u) != 0;
@@ -1295,6 +1299,41 @@ void setup_resident(avbd_ctx* c) {
     r.has_ground = lim.ground;
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     c->resident = true;
+}
+
+// The same for scenes of oriented particles only (rods, jointed bodies)
+// without dynamic contacts: the components are small and do not depend on each
+// other, so each stays with one workgroup.
+void setup_bundles(avbd_ctx* c) {
+    if (c->desc.flags & AVBD_FLAG_NO_PERSISTENT) return;
+    std::vector<uint32_t> so = c->scene_offsets;
+    if (so.empty()) so = {0u, c->d.n};
+    HostModel m;
+    m.n = c->d.n;
+    m.cos = &c->cos;
+    m.joints = &c->joints;
+    m.joints2 = &c->joints2;
+    m.scene_offsets = &so;
+    BundlePlan plan;
+    if (!build_bundles(m, c->plan, plan)) return;
+    auto put = [&](auto& dst, const auto& src) {
+        using T = std::decay_t<decltype(src[0])>;
+        T* p = dev_alloc<T>(c, std::max<size_t>(1, src.size()));
+        if (!src.empty()) upload(c, p, src);
+        dst = p;
+    };
+    BundleDev& b = c->bundles;
+    put(b.item_off, plan.item_off);
+    put(b.part_off, plan.part_off);
+    put(b.joint_off, plan.joint_off);
+    put(b.items, plan.items);
+    put(b.parts, plan.parts);
+    put(b.joints, plan.joints);
+    b.n_bundles = plan.n_bundles;
+    b.n_colors = plan.n_colors;
+    b.block = plan.block;
+    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    c->bundled = true;
 }
 
 }  // namespace
@@ -2238,6 +2277,7 @@ int avbd_build_graph(avbd_ctx* c) {
             c->fuse_cheb = true;
         }
         if (positional) setup_resident(c);
+        else if (c->d.n_rot == n && c->plan.conflict_list.empty()) setup_bundles(c);
         c->built = true;
 
         // timing events bracket the solve launches of a fixed-count step

@@ -358,7 +358,27 @@ struct SceneFreeze {
     const uint32_t* scene_of = nullptr;  // per particle
 };
 
+// The resident solve of oriented particles: bundles of connected components
+// (rods, jointed bodies), each run by one workgroup for a whole stretch of
+// iterations.  Offsets per bundle; items per bundle and colour (n_colors + 1
+// offsets each).
+struct BundlePlan {
+    uint32_t n_bundles = 0, n_colors = 0, block = 0;
+    std::vector<uint32_t> item_off, part_off, joint_off;
+    std::vector<OItem> items;
+    std::vector<uint32_t> parts, joints;   // particles; two-sided joint records
+};
+struct BundleDev {
+    const uint32_t *item_off = nullptr, *part_off = nullptr, *joint_off = nullptr;
+    const OItem* items = nullptr;
+    const uint32_t *parts = nullptr, *joints = nullptr;
+    uint32_t n_bundles = 0, n_colors = 0, block = 0;
+};
+
 void launch_eprev(hipStream_t s, const DevState& d, float dt);
+// iterations [0, iters) of a stretch from omega_tab[0] (residual mode: omega_tab[rc->iter])
+void launch_bundles(hipStream_t s, const DevState& d, const BundleDev& b, float dt, const ResCtl* rc,
+                    const float* omega_tab, uint32_t iters);
 void launch_solve_ocolor(hipStream_t s, const DevState& d, uint32_t item_begin, uint32_t item_count, float dt,
                          const uint32_t* done = nullptr);
 void launch_step_begin(hipStream_t s, const DevState& d, float dt, float g);
@@ -527,6 +547,10 @@ struct ColorPlan {
     std::vector<OItem> oitem_of;
     std::vector<uint32_t> static_off, static_nb;
 };
+
+// Bundles of the scenes (all particles oriented); false when one component has
+// too many items of a colour for a workgroup.
+bool build_bundles(const HostModel& m, const ColorPlan& plan, BundlePlan& out);
 
 // Colours every scene of a global static adjacency CSR (scene offsets,
 // vertex offsets, neighbours) into color, with the colour count per scene.

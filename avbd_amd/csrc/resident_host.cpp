@@ -266,4 +266,68 @@ void resident_shape(const ResidentPlan& plan, uint32_t colors, const ResidentLim
     block = lim.real_bytes == 4 && lanes * most > 512 ? 1024u : 512u;
 }
 
+bool build_bundles(const HostModel& m, const ColorPlan& plan, BundlePlan& out) {
+    const uint32_t n = m.n, nc = plan.num_colors;
+    // connected components over rod elements and two-sided joints
+    std::vector<uint32_t> root(n);
+    std::iota(root.begin(), root.end(), 0u);
+    auto find = [&](uint32_t v) {
+        while (root[v] != v) v = root[v] = root[root[v]];
+        return v;
+    };
+    auto join = [&](uint32_t a, uint32_t b) {   // the smaller index stays
+        a = find(a);
+        b = find(b);
+        root[std::max(a, b)] = std::min(a, b);
+    };
+    for (const HostCos& e : *m.cos) join(e.idx[0], e.idx[1]);
+    for (const HostJoint2& j : *m.joints2) join(j.p[0], j.p[1]);
+    // components in order of their first particle, bundled within a scene until
+    // a bundle has its share of the particles for 256 CUs, 128 at most (one to two
+    // wavefronts per phase, as the largest rods have)
+    std::vector<uint32_t> size(n, 0), bundle(n, NONE);
+    for (uint32_t v = 0; v < n; v++) size[find(v)]++;
+    const uint32_t share = std::max(1u, std::min(128u, n / 256u));
+    uint32_t filled = 0, scene = 0, bundles = 0, last_scene = NONE;
+    for (uint32_t v = 0; v < n; v++) {
+        while (v >= (*m.scene_offsets)[scene + 1]) scene++;
+        if (root[v] != v) {
+            bundle[v] = bundle[find(v)];
+            continue;
+        }
+        if (bundles == 0 || scene != last_scene || filled + size[v] > share) {
+            bundles++;
+            filled = 0;
+        }
+        last_scene = scene;
+        filled += size[v];
+        bundle[v] = bundles - 1;
+    }
+    std::vector<std::vector<uint32_t>> parts(bundles), joints(bundles);
+    for (uint32_t v = 0; v < n; v++) parts[bundle[v]].push_back(v);
+    const uint32_t first = (uint32_t)m.joints->size();   // two-sided records follow the one-sided ones
+    for (uint32_t j = 0; j < m.joints2->size(); j++) joints[bundle[(*m.joints2)[j].p[0]]].push_back(first + j);
+    out = BundlePlan{};
+    out.n_bundles = bundles;
+    out.n_colors = nc;
+    uint32_t most = 1;   // threads a phase of a bundle can use
+    for (uint32_t b = 0; b < bundles; b++) {
+        out.part_off.push_back((uint32_t)out.parts.size());
+        out.joint_off.push_back((uint32_t)out.joints.size());
+        out.parts.insert(out.parts.end(), parts[b].begin(), parts[b].end());
+        out.joints.insert(out.joints.end(), joints[b].begin(), joints[b].end());
+        for (uint32_t c = 0; c < nc; c++) {
+            out.item_off.push_back((uint32_t)out.items.size());
+            for (uint32_t v : parts[b])
+                if (plan.item_kind[v] == 2 && plan.color[v] == c) out.items.push_back(plan.oitem_of[v]);
+            most = std::max(most, 2u * (uint32_t)(out.items.size() - out.item_off.back()));
+        }
+        out.item_off.push_back((uint32_t)out.items.size());
+    }
+    out.part_off.push_back((uint32_t)out.parts.size());
+    out.joint_off.push_back((uint32_t)out.joints.size());
+    out.block = (most + 63u) / 64u * 64u;
+    return bundles > 0 && most <= 512u;
+}
+
 }  // namespace avbd

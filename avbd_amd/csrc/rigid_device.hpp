@@ -2,8 +2,7 @@
 // Cosserat rod, rigid-body ground contact and one-sided fixed joint energies,
 // their start-of-step and per-iteration AL updates, the rotation parts of the
 // inertial / Chebyshev / velocity phases, and the 6x6 vertex block solve.
-// Included by vbd_kernels.hip (one translation unit, so the persistent step
-// kernel can inline every phase).
+// Included by vbd_kernels.hip.
 #pragma once
 
 #include "dyn_device.hpp"
@@ -24,13 +23,28 @@ struct CosStrain {
     float3 q_diff;   // q2 [-] q1
     float4 q_mid;    // q1 [+] q_diff / 2
     float e[6];      // shear/stretch, bend/twist strain
+    float h, sin_h, cos_h, sin_h2;   // h = |q_diff| / 2: sin h, cos h, sin(h / 2)
 };
 
+// With q_rel = q1^-1 q2 = (u, w): |u| = sin h and w = cos h, and the half
+// rotation q_rel^(1/2) = (u sin(h/2) / |u|, cos(h/2)) follows by square roots.  One
+// atan2 per element is left of nine sines, cosines and logarithms, whose
+// range reductions were most of an item's instructions.
 __device__ __forceinline__ CosStrain cos_strain(const CosRec& c, float3 p1, float3 p2, float4 q1, float4 q2) {
     CosStrain s;
     const float inv_L = 1.f / c.L;
-    s.q_diff = minus_s3(q2, q1);
-    s.q_mid = plus_s3(q1, scl(0.5f, s.q_diff));
+    const float4 rel = qmul(qconj(q1), q2);
+    const float3 u = xyz(rel);
+    const float vm = normv(u);
+    const bool tiny = vm < 1e-6f;   // as in log_s3
+    s.h = tiny ? vm : atan2f(vm, rel.w);
+    s.q_diff = scl(tiny ? 2.f : 2.f * s.h / vm, u);
+    s.sin_h = vm;
+    s.cos_h = tiny ? 1.f : rel.w;
+    const float a = sqrtf(0.5f * (1.f + fabsf(s.cos_h))), b = 0.5f * vm / a;
+    s.sin_h2 = s.cos_h >= 0.f ? b : a;
+    const float cos_h2 = s.cos_h >= 0.f ? a : b, k = tiny ? 0.5f : s.sin_h2 / vm;
+    s.q_mid = qnormalize(qmul(q1, make_float4(k * u.x, k * u.y, k * u.z, cos_h2)));
     const float3 d = qrot(qconj(s.q_mid), sub(p2, p1));
     s.e[0] = inv_L * d.x;
     s.e[1] = inv_L * d.y;
@@ -56,29 +70,40 @@ __device__ __forceinline__ void cos_accumulate(const CosRec& c, float3 p1, float
                                                uint32_t local, Vec6& G, Sym6& H) {
     const CosStrain s = cos_strain(c, p1, p2, q1, q2);
     const float inv_L = 1.f / c.L;
-    const M3f gam_inv = jr_inv(s.q_diff);
+    // J_r^-1(q_diff), J_r(q_diff / 2) and Exp(q_diff / 2) of rot_math.hpp from the
+    // sines and cosines of the strain
+    const float n = 2.f * s.h, n2 = n * n, h2 = s.h * s.h;
+    const float sinc_h = s.h < 1e-6f ? 1.f : s.sin_h / s.h, sinc_h2 = s.h < 1e-6f ? 1.f : 2.f * s.sin_h2 / s.h;
+    const float vers = 0.5f * sinc_h2 * sinc_h2;   // (1 - cos h) / h^2
+    const M3f gam_inv = so3_poly(1.f, 0.5f,
+                                 n < 0.5f ? (1.f / 12.f) + n2 * ((1.f / 720.f) + n2 * (1.f / 30240.f))
+                                          : 1.f / n2 - s.cos_h / (2.f * n * s.sin_h),
+                                 s.q_diff);
     const float3 theta = scl(0.5f, s.q_diff);
     const M3f R = qmat(s.q_mid);
     const M3f Rt = mtrans(R);
     const M3f S = skew(mvec(Rt, scl(inv_L, sub(p2, p1))));
-    const M3f gam_theta = jr(theta);
-    M3f A, B, C;
-    if (local == 0) {
-        const M3f git = mtrans(gam_inv);
-        A = mscale(-inv_L, Rt);
-        M3f inner = mtrans(exp_so3(theta));
-        const M3f gd = mmul(gam_theta, mscale(-0.5f, git));
+    const M3f gam_theta =
+        so3_poly(1.f, -vers,
+                 s.h < 0.5f ? (1.f / 6.f) - h2 * ((1.f / 120.f) - h2 * (1.f / 5040.f)) : (s.h - s.sin_h) / (h2 * s.h),
+                 theta);
+    // node 0: M = J_r^-T, B = S (Exp(theta)^T - gam_theta M / 2); node 1: M = J_r^-1,
+    // B = S gam_theta M / 2.  One code path with selects, since the two lanes of an
+    // item (solve_oitem) take one node each.
+    const bool first = local == 0;
+    const float sg = first ? -1.f : 1.f;
+    const M3f E = so3_poly(1.f, sinc_h, vers, theta);
+    M3f M;
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+    for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) inner.m[i][j] += gd.m[i][j];
-        B = mmul(S, inner);
-        C = mscale(-inv_L, git);
-    } else {
-        A = mscale(inv_L, Rt);
-        B = mmul(mmul(S, gam_theta), mscale(0.5f, gam_inv));
-        C = mscale(inv_L, gam_inv);
-    }
+        for (int j = 0; j < 3; j++) M.m[i][j] = first ? gam_inv.m[j][i] : gam_inv.m[i][j];
+    M3f inner = mmul(gam_theta, mscale(0.5f * sg, M));
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) inner.m[i][j] += first ? E.m[j][i] : 0.f;
+    const M3f A = mscale(sg * inv_L, Rt), B = mmul(S, inner), C = mscale(sg * inv_L, M);
     const float k[6] = {c.k0, c.k1, c.k2, c.k3, c.k4, c.k5};
     float ke[6];
 #pragma unroll
@@ -449,23 +474,49 @@ __device__ __forceinline__ void rotation_velocity(const DevState& d, uint32_t r,
     d.q_prev[r] = q;
 }
 
+// The value of the other lane of a pair.
+__device__ __forceinline__ float swap_pair(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+}
+
+// Rod element e of an item, with the particle at its other end.
+struct Element {
+    CosRec c;
+    uint32_t local, other, rot;
+};
+__device__ __forceinline__ Element read_element(const DevState& d, const OItem& it, uint32_t e) {
+    Element el;
+    const uint32_t code = d.oinc[it.inc_begin + e];
+    el.c = d.cos[code >> 1];
+    el.local = code & 1u;
+    el.other = el.local ? el.c.i0 : el.c.i1;
+    el.rot = (uint32_t)d.rot_of[el.other];
+    return el;
+}
+
 // Gradient and Hessian of every static energy on oriented particle it.v, in
 // the reference's StaticEnergyType order: Cosserat, ground (positional block),
 // rigid-ground, joint (simulation/VBDSolver.hpp:297-397).
-template <bool DYN = false>
+// W lanes (1 or 2) share the rod elements of the particle; every lane ends with
+// the whole sum, which for two elements is the sum of one lane bit for bit.
+// `read`: the lane's first element, when the caller has read it already.
+template <bool DYN = false, int W = 1>
 __device__ __forceinline__ void accumulate6(const DevState& d, const OItem& it, float3 pos, float4 q, Vec6& G,
-                                            Sym6& H) {
+                                            Sym6& H, uint32_t lane = 0, const Element* read = nullptr) {
     const uint32_t ncos = it.n_cos & ~VITEM_CONFLICT;
-    uint32_t k = it.inc_begin;
-    for (uint32_t e = 0; e < ncos; e++, k++) {
-        const uint32_t code = d.oinc[k];
-        const CosRec c = d.cos[code >> 1];
-        const uint32_t local = code & 1u;
-        const uint32_t other = local ? c.i0 : c.i1;
-        const float3 po = xyz(d.x[other]);
-        const float4 qo = d.q[d.rot_of[other]];
-        if (local == 0) cos_accumulate(c, pos, po, q, qo, 0, G, H);
-        else cos_accumulate(c, po, pos, qo, q, 1, G, H);
+    uint32_t k = it.inc_begin + ncos;
+    for (uint32_t e = lane; e < ncos; e += W) {
+        const Element el = e == lane && read ? *read : read_element(d, it, e);
+        const float3 po = xyz(d.x[el.other]);
+        const float4 qo = d.q[el.rot];
+        const bool first = el.local == 0;
+        cos_accumulate(el.c, first ? pos : po, first ? po : pos, first ? q : qo, first ? qo : q, el.local, G, H);
+    }
+    if constexpr (W == 2) {
+#pragma unroll
+        for (int i = 0; i < 6; i++) G.v[i] += swap_pair(G.v[i]);
+#pragma unroll
+        for (int i = 0; i < 21; i++) H.a[i] += swap_pair(H.a[i]);
     }
     if (it.ground >= 0) {
         // CollisionConstraintEnergySolver::accumulate<6> with the ground constraint: positional block only
@@ -512,9 +563,11 @@ __device__ __forceinline__ void accumulate6(const DevState& d, const OItem& it, 
     }
 }
 
-// _solveParticle<6> (simulation/VBDSolver.hpp:450-486): one thread per oriented vertex.
-template <bool DYN = false>
-__device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, float inv_dt2) {
+// _solveParticle<6> (simulation/VBDSolver.hpp:450-486): W lanes per oriented vertex
+// (lane W - 1 writes).
+template <bool DYN = false, int W = 1>
+__device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, float inv_dt2, uint32_t lane = 0,
+                                            const Element* read = nullptr) {
     const float4 xv = d.x[it.v];
     const float3 pos = xyz(xv);
     const float4 q = d.q[it.rot];
@@ -522,7 +575,7 @@ __device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, 
     Sym6 H;
     vec6_zero(G);
     sym6_zero(H);
-    accumulate6<DYN>(d, it, pos, q, G, H);
+    accumulate6<DYN, W>(d, it, pos, q, G, H, lane, read);
     const float md = xv.w * inv_dt2;
     const float3 I = xyz(d.inertia[it.rot]);
     const float3 yv = xyz(d.y[it.v]);
@@ -540,6 +593,7 @@ __device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, 
     lu6(H, b, dx);
     const float4 nx = make_float4(pos.x + dx[0], pos.y + dx[1], pos.z + dx[2], xv.w);
     const float4 nq = plus_s3(q, v3(dx[3], dx[4], dx[5]));
+    if (lane != W - 1) return;
     if (it.n_cos & VITEM_CONFLICT) {
         d.x_buf[it.v] = nx;
         d.q_buf[it.rot] = nq;

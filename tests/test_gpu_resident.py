@@ -85,3 +85,29 @@ def test_resident_stops_where_one_launch_per_phase_stops(kind, n, check):
         assert (s.steps_at_budget, s.vertex_updates) == (s0.steps_at_budget, s0.vertex_updates)
         assert np.array_equal(r.ctx.scene_iterations(), runs[0].ctx.scene_iterations())
         assert np.array_equal(r.positions(), runs[0].positions())
+
+
+# one element; bundles of several short rods with a remainder; components of
+# more particles than a bundle's share; a phase of more pairs than one
+# workgroup holds (there is then one launch per phase)
+@pytest.mark.parametrize("nx,nz,segments,jointed", [(1, 1, 1, False), (3, 3, 2, True), (5, 7, 9, False), (2, 2, 200, True),
+                                                    (1, 1, 600, False)])
+def test_bundles_of_rods_match_one_launch_per_phase(nx, nz, segments, jointed, oracle):
+    """Oriented particles: the bundles' solve adds the two elements of a node in
+    two lanes, so it differs from one launch per phase by the rounding of
+    that sum; against the float64 oracle neither may be much further off than the
+    other (twice, plus 1e-6 of the size: a few roundings of a position of 1)."""
+    from avbd_amd.sim import Simulation
+    print(f"[gpu-test] bundles {nx}x{nz} rods of {segments} jointed {jointed}", flush=True)
+    sc = scenes.rod_grid(nx, nz, segments, iters=5, tip_joint=jointed)
+    o = oracle.from_scene(sc)
+    o.step(3)
+    xo, err = o.positions(), []
+    for kw in (dict(flags=_lib.FLAG_NO_PERSISTENT), dict(), dict(use_graph=False)):
+        s = Simulation(sc, **kw)
+        s.setup()
+        s.update(3)
+        err.append(np.abs(s.positions() - xo).max())
+    print(f"[gpu-test]   off the oracle: per phase {err[0]:.2e}, bundles {err[1]:.2e}", flush=True)
+    assert err[1] <= 2 * err[0] + 1e-6
+    assert err[1] == err[2]
