@@ -514,6 +514,7 @@ void alloc_lbvh(avbd_ctx* c, LbvhDev& b, uint32_t n) {
     b.bucket_count = dev_alloc<uint32_t>(c, 1u << 13);
     b.bucket_offset = dev_alloc<uint32_t>(c, (1u << 13) + 1);
     b.slots = dev_alloc<uint32_t>(c, n);
+    b.slot_keys = dev_alloc<uint64_t>(c, n);
     b.table = dev_alloc<double>(c, 6 * (size_t)lbvh_table_entries(n));
     b.node_box = dev_alloc<double>(c, 6 * (size_t)nn);
     b.trav = dev_alloc<TravNode>(c, n > 1 ? n - 1 : 1);

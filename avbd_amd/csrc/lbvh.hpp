@@ -34,12 +34,13 @@ struct LbvhDev {
     uint32_t* bucket_count = nullptr;    // 8,192 (zeroed by the build)
     uint32_t* bucket_offset = nullptr;   // 8,193
     uint32_t* slots = nullptr;           // n: primitives grouped by bucket
+    uint64_t* slot_keys = nullptr;       // n: their codes
     double* table = nullptr;        // aligned range unions, 6 per entry (lbvh_table_entries)
     double* node_box = nullptr;     // 6 per node
     TravNode* trav = nullptr;       // n - 1 internal nodes (record g - n of node g)
     uint32_t* pairs = nullptr;      // candidate leaf pairs (a < b)
     uint32_t pair_cap = 0;
-    uint32_t* counters = nullptr;   // [0] pair count, [1] status (bit0 stack overflow)
+    uint32_t* counters = nullptr;   // [0] pair count, [1] status (unused: the stack holds any tree)
 };
 
 uint32_t lbvh_table_entries(uint32_t n);

@@ -38,7 +38,7 @@ constexpr uint32_t table_entries(uint32_t n) {
 // Byte offsets of the LBVH arrays for n triangles inside the scratch array;
 // the counters and the pair list are the caller's output buffers.
 struct Carve {
-    size_t aabb, sbox, keys, keys_sorted, sorted, left, right, parent, range_hi, bcount, boffset, slots, table,
+    size_t aabb, sbox, keys, keys_sorted, sorted, left, right, parent, range_hi, bcount, boffset, slots, slot_keys, table,
         node_box, trav, total;
 };
 
@@ -58,6 +58,7 @@ constexpr Carve carve(uint32_t n) {
     c.bcount = o;      o += align256(sizeof(uint32_t) * kBuckets);
     c.boffset = o;     o += align256(sizeof(uint32_t) * (kBuckets + 1));
     c.slots = o;       o += align256(sizeof(uint32_t) * (size_t)n);
+    c.slot_keys = o;   o += align256(sizeof(uint64_t) * (size_t)n);
     c.table = o;       o += align256(6 * sizeof(double) * (size_t)table_entries(n));
     c.node_box = o;    o += align256(6 * sizeof(double) * nn);
     c.trav = o;        o += align256(sizeof(TravNode) * (size_t)(n > 1 ? n - 1 : 1));
@@ -143,6 +144,7 @@ extern "C" int avbd_detect_collisions_noalloc(const float* x4, const float* v4, 
         b.bucket_count = reinterpret_cast<uint32_t*>(base + c.bcount);
         b.bucket_offset = reinterpret_cast<uint32_t*>(base + c.boffset);
         b.slots = reinterpret_cast<uint32_t*>(base + c.slots);
+        b.slot_keys = reinterpret_cast<uint64_t*>(base + c.slot_keys);
         b.table = reinterpret_cast<double*>(base + c.table);
         b.node_box = reinterpret_cast<double*>(base + c.node_box);
         b.trav = reinterpret_cast<TravNode*>(base + c.trav);

@@ -194,3 +194,35 @@ def test_gpu_concurrent_broadphase_matches_serial(oracle):
         ga, gb = _gpu_bvh(a.ctx, n), _gpu_bvh(b.ctx, n)
         assert set(map(tuple, ga["pairs"].tolist())) == set(map(tuple, gb["pairs"].tolist()))
         assert np.array_equal(ga["left"], gb["left"]) and np.array_equal(ga["node_box"], gb["node_box"])
+
+
+# one leaf, one node, fewer leaves than a node's 16 lanes and one more, a second
+# table kernel (above 256), another round of the searches (above 4,096);
+# `same`: identical triangles, whose codes tie, so that the hierarchy is that of
+# the indices and every pair overlaps
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,same", [(1, False), (2, False), (3, True), (16, False), (17, True), (90, True), (257, False),
+                                    (5000, False)])
+def test_gpu_lbvh_at_the_edges_of_its_lane_groups(oracle, n, same):
+    from avbd_amd.sim import SimulationContext
+    from avbd_amd._lib import lib, check
+    import ctypes as C
+    print(f"[gpu-test] lbvh of {n} triangles, same {same}", flush=True)
+    rng = np.random.default_rng(n)
+    corners = rng.uniform(0, 1, (1 if same else n, 1, 3)) + rng.uniform(-0.04, 0.04, (1 if same else n, 3, 3))
+    x = np.broadcast_to(corners, (n, 3, 3)).reshape(-1, 3).astype(np.float32).astype(np.float64)
+    tris = np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+    ctx = SimulationContext(dt=1 / 60, solver_iters=1)
+    ctx.add_particles(x, mass=np.ones(3 * n))
+    check(lib.avbd_add_collision_triangles(ctx.handle, n, tris.ctypes.data_as(C.POINTER(C.c_uint32))), ctx.handle)
+    ctx.build_graph()
+    check(lib.avbd_detect_collisions(ctx.handle), ctx.handle)
+    xs, v = ctx.state()
+    g, o = _gpu_bvh(ctx, n), oracle.lbvh_build(tris, xs, v, 1 / 60)
+    for k in ("morton", "sorted", "left", "right", "parent", "root", "node_box"):
+        assert np.array_equal(g[k], o[k]), k
+    got = set(map(tuple, np.asarray(g["pairs"]).tolist()))
+    assert len(got) == len(g["pairs"])
+    assert got == (set(map(tuple, oracle.lbvh_self_pairs(o).tolist())) if n > 1 else set())
+    if same:
+        assert len(got) == n * (n - 1) // 2
