@@ -136,7 +136,11 @@ struct avbd_ctx {
     LbvhDev lbd;                   // LBVH over every primitive
     DetRec* d_det = nullptr;
     uint32_t det_cap = 0;
-    uint32_t* d_status = nullptr;  // [0] narrow-phase flags, [1] detected count
+    // [0] narrow-phase flags, [1] detected count, [2], [3] the broad phase's counters; the records follow
+    uint32_t* d_status = nullptr;
+    uint8_t* h_det = nullptr;      // pinned: the header and the first records
+    uint32_t *d_active = nullptr, *d_seeds = nullptr;   // of the last round sent
+    bool contacts_sent = false;    // the device holds the contact system's current arrays
     RecolourDev rdev;              // device recolouring and work-list layout
     uint32_t* h_layout = nullptr;  // pinned: the 3 x 257 per-colour offsets, then the 5 recolouring counters
     // dynamic contacts: a detection round has changed the colours or the
@@ -147,7 +151,7 @@ struct avbd_ctx {
         void* p = nullptr;
         size_t bytes = 0;
     };
-    Grow g_ops, g_active, g_off, g_ent, g_nboff, g_nb, g_seeds;
+    Grow g_round, g_active, g_off, g_ent;
     // residual mode with dynamic contacts: what the captured step graphs
     // were recorded with (launch sizes and device buffers); they are
     // captured again when a detection round changes any of it
@@ -155,7 +159,7 @@ struct avbd_ctx {
     // pinned staging for a detection round's uploads (written only after the
     // round's stream synchronisation, so one buffer serves every round)
     uint8_t* stage = nullptr;
-    size_t stage_cap = 0, stage_used = 0;
+    size_t stage_cap = 0;
 
     // iterations per step: the budget in residual mode, else solver_iters
     uint32_t iters() const { return res_tol > 0 ? res_max_iters : desc.solver_iters; }
@@ -617,7 +621,7 @@ void enqueue_head(avbd_ctx* c, bool with_events) {
     // dynamic contacts' updateAfterTimeStep reads the start-of-step positions
     const uint32_t n_active = c->dynamic ? (uint32_t)c->cs.active.size() : 0u;
     if (n_active) {
-        const uint32_t* act = static_cast<const uint32_t*>(c->g_active.p);
+        const uint32_t* act = c->d_active;
         if (c->fp64) launch_dyn_step_begin_f64(s, f64_state(c), act, n_active);
         else launch_dyn_step_begin(s, c->d, act, n_active);
     }
@@ -659,7 +663,7 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
     hipStream_t s = c->stream;
     const uint32_t* done = c->rc ? &c->rc->done : nullptr;
     const ResCtl* rc = c->rc;
-    const uint32_t* d_active = static_cast<const uint32_t*>(c->g_active.p);
+    const uint32_t* d_active = c->d_active;
     const uint32_t n_active = c->dynamic ? (uint32_t)c->cs.active.size() : 0u;
     // a dynamic-contact step with no active contact on the set-up work list
     // is the static step: the static kernels, fused as at set-up
@@ -864,7 +868,7 @@ void dyn_residual_graphs(avbd_ctx* c) {
     key.insert(key.end(), p.conflict_offsets.begin(), p.conflict_offsets.end());
     key.push_back(c->cs.active.size());
     key.push_back(dyn_quiet(c) ? 1u : 0u);
-    for (const void* ptr : {(const void*)c->g_active.p, (const void*)c->d.dyn_off, (const void*)c->d.dyn_ent})
+    for (const void* ptr : {(const void*)c->d_active, (const void*)c->d.dyn_off, (const void*)c->d.dyn_ent})
         key.push_back((uint64_t)(uintptr_t)ptr);
     if (c->head_exec && key == c->dyn_graph_key) return;
     destroy_graph(c);
@@ -913,11 +917,9 @@ void run_residual_step(avbd_ctx* c, bool graphs) {
     else enqueue_tail(c, false);
 }
 
-// Pinned staging of a detection round's host arrays: reserve the round's
-// total first (may reallocate: the stream is idle then), then each array is
-// copied in and sent with a truly asynchronous H2D copy.
+// Pinned staging of a detection round's host arrays (may reallocate: the
+// stream is idle then).
 void stage_reserve(avbd_ctx* c, size_t bytes) {
-    c->stage_used = 0;
     if (bytes <= c->stage_cap) return;
     if (c->stage) hip_check(hipHostFree(c->stage), "hipHostFree");
     c->stage = nullptr;
@@ -930,18 +932,8 @@ void stage_reserve(avbd_ctx* c, size_t bytes) {
 }
 
 constexpr size_t kStageAlign = 256;
-inline size_t stage_bytes(size_t bytes) { return (bytes + kStageAlign - 1) / kStageAlign * kStageAlign; }
-
-template <class T>
-void stage_upload(avbd_ctx* c, T* dst, const std::vector<T>& src) {
-    if (src.empty()) return;
-    const size_t bytes = src.size() * sizeof(T);
-    if (c->stage_used + stage_bytes(bytes) > c->stage_cap) throw std::logic_error("staging buffer overrun");
-    uint8_t* p = c->stage + c->stage_used;
-    std::memcpy(p, src.data(), bytes);
-    c->stage_used += stage_bytes(bytes);
-    hip_check(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, c->stream), "hipMemcpyAsync H2D");
-}
+constexpr size_t kDetHeader = 64;   // bytes before the detected records
+constexpr size_t kDetFirst = 128;   // records that come back with the header
 
 // One round of CollisionDetector::detectCollisionsAndRecolor_Parallel
 // (collision/CollisionDetector.cpp:57-129) at the start of a step: device
@@ -954,9 +946,8 @@ void stage_upload(avbd_ctx* c, T* dst, const std::vector<T>& src) {
 // them.
 void read_layout(avbd_ctx* c) {
     hipStream_t s = c->stream;
-    hip_check(hipMemcpyAsync(c->h_layout, c->rdev.offsets, 3 * 257 * sizeof(uint32_t), hipMemcpyDeviceToHost, s),
-              "D2H");
-    hip_check(hipMemcpyAsync(c->h_layout + 3 * 257, c->rdev.counters, 5 * sizeof(uint32_t), hipMemcpyDeviceToHost, s),
+    // (the counters follow the offsets in memory)
+    hip_check(hipMemcpyAsync(c->h_layout, c->rdev.offsets, (3 * 257 + 5) * sizeof(uint32_t), hipMemcpyDeviceToHost, s),
               "D2H");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     const uint32_t* cnt = c->h_layout + 3 * 257;
@@ -986,52 +977,70 @@ void detect_round(avbd_ctx* c) {
     launch_lbvh_tree(s, c->lbd);
     launch_narrow(s, c->dp, c->lbd, c->d, dt, c->cs.margin, c->d_det, c->det_cap, c->d_status);
     hip_check(hipGetLastError(), "kernel launch");
-    uint32_t st[4] = {0, 0, 0, 0};
-    hip_check(hipMemcpyAsync(st, c->d_status, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s), "D2H");
-    hip_check(hipMemcpyAsync(st + 2, c->lbd.counters, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, s), "D2H");
+    // the flags, the pair counter and the first records come back in one copy
+    hip_check(hipMemcpyAsync(c->h_det, c->d_status, kDetHeader + kDetFirst * sizeof(DetRec), hipMemcpyDeviceToHost, s),
+              "D2H");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    const uint32_t* st = reinterpret_cast<const uint32_t*>(c->h_det);
     if (st[2] > c->lbd.pair_cap || (st[3] & 1u))
         throw CodeError(AVBD_E_CAPACITY, "broad phase: candidate pairs exceeded capacity");
     if (st[0] & NARROW_UNSUPPORTED) throw CodeError(AVBD_E_UNSUPPORTED_CONTACT, "Unsupported collision!");
     if (st[1] > c->det_cap) throw CodeError(AVBD_E_CAPACITY, "narrow phase: detected contacts exceeded capacity");
     std::vector<DetRec> det(st[1]);
-    if (!det.empty()) {
-        hip_check(hipMemcpyAsync(det.data(), c->d_det, det.size() * sizeof(DetRec), hipMemcpyDeviceToHost, s), "D2H");
+    const size_t first = std::min<size_t>(det.size(), kDetFirst);
+    if (first) std::memcpy(static_cast<void*>(det.data()), c->h_det + kDetHeader, first * sizeof(DetRec));
+    if (det.size() > first) {
+        hip_check(hipMemcpyAsync(det.data() + first, c->d_det + first, (det.size() - first) * sizeof(DetRec),
+                                 hipMemcpyDeviceToHost, s),
+                  "D2H");
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     }
-    c->cs.process(det, c->prims, c->mass, dt);
     ContactSystem& cs = c->cs;
-    // the stream is idle here (synchronised above): reserve the staging for
-    // every upload of this round, then queue them; the recolouring and the
-    // solve follow on the same stream
-    const size_t total = stage_bytes(cs.ops.size() * sizeof(DynOp)) + stage_bytes(cs.active.size() * sizeof(uint32_t)) +
-                         stage_bytes(cs.dyn_off.size() * sizeof(uint32_t)) +
-                         stage_bytes(cs.dyn_ent.size() * sizeof(uint32_t)) +
-                         stage_bytes(cs.nb_off.size() * sizeof(uint32_t)) + stage_bytes(cs.nb.size() * sizeof(uint32_t)) +
-                         stage_bytes(cs.seeds.size() * sizeof(uint32_t));
-    stage_reserve(c, total);
-    if (!cs.ops.empty()) {
-        auto* d_ops = static_cast<DynOp*>(grow(c, c->g_ops, cs.ops.size() * sizeof(DynOp)));
-        stage_upload(c, d_ops, cs.ops);
-        launch_dyn_apply(s, c->d, d_ops, (uint32_t)cs.ops.size());
+    const bool sent = c->contacts_sent;
+    c->contacts_sent = false;   // (also when the next line throws)
+    if (cs.process(det, c->prims, c->mass, dt) || !sent) {
+        // the stream is idle here (synchronised above): the round's arrays are
+        // staged side by side and go up in one copy (seven took 10 us each);
+        // the recolouring and the solve follow on the same stream.  Arrays of
+        // changing length get room in steps, so that they rarely move (captured
+        // graphs hold their addresses).
+        constexpr size_t kRoom = 16384;
+        size_t total = 0;
+        auto place = [&](size_t bytes, size_t step) {
+            const size_t at = total;
+            total += (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+            return at;
+        };
+        auto bytes = [](const auto& v) { return v.size() * sizeof(v[0]); };
+        const size_t o_off = place(bytes(cs.dyn_off), kStageAlign), o_nboff = place(bytes(cs.nb_off), kStageAlign),
+                     o_act = place(bytes(cs.active), kRoom), o_ent = place(bytes(cs.dyn_ent), kRoom),
+                     o_nb = place(bytes(cs.nb), kRoom), o_seeds = place(bytes(cs.seeds), kRoom),
+                     o_ops = place(bytes(cs.ops), kStageAlign);
+        stage_reserve(c, total);
+        auto stage = [&](size_t at, const auto& v) {
+            if (!v.empty()) std::memcpy(c->stage + at, v.data(), bytes(v));
+        };
+        stage(o_off, cs.dyn_off);
+        stage(o_nboff, cs.nb_off);
+        stage(o_act, cs.active);
+        stage(o_ent, cs.dyn_ent);
+        stage(o_nb, cs.nb);
+        stage(o_seeds, cs.seeds);
+        stage(o_ops, cs.ops);
+        auto* d = static_cast<uint8_t*>(grow(c, c->g_round, total));
+        hip_check(hipMemcpyAsync(d, c->stage, o_ops + bytes(cs.ops), hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+        if (!cs.ops.empty())
+            launch_dyn_apply(s, c->d, reinterpret_cast<DynOp*>(d + o_ops), (uint32_t)cs.ops.size());
+        auto words = [&](size_t at) { return reinterpret_cast<uint32_t*>(d + at); };
+        c->d_active = words(o_act);
+        c->d.dyn_off = words(o_off);
+        c->d.dyn_ent = words(o_ent);
+        c->rdev.d_off = words(o_nboff);
+        c->rdev.d_nb = words(o_nb);
+        c->d_seeds = words(o_seeds);
     }
-    auto* d_act = static_cast<uint32_t*>(grow(c, c->g_active, cs.active.size() * sizeof(uint32_t)));
-    stage_upload(c, d_act, cs.active);
-    auto* d_off = static_cast<uint32_t*>(grow(c, c->g_off, cs.dyn_off.size() * sizeof(uint32_t)));
-    stage_upload(c, d_off, cs.dyn_off);
-    auto* d_ent = static_cast<uint32_t*>(grow(c, c->g_ent, cs.dyn_ent.size() * sizeof(uint32_t)));
-    stage_upload(c, d_ent, cs.dyn_ent);
-    c->d.dyn_off = d_off;
-    c->d.dyn_ent = d_ent;
+    c->contacts_sent = true;
     // incremental recolouring and the new work list, on the device
-    auto* d_nboff = static_cast<uint32_t*>(grow(c, c->g_nboff, cs.nb_off.size() * sizeof(uint32_t)));
-    stage_upload(c, d_nboff, cs.nb_off);
-    auto* d_nb = static_cast<uint32_t*>(grow(c, c->g_nb, std::max<size_t>(cs.nb.size(), 1) * sizeof(uint32_t)));
-    stage_upload(c, d_nb, cs.nb);
-    auto* d_seeds = static_cast<uint32_t*>(grow(c, c->g_seeds, std::max<size_t>(cs.seeds.size(), 1) * sizeof(uint32_t)));
-    stage_upload(c, d_seeds, cs.seeds);
-    c->rdev.d_off = d_nboff;
-    c->rdev.d_nb = d_nb;
     // no new contact, nothing left dirty or conflicted by the last round: the
     // recolouring would change nothing (ColorList only recolours from dirty
     // particles), so the colours, the work list and its offsets stand
@@ -1040,7 +1049,7 @@ void detect_round(avbd_ctx* c) {
         hip_check(hipGetLastError(), "kernel launch");
         return;
     }
-    launch_recolour(s, c->rdev, d_seeds, (uint32_t)cs.seeds.size());
+    launch_recolour(s, c->rdev, c->d_seeds, (uint32_t)cs.seeds.size());
     launch_relayout(s, c->rdev, c->d.items, c->d.oitems, c->d_conflicts, false);
     hip_check(hipGetLastError(), "kernel launch");
     read_layout(c);
@@ -1397,6 +1406,7 @@ void avbd_destroy(avbd_ctx* c) {
     for (auto ev : c->part_ev) (void)hipEventDestroy(ev);
     if (c->h_conv) (void)hipHostFree(c->h_conv);
     if (c->h_layout) (void)hipHostFree(c->h_layout);
+    if (c->h_det) (void)hipHostFree(c->h_det);
     if (c->stage) (void)hipHostFree(c->stage);
     if (c->ev_lb0) (void)hipEventDestroy(c->ev_lb0);
     if (c->ev_lb1) (void)hipEventDestroy(c->ev_lb1);
@@ -3105,11 +3115,21 @@ int avbd_set_dynamic_contacts(avbd_ctx* c, double margin, uint32_t capacity) {
         upload(c, c->dp.object, ob);
         upload(c, c->dp.radius, rad);
         c->det_cap = c->lbd.pair_cap;
-        c->d_det = dev_alloc<DetRec>(c, c->det_cap);
-        c->d_status = dev_alloc<uint32_t>(c, 2);
+        // flags and counters, then the records: one block, read back in one copy
+        auto* block = dev_alloc<uint8_t>(c, kDetHeader + std::max<size_t>(c->det_cap, kDetFirst) * sizeof(DetRec));
+        c->d_status = reinterpret_cast<uint32_t*>(block);
+        c->d_det = reinterpret_cast<DetRec*>(block + kDetHeader);
+        c->lbd.counters = c->d_status + 2;
+        if (!c->h_det) {
+            void* hd = nullptr;
+            hip_check(hipHostMalloc(&hd, kDetHeader + kDetFirst * sizeof(DetRec), hipHostMallocDefault),
+                      "hipHostMalloc");
+            c->h_det = static_cast<uint8_t*>(hd);
+        }
         c->d.dyn = dev_alloc<DynRec>(c, DYN_KINDS * (size_t)cap);
         if (c->fp64) c->f.x_buf = dev_alloc<double4>(c, n);   // conflicted particles' buffered positions
         c->cs.init(n, cap, margin);
+        c->contacts_sent = false;
         auto* d_off = static_cast<uint32_t*>(grow(c, c->g_off, (n + 1) * sizeof(uint32_t)));
         upload(c, d_off, c->cs.dyn_off);
         c->d.dyn_off = d_off;
@@ -3127,8 +3147,8 @@ int avbd_set_dynamic_contacts(avbd_ctx* c, double margin, uint32_t capacity) {
         r.touched = dev_alloc<uint32_t>(c, 7 * (size_t)n);
         r.touched_conf = dev_alloc<uint32_t>(c, n);
         r.conflicted = dev_alloc<uint32_t>(c, n);
-        r.counters = dev_alloc<uint32_t>(c, 8);
-        r.offsets = dev_alloc<uint32_t>(c, 3 * 257);
+        r.offsets = dev_alloc<uint32_t>(c, 3 * 257 + 8);
+        r.counters = r.offsets + 3 * 257;
         upload(c, r.color, plan.color);
         c->setup_color = plan.color;
         c->layout_changed = false;
@@ -3389,8 +3409,10 @@ int avbd_load_checkpoint(avbd_ctx* c, const void* buf, uint64_t size) {
             upload(c, d_off, c->cs.dyn_off);
             auto* d_ent = static_cast<uint32_t*>(grow(c, c->g_ent, c->cs.dyn_ent.size() * sizeof(uint32_t)));
             upload(c, d_ent, c->cs.dyn_ent);
+            c->d_active = d_act;
             c->d.dyn_off = d_off;
             c->d.dyn_ent = d_ent;
+            c->contacts_sent = false;   // (without the adjacency)
         }
         c->steps_taken = h.steps_taken;
         c->vertex_updates = h.vertex_updates;

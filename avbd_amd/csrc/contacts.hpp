@@ -96,8 +96,9 @@ public:
     // Merge this round's detected contacts (any order) with the previous
     // round's and rebuild the dynamic adjacency.  Fills ops / active /
     // dyn_off / dyn_ent / nb_off / nb and the particles of the added contacts
-    // (seeds), which the device recolouring marks dirty.
-    void process(std::vector<DetRec>& det, const std::vector<HostPrim>& prims, const std::vector<double>& mass,
+    // (seeds), which the device recolouring marks dirty.  False when nothing was
+    // or is in contact: every array stays as it was.
+    bool process(std::vector<DetRec>& det, const std::vector<HostPrim>& prims, const std::vector<double>& mass,
                  double dt);
 
     std::vector<DynOp> ops;

@@ -73,10 +73,11 @@ void ContactSystem::init(uint32_t n_particles, uint32_t capacity, double collisi
     active.clear();
 }
 
-void ContactSystem::process(std::vector<DetRec>& det, const std::vector<HostPrim>& prims,
+bool ContactSystem::process(std::vector<DetRec>& det, const std::vector<HostPrim>& prims,
                             const std::vector<double>& mass, double dt) {
     ops.clear();
     seeds.clear();
+    if (det.empty() && prev.empty() && active.empty()) return false;
     // _handleDetectedCollisions (collision/CollisionDetector.cpp:272-327): key order
     std::sort(det.begin(), det.end(), [](const DetRec& a, const DetRec& b) { return a.key < b.key; });
     std::vector<Entry> cur(det.size());
@@ -194,6 +195,7 @@ void ContactSystem::process(std::vector<DetRec>& det, const std::vector<HostPrim
             }
         }
     }
+    return true;
 }
 
 namespace {
