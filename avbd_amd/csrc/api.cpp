@@ -1055,9 +1055,6 @@ void detect_round(avbd_ctx* c) {
     read_layout(c);
 }
 
-// Autotuner: time the colour-phase solve of one iteration for each candidate
-// (lanes per vertex, block size), writing into a scratch sink so that the
-// state is untouched, and keep the fastest.
 // Temporary device buffers, freed when the holder goes out of scope.
 struct DevTemp {
     std::vector<void*> ptrs;
@@ -1122,21 +1119,21 @@ void solve_into_scratch(avbd_ctx* c, const LaunchCfg& cfg, uint32_t b, uint32_t 
     }
 }
 
-// Lanes per vertex, block size and gather batch: time every candidate on
-// the scene's colour phases and keep the fastest.
+// Block size and gather batch: time every candidate on the scene's colour
+// phases and keep the fastest.  Neither changes a result.  The lanes per vertex
+// do (the order of a vertex's sum), so they are not timed but given or 8: timing
+// chose 8 for a batch of cubes and 4 or 16, by chance, for a block under spheres,
+// where a context rebuilt from a checkpoint could then go on with other roundings.
 void autotune(avbd_ctx* c) {
-    const uint32_t lanes_c[] = {4, 8, 16, 32};
     const uint32_t block_c[] = {64, 128, 256};
     const uint32_t batch_c[] = {1, 2, 4};
     float best = 1e30f;
     LaunchCfg best_cfg = c->cfg;
-    for (uint32_t L : lanes_c) {
-        if (c->desc.lanes_per_vertex && L != c->desc.lanes_per_vertex) continue;
-        for (uint32_t B : block_c)
+    for (uint32_t B : block_c)
         for (uint32_t U : batch_c) {
             if (c->desc.block_size && B != c->desc.block_size) continue;
             if (c->desc.gather_batch && U != c->desc.gather_batch) continue;
-            LaunchCfg cfg{L, B, U};
+            const LaunchCfg cfg{c->cfg.lanes, B, U};
             auto run = [&] {
                 for (uint32_t col = 0; col < c->plan.num_colors; col++) {
                     const uint32_t b = c->plan.item_offsets[col], e = c->plan.item_offsets[col + 1];
@@ -1155,7 +1152,6 @@ void autotune(avbd_ctx* c) {
                 best_cfg = cfg;
             }
         }
-    }
     c->cfg = best_cfg;
 }
 
