@@ -1299,9 +1299,9 @@ void setup_resident(avbd_ctx* c) {
     r.lds_bytes = plan.lds_bytes;
     r.max_cluster = plan.max_cluster;
     resident_shape(plan, c->plan.num_colors, lim, c->desc.lanes_per_vertex, r.lanes, r.block);
-    // 10 ms: what the scene costs alone, so that waiting at most doubles a launch
-    // that another stream's work keeps from being resident
-    r.gather_ticks = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 1000000u;
+    // 50 ms: half of what 100 iterations of a large scene take alone (1 ms each at
+    // 32^3), so that waiting for another stream's work costs less than giving up
+    r.gather_ticks = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 5000000u;
     r.has_ground = lim.ground;
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     c->resident = true;
