@@ -358,35 +358,19 @@ JointRec to_dev(const HostJoint2& h) {
     return r;
 }
 
-// Edge constants of a tet (EdgeRec), in FP64 from Q, V lambda, V mu and alpha.
-TetEdges<double> edges_of(const double* Q, double VL, double VM, double alpha) {
+// Edge constants of a tet (EdgeRec64), in FP64 from the device's FP32 record.
+TetEdges tet_edges(const TetRec& r) {
+    const double VL = r.VL, VM = r.VM, alpha = r.alpha;
     double q[4][3];
     for (int j = 0; j < 3; j++) {
-        for (int a = 0; a < 3; a++) q[a][j] = Q[3 * a + j];
+        for (int a = 0; a < 3; a++) q[a][j] = r.q[3 * a + j];
         q[3][j] = -(q[0][j] + q[1][j] + q[2][j]);
     }
     const double det = q[0][0] * (q[1][1] * q[2][2] - q[1][2] * q[2][1]) -
                        q[0][1] * (q[1][0] * q[2][2] - q[1][2] * q[2][0]) +
                        q[0][2] * (q[1][0] * q[2][1] - q[1][1] * q[2][0]);
     auto w = [&](int a, int b) { return VM * (q[a][0] * q[b][0] + q[a][1] * q[b][1] + q[a][2] * q[b][2]); };
-    return TetEdges<double>{{w(0, 1), w(0, 2), w(0, 3), w(1, 2), w(1, 3), w(2, 3)}, VL * det * det, VL * det * alpha};
-}
-
-// FP32 state: rounded once from the staged FP64 material.
-TetEdges<float> tet_edges(const HostNH& t) {
-    const TetEdges<double> e = edges_of(t.Q, t.V * t.lambda, t.V * t.mu, t.mu / t.lambda + 1.0);
-    TetEdges<float> f;
-    for (int k = 0; k < 6; k++) f.w[k] = (float)e.w[k];
-    f.h = (float)e.h;
-    f.b = (float)e.b;
-    return f;
-}
-
-// FP64 state: from the device's FP32 record, which defines the model there.
-TetEdges<double> tet_edges(const TetRec& r) {
-    double Q[9];
-    for (int k = 0; k < 9; k++) Q[k] = r.q[k];
-    return edges_of(Q, r.VL, r.VM, r.alpha);
+    return TetEdges{{w(0, 1), w(0, 2), w(0, 3), w(1, 2), w(1, 3), w(2, 3)}, VL * det * det, VL * det * alpha};
 }
 
 // Append one particle to the FP64 staging pools (ParticlePool::addParticle).
@@ -2114,16 +2098,26 @@ int avbd_build_graph(avbd_ctx* c) {
             // per-incidence records (work-item order) for the vertex solve
             if (n >= (1u << 30)) throw std::runtime_error("more than 2^30 particles");
             const std::vector<uint32_t>& inc = c->plan.inc;
-            auto put = [&](auto& rec, const auto& e, size_t k) {
-                const uint32_t t = inc[k] >> 2, a = inc[k] & 3u;
-                for (int j = 0; j < 3; j++) {
-                    rec.w[j] = e.w[kEdgeWeight[a][j]];
-                    rec.i[j] = tr[t].idx[kEdgeCorner[a][j]];
+            if (c->fp64 && !c->damping) {
+                std::vector<TetEdges> te(d.n_tets);
+                for (uint32_t t = 0; t < d.n_tets; t++) te[t] = tet_edges(tr[t]);
+                std::vector<EdgeRec64> er(inc.size());
+                for (size_t k = 0; k < er.size(); k++) {
+                    const uint32_t t = inc[k] >> 2, a = inc[k] & 3u;
+                    for (int j = 0; j < 3; j++) {
+                        er[k].w[j] = te[t].w[kEdgeWeight[a][j]];
+                        er[k].i[j] = tr[t].idx[kEdgeCorner[a][j]];
+                    }
+                    er[k].h = te[t].h;
+                    er[k].b = te[t].b;
                 }
-                rec.h = e.h;
-                rec.b = e.b;
-            };
-            if (c->damping) {
+                EdgeRec64* p = dev_alloc<EdgeRec64>(c, er.size());
+                upload(c, p, er);
+                c->f.erec = p;
+                TetEdges* pe = dev_alloc<TetEdges>(c, te.size());
+                upload(c, pe, te);
+                c->res.edges = pe;
+            } else {
                 std::vector<TetRec> ir(inc.size());
                 for (size_t k = 0; k < ir.size(); k++) {
                     ir[k] = tr[inc[k] >> 2];
@@ -2131,27 +2125,6 @@ int avbd_build_graph(avbd_ctx* c) {
                 }
                 d.irec = dev_alloc<TetRec>(c, ir.size());
                 upload(c, d.irec, ir);
-            } else if (c->fp64) {
-                std::vector<TetEdges<double>> te(d.n_tets);
-                for (uint32_t t = 0; t < d.n_tets; t++) te[t] = tet_edges(tr[t]);
-                std::vector<EdgeRec64> er(inc.size());
-                for (size_t k = 0; k < er.size(); k++) put(er[k], te[inc[k] >> 2], k);
-                EdgeRec64* p = dev_alloc<EdgeRec64>(c, er.size());
-                upload(c, p, er);
-                c->f.erec = p;
-                TetEdges<double>* pe = dev_alloc<TetEdges<double>>(c, te.size());
-                upload(c, pe, te);
-                c->res.edges = pe;
-            } else {
-                std::vector<TetEdges<float>> te(d.n_tets);
-                for (uint32_t t = 0; t < d.n_tets; t++) te[t] = tet_edges(c->nh[t]);
-                std::vector<EdgeRec> er(inc.size());
-                for (size_t k = 0; k < er.size(); k++) put(er[k], te[inc[k] >> 2], k);
-                d.erec = dev_alloc<EdgeRec>(c, er.size());
-                upload(c, d.erec, er);
-                TetEdges<float>* pe = dev_alloc<TetEdges<float>>(c, te.size());
-                upload(c, pe, te);
-                c->res.edges = pe;
             }
         }
         upload(c, d.items, c->plan.items);

@@ -36,22 +36,16 @@ struct alignas(16) TetRec {
 };
 static_assert(sizeof(TetRec) == 64, "TetRec must be 64 bytes");
 
-// One incidence of an undamped tet, seen from vertex a (edges e_i = x_i - x_a to
-// the other three, ordered so that their face has the tet's orientation).
-// With Q the inverse rest shape, q_a its row (q_3 = -sum of the rows) and
-// s = det Q, F q_a = sum_i (q_i . q_a) e_i and cof(F) q_a = s n with the face
-// normal n = (e_2 - e_1) x (e_3 - e_1), J = -s n . e_1; so the stable
+// One incidence of an undamped tet of the FP64 state, seen from vertex a (edges
+// e_i = x_i - x_a to the other three, ordered so that their face has the tet's
+// orientation).  With Q the inverse rest shape, q_a its row (q_3 = -sum of the
+// rows) and s = det Q, F q_a = sum_i (q_i . q_a) e_i and cof(F) q_a = s n with
+// the face normal n = (e_2 - e_1) x (e_3 - e_1), J = -s n . e_1; so the stable
 // Neo-Hookean gradient and Hessian need five constants:
 //   w_i = V mu (q_i . q_a), h = V lambda s^2, b = V lambda s alpha
 //   gradient  sum w_i e_i - (h (n . e_1) + b) n
 //   Hessian   h n n^T - (w_1 + w_2 + w_3) I
-// about 55 multiply-adds against 115 through F and its cofactors, from 32
-// bytes (FP64: 64) instead of 64.
-struct alignas(16) EdgeRec {
-    float w[3], h, b;
-    uint32_t i[3];
-};
-static_assert(sizeof(EdgeRec) == 32, "EdgeRec must be 32 bytes");
+// about 55 multiply-adds against 115 through F and its cofactors.
 struct alignas(16) EdgeRec64 {
     double w[3], h, b;
     uint32_t i[3], pad[3];
@@ -63,11 +57,10 @@ static_assert(sizeof(EdgeRec64) == 64, "EdgeRec64 must be 64 bytes");
 constexpr uint8_t kEdgeCorner[4][3] = {{1, 2, 3}, {0, 3, 2}, {0, 1, 3}, {0, 2, 1}};
 constexpr uint8_t kEdgeWeight[4][3] = {{0, 1, 2}, {0, 4, 3}, {1, 3, 5}, {2, 5, 4}};
 
-// w01 w02 w03 w12 w13 w23, h, b of a tet (R = double: from the record the
-// device holds, so that the FP64 state solves the same model; float: rounded once)
-template <class R>
+// w01 w02 w03 w12 w13 w23, h, b of a tet (from the FP32 record the device holds,
+// which defines the model of the FP64 state)
 struct TetEdges {
-    R w[6], h, b;
+    double w[6], h, b;
 };
 
 // Strain-rate damping part (only read when some tet has kd != 0).
@@ -233,10 +226,8 @@ struct DevState {
     GroundRec* ground = nullptr;
     uint32_t* inc = nullptr;       // (tet << 2) | local, grouped per work item
     // per incidence, in inc order: a copy of the tet record with the local
-    // vertex index in the top two bits of idx[3] (scenes with damping), or
-    // the incidence's edge record (FP32 state, no damping)
+    // vertex index in the top two bits of idx[3] (not for an undamped FP64 state)
     TetRec* irec = nullptr;
-    EdgeRec* erec = nullptr;
     VItem* items = nullptr;        // all colours back to back
     double* reduce = nullptr;      // residual / IP partial sums
     uint32_t n = 0, n_tets = 0, n_ground = 0, n_inc = 0, n_items = 0;

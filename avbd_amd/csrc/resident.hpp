@@ -34,11 +34,15 @@ struct alignas(16) ResidentGround {
     uint32_t flags;
 };
 
+// An undamped FP64 state works on the tets' edge constants (TetEdges); FP32 and
+// damped scenes on the rest shape.
+__host__ __device__ constexpr bool resident_edges(uint32_t real, bool damp) { return real == 8 && !damp; }
+
 // LDS layout of a patch, in bytes (the same function sizes the launch and
-// carves the array in the kernel).  Undamped tets: eight arrays of their edge
-// constants (TetEdges; arrays and not records, whose 16- or 32-word stride would
-// put every lane on the same few banks) and 8 bytes per incidence; damped
-// tets: rest shape, E_prev and corners, 2 bytes per incidence.
+// carves the array in the kernel).  Edge constants: eight arrays (arrays and not
+// records, whose 32-word stride would put every lane on the same few banks) and
+// 8 bytes per incidence; else rest shape, corners, with damping E_prev, and
+// 2 bytes per incidence.
 struct ResidentLds {
     uint32_t edge, quad, damp, tix, x, last, lastlast, ym, ground, force, gof, item, target, col, inc, total;
 };
@@ -46,17 +50,18 @@ __host__ __device__ inline ResidentLds resident_lds(uint32_t own, uint32_t items
                                                     uint32_t inc, uint32_t targets, uint32_t colors, uint32_t real,
                                                     bool damp, bool ground) {
     ResidentLds l;
+    const bool edges = resident_edges(real, damp);
     uint32_t at = 0;
     auto take = [&](uint32_t bytes) {
         const uint32_t o = at;
         at += (bytes + 15u) & ~15u;
         return o;
     };
-    l.edge = take(damp ? 0u : 8u * real * tets);
-    l.quad = take(damp ? 48u * tets : 0u);
+    l.edge = take(edges ? 8u * real * tets : 0u);
+    l.quad = take(edges ? 0u : 48u * tets);
     l.damp = take(damp ? 32u * tets : 0u);
-    l.tix = take(damp ? 8u * tets : 0u);
-    l.inc = take((damp ? 2u : 8u) * inc);
+    l.tix = take(edges ? 0u : 8u * tets);
+    l.inc = take((edges ? 8u : 2u) * inc);
     l.x = take(3u * real * local);
     l.last = take(3u * real * local);
     l.lastlast = take(3u * real * local);
@@ -133,7 +138,7 @@ struct ResidentDev {
     const uint2* item = nullptr;
     const uint32_t* target = nullptr;
     const uint32_t* col = nullptr;
-    const void* edges = nullptr;         // TetEdges of the state's precision per tet (no damping)
+    const TetEdges* edges = nullptr;     // per tet (undamped FP64 state)
     unsigned long long* xch = nullptr;   // per halo slot 3 (FP32) or 6 (FP64) tagged words
     unsigned long long* sums = nullptr;  // two sets of two tagged words per patch: its residual sum
     uint32_t* epoch = nullptr;           // per patch: exchanges per colour so far (the tag base)

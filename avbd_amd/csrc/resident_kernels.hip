@@ -95,14 +95,23 @@ struct Kind<double> {
     }
 };
 
-__device__ __forceinline__ void damped_incidence(float3 p0, float3 p1, float3 p2, float3 p3, float4 r1, float4 r2, float4 r3,
-                                          uint32_t local, const TetDamp* damp, uint32_t t, float inv_dt, float3& g,
-                                          Sym3& h) {
-    nh_incidence_pos<true>(p0, p1, p2, p3, r1, r2, r3, local, damp, t, inv_dt, g, h);
+template <bool DAMP>
+__device__ __forceinline__ void shape_incidence(float3 p0, float3 p1, float3 p2, float3 p3, float4 r1, float4 r2,
+                                                float4 r3, uint32_t local, const TetDamp* damp, uint32_t t,
+                                                float inv_dt, float3& g, Sym3& h) {
+    nh_incidence_pos<DAMP>(p0, p1, p2, p3, r1, r2, r3, local, damp, t, inv_dt, g, h);
 }
-__device__ __forceinline__ void damped_incidence(D3 p0, D3 p1, D3 p2, D3 p3, float4 r1, float4 r2, float4 r3, uint32_t local,
-                                          const TetDamp* damp, uint32_t t, double inv_dt, D3& g, SymD& h) {
-    nh_incidence<true>(p0, p1, p2, p3, r1, r2, r3, local, damp, t, inv_dt, g, h);
+template <bool DAMP>
+__device__ __forceinline__ void shape_incidence(D3 p0, D3 p1, D3 p2, D3 p3, float4 r1, float4 r2, float4 r3,
+                                                uint32_t local, const TetDamp* damp, uint32_t t, double inv_dt, D3& g,
+                                                SymD& h) {
+    nh_incidence<DAMP>(p0, p1, p2, p3, r1, r2, r3, local, damp, t, inv_dt, g, h);
+}
+// Place of a lane's terms in its group's sum (FP64 adds them in lane order).
+template <class R, int L>
+__device__ __forceinline__ uint32_t first_incidence(uint32_t lane) {
+    if constexpr (sizeof(R) == 4) return sum_place<L>(lane);
+    else return lane;
 }
 __device__ __forceinline__ void dual(GroundRec& c, float3 p) { ground_dual_update(c, make_float4(p.x, p.y, p.z, 0.f)); }
 __device__ __forceinline__ void dual(GroundRec& c, D3 p) { ground_dual_update(c, p); }
@@ -115,7 +124,7 @@ struct Args {
     const int32_t* ground_of;
     const TetRec* tets;
     const TetDamp* damp;
-    const TetEdges<R>* edges;
+    const TetEdges* edges;
     const ResCtl* rc;
     const float* omega_tab;
     const uint32_t* frozen;
@@ -219,21 +228,22 @@ __device__ __forceinline__ void run_alone(const Args<R>& a, uint32_t first, uint
         const V4 p = a.x[v];
         return K::v3(p.x, p.y, p.z);
     };
+    constexpr bool EDGES = resident_edges(sizeof(R), DAMP);
     auto item = [&](const ResidentPatch& p, uint32_t k, V3 xa, V3& g, typename K::Sym& h) {
         const uint32_t it = a.r.item[p.item_off + k].x, begin = it & 0xffffu, cnt = it >> 16;
         g = K::v3(0, 0, 0);
         h = {0, 0, 0, 0, 0, 0};
-        for (uint32_t j = lane; j < cnt; j += L) {
+        for (uint32_t j = first_incidence<R, L>(lane); j < cnt; j += L) {
             const uint32_t code = a.r.inc[p.inc_off + begin + j].y >> 16, c = code & 3u;
             const uint32_t t = a.r.tet[p.tet_off + (code >> 2)];
             uint4 idx;
             float4 r1, r2, r3;
             load_tet(a.tets, t, idx, r1, r2, r3);
-            if constexpr (DAMP) {
-                damped_incidence(pos(idx.x), pos(idx.y), pos(idx.z), pos(idx.w), r1, r2, r3, c, a.damp, t, a.inv_dt, g,
-                                 h);
+            if constexpr (!EDGES) {
+                shape_incidence<DAMP>(pos(idx.x), pos(idx.y), pos(idx.z), pos(idx.w), r1, r2, r3, c, a.damp, t,
+                                      a.inv_dt, g, h);
             } else {
-                const TetEdges<R>& e = a.edges[t];
+                const TetEdges& e = a.edges[t];
                 const uint32_t n[4] = {idx.x, idx.y, idx.z, idx.w};
                 // the other corners in kEdgeCorner order
                 const uint32_t i1 = c == 0 ? n[1] : n[0], i2 = c == 0 || c == 3 ? n[2] : (c == 1 ? n[3] : n[1]),
@@ -337,10 +347,8 @@ struct LdsView {
     R inv_dt;
     __device__ typename Kind<R>::V3 pos(uint32_t k) const { return Kind<R>::v3(x[3 * k], x[3 * k + 1], x[3 * k + 2]); }
 };
-template <class R, bool DAMP>
-struct Staged;
-template <class R>
-struct Staged<R, true> {
+template <class R, bool DAMP, bool EDGES = resident_edges(sizeof(R), DAMP)>
+struct Staged {
     uint32_t code;
     uint2 ix;
     float4 r1, r2, r3;
@@ -360,11 +368,11 @@ struct Staged<R, true> {
     }
     __device__ void add(const LdsView<R>& v, const Pos& p, typename Kind<R>::V3, typename Kind<R>::V3& g,
                         typename Kind<R>::Sym& h) const {
-        damped_incidence(p.p0, p.p1, p.p2, p.p3, r1, r2, r3, code & 3u, v.damp, code >> 2, v.inv_dt, g, h);
+        shape_incidence<DAMP>(p.p0, p.p1, p.p2, p.p3, r1, r2, r3, code & 3u, v.damp, code >> 2, v.inv_dt, g, h);
     }
 };
-template <class R>
-struct Staged<R, false> {
+template <class R, bool DAMP>
+struct Staged<R, DAMP, true> {
     uint2 e;   // the three other particles, (tet << 2) | corner
     R w1, w2, w3, h, b;
     __device__ void read(const LdsView<R>& v, uint32_t k) {
@@ -441,7 +449,7 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
     // ---- load the patch
     for (uint32_t t = tid; t < p.tets; t += B) {
         const uint32_t g = a.r.tet[p.tet_off + t];
-        if constexpr (DAMP) {
+        if constexpr (!resident_edges(sizeof(R), DAMP)) {
             uint4 idx;
             float4 r1, r2, r3;
             load_tet(a.tets, g, idx, r1, r2, r3);
@@ -449,9 +457,9 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
             quad[3 * t + 1] = r2;
             quad[3 * t + 2] = r3;
             tix[t] = a.r.tix[p.tet_off + t];
-            damp[t] = a.damp[g];
+            if constexpr (DAMP) damp[t] = a.damp[g];
         } else {
-            const TetEdges<R> e = a.edges[g];
+            const TetEdges e = a.edges[g];
 #pragma unroll
             for (int j = 0; j < 6; j++) edge[j * p.tets + t] = e.w[j];
             edge[6 * p.tets + t] = e.h;
@@ -492,7 +500,8 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
     for (uint32_t k = tid; k < 2u * (nc + 1u); k += B) col[k] = a.r.col[p.col_off + k];
     for (uint32_t k = tid; k < p.inc; k += B) {
         const uint2 e = a.r.inc[p.inc_off + k];
-        if constexpr (DAMP) reinterpret_cast<uint16_t*>(lds + o.inc)[k] = (uint16_t)(e.y >> 16);
+        if constexpr (!resident_edges(sizeof(R), DAMP))
+            reinterpret_cast<uint16_t*>(lds + o.inc)[k] = (uint16_t)(e.y >> 16);
         else reinterpret_cast<uint2*>(lds + o.inc)[k] = e;
     }
     const uint32_t base = p.count > 1 ? a.r.epoch[blockIdx.x] : 0u;
@@ -535,7 +544,7 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
         }
     }
 
-    const uint32_t lane = tid % L, group = tid / L;
+    const uint32_t lane = tid % L, group = tid / L, place = first_incidence<R, L>(lane);
     constexpr uint32_t groups = B / L;
     // the payload of an exchange word, once it carries `tag`
     auto wait_word = [&](const word_t* src, uint32_t tag) {
@@ -585,7 +594,7 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
     Staged<R, DAMP> st;
     auto read_item = [&](uint32_t k) {
         it = item[k];
-        if (lane < it.x >> 16) st.read(view, (it.x & 0xffffu) + lane);
+        if (place < it.x >> 16) st.read(view, (it.x & 0xffffu) + place);
     };
     // The item's own state, which its phases before do not change either (only
     // the Chebyshev / dual step does).
@@ -619,7 +628,7 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
         const uint32_t begin = it.x & 0xffffu, cnt = it.x >> 16;
         g = K::v3(0, 0, 0);
         h = {0, 0, 0, 0, 0, 0};
-        for (uint32_t j = lane; j < cnt;) {
+        for (uint32_t j = place; j < cnt;) {
             st.add(view, st.gather(view), xa, g, h);
             j += L;
             if (j < cnt) st.read(view, begin + j);
@@ -780,7 +789,7 @@ void launch_resident(hipStream_t s, const ResidentDev& r, const DevState& d, boo
                      const float* omega_tab, const ResidentCheck& chk) {
     if (chk.every == 0) return;
     Args<float> a{r,      d.x,       d.y,      d.x_last, d.x_lastlast, d.ground,
-                  d.ground_of, d.tets, d.damp, static_cast<const TetEdges<float>*>(r.edges), rc, omega_tab,
+                  d.ground_of, d.tets, d.damp, r.edges, rc, omega_tab,
                   d.frozen, chk, 1.0f / dt, 1.0f / (dt * dt)};
     launch<float>(s, a, damping);
 }
@@ -790,7 +799,7 @@ void launch_resident_f64(hipStream_t s, const ResidentDev& r, const F64State& f,
     if (chk.every == 0) return;
     const double inv_dt = 1.0 / dt;
     Args<double> a{r,      f.x,       f.y,      f.x_last, f.x_lastlast, f.ground,
-                   f.ground_of, f.tets, f.damp, static_cast<const TetEdges<double>*>(r.edges), rc, omega_tab,
+                   f.ground_of, f.tets, f.damp, r.edges, rc, omega_tab,
                    f.frozen, chk, inv_dt, inv_dt * inv_dt};
     launch<double>(s, a, damping);
 }

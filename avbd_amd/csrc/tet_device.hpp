@@ -3,9 +3,14 @@
 // dual update), shared by the per-phase kernels (vbd_kernels.hip) and the
 // resident solve (resident_kernels.hip).  Both files are compiled with
 // -ffp-contract=on, so a function rounds the same way in either.
+//
+// The order of every sum and each rounding here is part of the framework's
+// results: friction branches on the last bit (ground_dual_update), and over a
+// batch of 942,000 vertices a form that differs by one rounding moves single
+// vertices by up to a third of the velocities' rms (an energy from edge vectors and
+// a solve by reciprocals took 32 instead of 40 ms there per 10 steps, and were taken
+// back for that).
 #pragma once
-
-#include <type_traits>
 
 #include "internal.hpp"
 
@@ -106,30 +111,10 @@ __device__ __forceinline__ void nh_incidence_pos(float3 p0, float3 p1, float3 p2
     }
 }
 
-// One incidence of an undamped tet from its edges (EdgeRec).
-__device__ __forceinline__ void edge_incidence(float3 e1, float3 e2, float3 e3, float w1, float w2, float w3, float hn,
-                                               float b, float3& g, Sym3& h) {
-    const float3 u = e2 - e1, v = e3 - e1;
-    const float3 n = make_float3(__builtin_fmaf(u.y, v.z, -(u.z * v.y)), __builtin_fmaf(u.z, v.x, -(u.x * v.z)),
-                                 __builtin_fmaf(u.x, v.y, -(u.y * v.x)));
-    const float k = -__builtin_fmaf(hn, __builtin_fmaf(n.x, e1.x, __builtin_fmaf(n.y, e1.y, n.z * e1.z)), b);
-    g.x += __builtin_fmaf(k, n.x, __builtin_fmaf(w1, e1.x, __builtin_fmaf(w2, e2.x, w3 * e3.x)));
-    g.y += __builtin_fmaf(k, n.y, __builtin_fmaf(w1, e1.y, __builtin_fmaf(w2, e2.y, w3 * e3.y)));
-    g.z += __builtin_fmaf(k, n.z, __builtin_fmaf(w1, e1.z, __builtin_fmaf(w2, e2.z, w3 * e3.z)));
-    const float dev = (w1 + w2) + w3;
-    const float3 t = hn * n;
-    h.a00 += __builtin_fmaf(t.x, n.x, -dev);
-    h.a11 += __builtin_fmaf(t.y, n.y, -dev);
-    h.a22 += __builtin_fmaf(t.z, n.z, -dev);
-    h.a01 = __builtin_fmaf(t.x, n.y, h.a01);
-    h.a02 = __builtin_fmaf(t.x, n.z, h.a02);
-    h.a12 = __builtin_fmaf(t.y, n.z, h.a12);
-}
-
 // A lane's incidence of the work-item order: the record, then the gathered
 // positions, then the terms (three steps, so that several can be in flight).
-struct TetInc {   // scenes with damping
-    using Rec = TetRec;
+template <bool DAMP>
+struct TetInc {
     uint4 idx;
     float4 r1, r2, r3;
     struct Pos {
@@ -139,29 +124,11 @@ struct TetInc {   // scenes with damping
     __device__ Pos gather(const float4* x) const {
         return Pos{f3(x[idx.x]), f3(x[idx.y]), f3(x[idx.z]), f3(x[idx.w & 0x3fffffffu])};
     }
-    __device__ void add(const Pos& p, float3, const TetDamp* __restrict__ damp, uint32_t t, float inv_dt, float3& g,
+    __device__ void add(const Pos& p, const TetDamp* __restrict__ damp, uint32_t t, float inv_dt, float3& g,
                         Sym3& h) const {
-        nh_incidence_pos<true>(p.p0, p.p1, p.p2, p.p3, r1, r2, r3, idx.w >> 30, damp, t, inv_dt, g, h);
+        nh_incidence_pos<DAMP>(p.p0, p.p1, p.p2, p.p3, r1, r2, r3, idx.w >> 30, damp, t, inv_dt, g, h);
     }
 };
-struct EdgeInc {   // without
-    using Rec = EdgeRec;
-    float4 c;   // w1 w2 w3 h
-    uint4 d;    // b, the other three vertices
-    struct Pos {
-        float3 p1, p2, p3;
-    };
-    __device__ void load(const EdgeRec* __restrict__ irec, uint32_t k) {
-        c = reinterpret_cast<const float4*>(irec + k)[0];
-        d = reinterpret_cast<const uint4*>(irec + k)[1];
-    }
-    __device__ Pos gather(const float4* x) const { return Pos{f3(x[d.y]), f3(x[d.z]), f3(x[d.w])}; }
-    __device__ void add(const Pos& p, float3 xa, const TetDamp*, uint32_t, float, float3& g, Sym3& h) const {
-        edge_incidence(p.p1 - xa, p.p2 - xa, p.p3 - xa, c.x, c.y, c.z, c.w, __uint_as_float(d.x), g, h);
-    }
-};
-template <bool DAMP>
-using Inc32 = std::conditional_t<DAMP, TetInc, EdgeInc>;
 
 // Ground AL contact contribution (CollisionConstraintEnergySolver::accumulate<3>,
 // energy/collision/CollisionConstraintEnergySolver.hpp:180-285 with the ground
@@ -197,21 +164,17 @@ __device__ __forceinline__ void ground_accumulate(const GroundRec& c, float3 p, 
 
 // Solve (m/dt^2 I + H) dx = b for symmetric positive definite H by LDL^T.
 __device__ __forceinline__ float3 ldlt3(const Sym3& A, float3 b) {
-    // one reciprocal per pivot: eight quotients took five more division sequences
     const float d0 = A.a00;
-    const float r0 = 1.0f / d0;
-    const float l10 = A.a01 * r0, l20 = A.a02 * r0;
+    const float l10 = A.a01 / d0, l20 = A.a02 / d0;
     const float d1 = A.a11 - l10 * A.a01;
-    const float r1 = 1.0f / d1;
-    const float l21 = (A.a12 - l20 * A.a01) * r1;
+    const float l21 = (A.a12 - l20 * A.a01) / d1;
     const float d2 = A.a22 - l20 * A.a02 - l21 * l21 * d1;
-    const float r2 = 1.0f / d2;
     const float z0 = b.x;
     const float z1 = b.y - l10 * z0;
     const float z2 = b.z - l20 * z0 - l21 * z1;
-    const float x2 = z2 * r2;
-    const float x1 = z1 * r1 - l21 * x2;
-    const float x0 = z0 * r0 - l10 * x1 - l20 * x2;
+    const float x2 = z2 / d2;
+    const float x1 = z1 / d1 - l21 * x2;
+    const float x0 = z0 / d0 - l10 * x1 - l20 * x2;
     return make_float3(x0, x1, x2);
 }
 
@@ -219,6 +182,14 @@ __device__ __forceinline__ float3 ldlt3(const Sym3& A, float3 b) {
 // DPP moves (quad permutes, then mirrors of 8 and 16 lanes, which meet a lane
 // of the other half since each half is already uniform): a register operand
 // modifier instead of an LDS-pipe permute of about 130 cycles per step.
+// Lane l holds the terms of place sum_place<L>(l), l with its bits reversed, so
+// that the places are added as a butterfly from L / 2 down to 1 does: that order is
+// part of an FP32 step's result (a contact that leaves static friction by one last
+// bit moves a vertex by millimetres).
+template <int L>
+__device__ __forceinline__ uint32_t sum_place(uint32_t lane) {
+    return __brev(lane) >> (32 - __builtin_ctz(L));
+}
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_move(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, false);

@@ -117,7 +117,8 @@ __device__ __forceinline__ void edge_incidence(D3 e1, D3 e2, D3 e3, double w1, d
     h.a12 = __builtin_fma(t.y, n.z, h.a12);
 }
 
-// A lane's incidence (see TetInc / EdgeInc of tet_device.hpp).
+// A lane's incidence (see TetInc of tet_device.hpp): with damping the rest shape,
+// without the edge constants.
 struct TetInc64 {
     using Rec = TetRec;
     uint4 idx;

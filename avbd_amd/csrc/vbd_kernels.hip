@@ -86,27 +86,28 @@ __device__ __forceinline__ uint32_t xcd_logical_block() {
 
 // The tet incidences of one work item summed over the L lanes of its group
 // (every lane gets the sums; every lane of the group must call it).  A lane
-// takes its incidences (lane, lane + L, ...) in batches of U: a batch's records
+// takes its incidences (place, place + L, ...) in batches of U: a batch's records
 // are loaded together, then its vertex positions together with the next
 // batch's records, then its terms are added in incidence order -- the same
 // order and arithmetic as one at a time, with fewer dependent memory round trips.
-// xa: the item's own position.  With `da` the lanes share the item's dynamic
-// contacts as well, ahead of the sum (the leader alone took them one after the
-// other behind it: 8.3 -> 5.1 us per colour phase of 24^3 cells under 36 spheres).
+// With `da` the lanes share the item's dynamic contacts as well, ahead of the sum
+// (the leader alone took them one after the other behind it: 8.3 -> 5.1 us per
+// colour phase of 24^3 cells under 36 spheres).
 template <int L, bool DAMP, int U>
 __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, const uint32_t* __restrict__ inc,
-                                              const typename Inc32<DAMP>::Rec* __restrict__ irec,
-                                              const TetDamp* __restrict__ damp, const float4* x, float3 xa,
-                                              float inv_dt, float3& g, Sym3& h, const DynArgs* da = nullptr) {
-    using Inc = Inc32<DAMP>;
+                                              const TetRec* __restrict__ irec, const TetDamp* __restrict__ damp,
+                                              const float4* x, float inv_dt, float3& g, Sym3& h,
+                                              const DynArgs* da = nullptr) {
+    using Inc = TetInc<DAMP>;
+    const uint32_t place = sum_place<L>(lane);
     const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT, base = it.inc_begin;
     g = make_float3(0.f, 0.f, 0.f);
     h = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     Inc cur[U];
 #pragma unroll
     for (int u = 0; u < U; u++)
-        if (lane + u * L < cnt) cur[u].load(irec, base + lane + u * L);
-    for (uint32_t j0 = lane; j0 < cnt; j0 += U * L) {
+        if (place + u * L < cnt) cur[u].load(irec, base + place + u * L);
+    for (uint32_t j0 = place; j0 < cnt; j0 += U * L) {
         typename Inc::Pos P[U];
 #pragma unroll
         for (int u = 0; u < U; u++)
@@ -117,7 +118,7 @@ __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, co
             if (j0 + (U + u) * L < cnt) next[u].load(irec, base + j0 + (U + u) * L);
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (j0 + u * L < cnt) cur[u].add(P[u], xa, damp, DAMP ? (inc[base + j0 + u * L] >> 2) : 0u, inv_dt, g, h);
+            if (j0 + u * L < cnt) cur[u].add(P[u], damp, DAMP ? (inc[base + j0 + u * L] >> 2) : 0u, inv_dt, g, h);
 #pragma unroll
         for (int u = 0; u < U; u++) cur[u] = next[u];
     }
@@ -133,12 +134,6 @@ __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, co
     h.a12 = group_sum<L>(h.a12);
 }
 
-template <bool DAMP>
-__host__ __device__ __forceinline__ const typename Inc32<DAMP>::Rec* inc_records(const DevState& d) {
-    if constexpr (DAMP) return d.irec;
-    else return d.erec;
-}
-
 // The group leader's part of the vertex block solve: ground AL terms, inertia
 // and the 3x3 solve; returns the new position.
 __device__ __forceinline__ float4 item_solve(const VItem& it, float4 xv, float4 yv, const GroundRec& gr, float3 g,
@@ -152,23 +147,23 @@ __device__ __forceinline__ float4 item_solve(const VItem& it, float4 xv, float4 
 // by the L lanes of a group; every lane of the group must call it.
 template <int L, bool DAMP, bool DYN = false, int U = 1>
 __device__ __forceinline__ void solve_item(const VItem& it, uint32_t lane, const uint32_t* __restrict__ inc,
-                                           const typename Inc32<DAMP>::Rec* __restrict__ irec,
-                                           const TetDamp* __restrict__ damp, float4* x, const float4* __restrict__ y,
+                                           const TetRec* __restrict__ irec, const TetDamp* __restrict__ damp,
+                                           float4* x, const float4* __restrict__ y,
                                            const GroundRec* __restrict__ ground, float4* x_out, float4* x_buf,
                                            float inv_dt, float inv_dt2, const DynArgs& da) {
     // the group leader's own state is loaded first, so that its latency
     // overlaps the incidence gathers instead of following the reduction
-    const float4 xv = x[it.v];
-    float4 yv = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 xv = make_float4(0.f, 0.f, 0.f, 0.f), yv = xv;
     GroundRec gr{};
     const bool lead = lane == 0;
     if (lead) {
+        xv = x[it.v];
         yv = y[it.v];
         if (it.ground >= 0) gr = ground[it.ground];
     }
     float3 g;
     Sym3 h;
-    item_gradient<L, DAMP, U>(it, lane, inc, irec, damp, x, f3(xv), inv_dt, g, h, DYN ? &da : nullptr);
+    item_gradient<L, DAMP, U>(it, lane, inc, irec, damp, x, inv_dt, g, h, DYN ? &da : nullptr);
     if (!lead) return;
     const float4 nx = item_solve(it, xv, yv, gr, g, h, inv_dt2);
     if (it.inc_count & VITEM_CONFLICT) x_buf[it.v] = nx;
@@ -178,7 +173,7 @@ __device__ __forceinline__ void solve_item(const VItem& it, uint32_t lane, const
 template <int L, bool DAMP, bool DYN, int U>
 __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_color_kernel(const VItem* __restrict__ items, uint32_t n_items,
                                                            const uint32_t* __restrict__ inc,
-                                                           const typename Inc32<DAMP>::Rec* __restrict__ irec,
+                                                           const TetRec* __restrict__ irec,
                                                            const TetDamp* __restrict__ damp, float4* x,
                                                            const float4* __restrict__ y,
                                                            const GroundRec* __restrict__ ground, float4* x_out,
@@ -409,7 +404,7 @@ __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_cheb_kernel(
     DevState d, const VItem* __restrict__ items, uint32_t n_items, uint32_t sx, uint32_t cx,
     const uint32_t* __restrict__ cheb_list, uint32_t n_cheb, float4* __restrict__ x_next, float omega_fixed,
     const ResCtl* rc, const float* __restrict__ omega_tab, uint32_t j, float inv_dt, float inv_dt2) {
-    kernarg_prefetch(d.x, d.y, d.x_last, d.x_lastlast, d.ground, d.ground_of, d.inc, d.irec, d.erec, d.damp, d.frozen,
+    kernarg_prefetch(d.x, d.y, d.x_last, d.x_lastlast, d.ground, d.ground_of, d.inc, d.irec, d.damp, d.frozen,
                      d.scene_of, items, n_items, sx, cx, cheb_list, n_cheb, x_next, rc, inv_dt, inv_dt2, blockDim.x);
     const uint32_t xcd = blockIdx.x % 8u, q = blockIdx.x / 8u;
     if (q < sx) {
@@ -424,11 +419,11 @@ __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_cheb_kernel(
             if (lane == 0) x_next[v] = d.x[v];
             return;
         }
-        const float4 xv = d.x[v];
-        float4 yv = make_float4(0.f, 0.f, 0.f, 0.f), xl = yv, xll = yv;
+        float4 xv = make_float4(0.f, 0.f, 0.f, 0.f), yv = xv, xl = xv, xll = xv;
         GroundRec gr{};
         const bool lead = lane == 0;
         if (lead) {
+            xv = d.x[v];
             yv = d.y[v];
             xl = d.x_last[v];
             xll = d.x_lastlast[v];
@@ -436,7 +431,7 @@ __global__ __launch_bounds__(U > 1 ? 256 : 1024) void solve_cheb_kernel(
         }
         float3 g;
         Sym3 h;
-        item_gradient<L, DAMP, U>(it, lane, d.inc, inc_records<DAMP>(d), d.damp, d.x, f3(xv), inv_dt, g, h);
+        item_gradient<L, DAMP, U>(it, lane, d.inc, d.irec, d.damp, d.x, inv_dt, g, h);
         if (!lead) return;
         const float4 xp = cheb_apply(item_solve(it, xv, yv, gr, g, h, inv_dt2), xll, omega);
         x_next[v] = xp;
@@ -655,12 +650,11 @@ __global__ __launch_bounds__(kBundleBlock) void bundle_kernel(DevState d, Bundle
 template <int L, bool DAMP>
 __device__ __forceinline__ float residual_item(const VItem& it, uint32_t lane, const DevState& d, float inv_dt,
                                                float inv_dt2) {
-    const float4 xv = d.x[it.v];
     float3 g;
     Sym3 h;
-    item_gradient<L, DAMP, 1>(it, lane, d.inc, inc_records<DAMP>(d), d.damp, d.x, f3(xv), inv_dt, g, h);
+    item_gradient<L, DAMP, 1>(it, lane, d.inc, d.irec, d.damp, d.x, inv_dt, g, h);
     if (lane != 0) return 0.f;
-    const float4 yv = d.y[it.v];
+    const float4 xv = d.x[it.v], yv = d.y[it.v];
     if (it.ground >= 0) ground_accumulate(d.ground[it.ground], f3(xv), g, h);
     const float md = xv.w * inv_dt2;
     const float rx = md * (xv.x - yv.x) + g.x, ry = md * (xv.y - yv.y) + g.y, rz = md * (xv.z - yv.z) + g.z;
@@ -900,7 +894,7 @@ __global__ __launch_bounds__(256) void warm_features_kernel(DevState d, WarmIO i
     float3 gp = make_float3(0.f, 0.f, 0.f), gi = make_float3(0.f, 0.f, 0.f);
     Sym3 h = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     float ssum = 0.f, smax = 0.f, nfix = 0.f;
-    for (uint32_t j = lane; j < cnt; j += L) {
+    for (uint32_t j = sum_place<L>(lane); j < cnt; j += L) {
         const uint32_t e = d.inc[it.inc_begin + j];
         nh_incidence<false>(d.x_prev, d.tets, d.damp, e, inv_dt, gp, h);
         nh_incidence<false>(d.x, d.tets, d.damp, e, inv_dt, gi, h);
@@ -1128,7 +1122,7 @@ __global__ __launch_bounds__(1024) void stats_items_kernel(const VItem* __restri
         const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT;
         float3 g = make_float3(0.f, 0.f, 0.f);
         Sym3 h = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (uint32_t j = lane; j < cnt; j += L)
+        for (uint32_t j = sum_place<L>(lane); j < cnt; j += L)
             nh_incidence<DAMP>(x, tets, damp, inc[it.inc_begin + j], inv_dt, g, h);
         g.x = group_sum<L>(g.x);
         g.y = group_sum<L>(g.y);
@@ -1235,7 +1229,7 @@ void solve_dispatch(hipStream_t s, const DevState& d, uint32_t block, uint32_t b
     const uint32_t threads = count * L;
     const dim3 grid(blocks_for(threads, block)), blk(block);
 #define AVBD_SOLVE_ARGS \
-    d.items + begin, count, d.inc, inc_records<DAMP>(d), d.damp, d.x, d.y, d.ground, x_out, d.x_buf, 1.0f / dt, 1.0f / (dt * dt), \
+    d.items + begin, count, d.inc, d.irec, d.damp, d.x, d.y, d.ground, x_out, d.x_buf, 1.0f / dt, 1.0f / (dt * dt), \
         done, dyn_args(d), d.frozen, d.scene_of
     if (block > 256) batch = 1;   // the batched variants are built for blocks of <= 256 threads
     if (d.dyn_off) hipLaunchKernelGGL((solve_color_kernel<L, DAMP, true, 1>), grid, blk, 0, s, AVBD_SOLVE_ARGS);
