@@ -1039,6 +1039,27 @@ void detect_round(avbd_ctx* c) {
     read_layout(c);
 }
 
+// Lanes per vertex when the caller gives none.  They fix the order of a vertex's
+// sum and with it the roundings of a step, so they follow from the scene alone
+// (timing them chose 8 or 16 by chance at 28^3 cells, and a context rebuilt from a
+// checkpoint could go on with other roundings), and every path of the context uses
+// the same: resident, per phase, timed, warm start.  The lines lie where timing
+// the colour phases changed its choice: undamped FP32 32 lanes up to 22^3 cells
+// (3,042 items in the largest colour) and 8 from 3,479 (16 cubes) and 24^3 (3,907) on; FP64
+// 32 up to 14^3 (844), 8 from 16^3 (1,229) on; damped, whose incidence is twice the
+// work, 32 up to 24^3 (3,907), 16 at 32^3 (8,985).  The resident solve agrees but
+// for a few per cent between the lines; step of 10 iterations at 8 / 16 / 32 lanes in
+// us: FP32 15^3 151 / 134 / 125, 22^3 160 / 142 / 137, 28^3 168 / 159 / 170, 32^3 189 /
+// 179 / 205; FP64 14^3 132 / 123 / 125, 32^3 177 / 192 / 251; damped 16^3 180 / 155 /
+// 137, 24^3 192 / 170 / 165, 32^3 226 / 217 / 236.
+uint32_t default_lanes(const ColorPlan& plan, bool fp64, bool damping) {
+    uint32_t most = 0;
+    for (uint32_t c = 0; c < plan.num_colors; c++)
+        most = std::max(most, plan.item_offsets[c + 1] - plan.item_offsets[c]);
+    if (damping) return most <= 4608 ? 32u : (most <= 9216 ? 16u : 8u);
+    return most <= (fp64 ? 1024u : 3072u) ? 32u : 8u;
+}
+
 // Temporary device buffers, freed when the holder goes out of scope.
 struct DevTemp {
     std::vector<void*> ptrs;
@@ -1104,10 +1125,7 @@ void solve_into_scratch(avbd_ctx* c, const LaunchCfg& cfg, uint32_t b, uint32_t 
 }
 
 // Block size and gather batch: time every candidate on the scene's colour
-// phases and keep the fastest.  Neither changes a result.  The lanes per vertex
-// do (the order of a vertex's sum), so they are not timed but given or 8: timing
-// chose 8 for a batch of cubes and 4 or 16, by chance, for a block under spheres,
-// where a context rebuilt from a checkpoint could then go on with other roundings.
+// phases and keep the fastest.  Neither changes a result.
 void autotune(avbd_ctx* c) {
     const uint32_t block_c[] = {64, 128, 256};
     const uint32_t batch_c[] = {1, 2, 4};
@@ -1282,7 +1300,8 @@ void setup_resident(avbd_ctx* c) {
     r.n_colors = c->plan.num_colors;
     r.lds_bytes = plan.lds_bytes;
     r.max_cluster = plan.max_cluster;
-    resident_shape(plan, c->plan.num_colors, lim, c->desc.lanes_per_vertex, r.lanes, r.block);
+    r.lanes = c->cfg.lanes;
+    r.block = resident_block(plan, c->plan.num_colors, lim, r.lanes);
     // 50 ms: half of what 100 iterations of a large scene take alone (1 ms each at
     // 32^3), so that waiting for another stream's work costs less than giving up
     r.gather_ticks = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 5000000u;
@@ -1942,6 +1961,7 @@ int avbd_build_graph(avbd_ctx* c) {
         c->damping = false;
         for (const auto& t : c->nh)
             if (t.kd != 0.0) c->damping = true;
+        if (!c->desc.lanes_per_vertex) c->cfg.lanes = default_lanes(c->plan, c->fp64, c->damping);
 
         DevState& d = c->d;
         d.n = n;

@@ -103,18 +103,10 @@ struct ResidentLimits {
 bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos, const ResidentLimits& lim,
                     ResidentPlan& out);
 
-// Lanes per vertex (when not given) and threads of a patch's workgroup.  A phase
-// is one chain of latencies per item, so the lanes grow while the largest phase
-// still has a group for each item in 512 threads: 16 for an undamped vertex (24
-// incidences, then two reads per lane; 32 only adds a reduction step), 32 for a
-// damped one, whose incidence is twice the work.  Step of 20 iterations at 8 / 16 /
-// 32 lanes: 14^3 particles damped 6.2 / 3.9 / 3.2 ms, 15^3 undamped 2.41 / 2.27 /
-// 2.33 ms; 32^3 (35 items per phase, two passes at 16) 2.37 / 2.40 / 2.73 ms.
-// 1024 threads where one phase has more items than 512 threads hold groups
-// (512 scenes: 38.0 -> 34.4 ms; idle wavefronts cost 2.4 -> 3.3 ms at 32^3); FP64
-// stays at 512, where its registers fit.
-void resident_shape(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t given,
-                    uint32_t& lanes, uint32_t& block);
+// Threads of a patch's workgroup: 1024 where one phase has more items than 512
+// threads hold groups of `lanes` (512 scenes: 38.0 -> 34.4 ms; idle wavefronts cost
+// 2.4 -> 3.3 ms at 32^3); FP64 stays at 512, where its registers fit.
+uint32_t resident_block(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t lanes);
 
 // What a launch runs: check intervals of `every` iterations until the scene has
 // converged, per_launch of them at most and `total` in a step (hist set), or

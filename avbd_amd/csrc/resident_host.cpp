@@ -302,18 +302,12 @@ bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos
     return !out.patches.empty() && (uint64_t)out.slots * words < (1u << 28);
 }
 
-void resident_shape(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t given,
-                    uint32_t& lanes, uint32_t& block) {
+uint32_t resident_block(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t lanes) {
     uint32_t most = 0;   // items of one colour in one patch
     for (const ResidentPatch& p : plan.patches)
         for (uint32_t c = 0; c < colors; c++)
             most = std::max(most, plan.col[p.col_off + c + 1] - plan.col[p.col_off + c]);
-    lanes = given;
-    if (!lanes) {
-        lanes = 8;
-        while (lanes < (lim.damp ? 32u : 16u) && 2 * lanes * most <= 512) lanes *= 2;
-    }
-    block = lim.real_bytes == 4 && lanes * most > 512 ? 1024u : 512u;
+    return lim.real_bytes == 4 && lanes * most > 512 ? 1024u : 512u;
 }
 
 bool build_bundles(const HostModel& m, const ColorPlan& plan, BundlePlan& out) {

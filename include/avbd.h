@@ -106,7 +106,10 @@ typedef struct {
     double iter_acceleration;      /* Chebyshev rho */
     uint32_t flags;
     int32_t device;                /* HIP device ordinal */
-    uint32_t lanes_per_vertex;     /* 0 = autotuned; else 4, 8, 16 or 32 */
+    uint32_t lanes_per_vertex;     /* 4, 8, 16 or 32, or 0 = 8 to 32 by the size of the largest colour,
+                                      precision and damping of the context.  The lanes fix the order of a
+                                      vertex's sum: give them where a scene in a batch and the same scene
+                                      in a context of its own have to agree bit for bit */
     uint32_t block_size;           /* 0 = autotuned; else 64..1024, multiple of 64 */
     uint32_t gather_batch;         /* tet incidences a lane gathers at once: 0 = autotuned
                                       (1 when lanes and block size are both given); else 1, 2 or 4 */
@@ -359,8 +362,10 @@ int avbd_get_stats(avbd_ctx* ctx, avbd_stats* out);
 /* Introspection for tests and the bench -------------------------------------- */
 uint32_t avbd_num_particles(avbd_ctx* ctx);
 uint32_t avbd_num_energies(avbd_ctx* ctx, int type);
-/* Kernel launch geometry actually in use (after autotuning); *gather_batch =
- * tet incidences one lane gathers at once (1, 2 or 4). Any pointer may be null. */
+/* Kernel launch geometry in use: *lanes_per_vertex of every path (passed back in
+ * avbd_scene_desc it gives the same results); *block_size and *gather_batch (tet
+ * incidences one lane gathers at once: 1, 2 or 4) of the per-phase launches, after
+ * autotuning; neither changes a result. Any pointer may be null. */
 int avbd_get_launch_config(avbd_ctx* ctx, uint32_t* lanes_per_vertex, uint32_t* block_size, uint32_t* gather_batch);
 /* *persistent_grid = blocks of the persistent step kernel, or 0 when the
  * step runs as one launch per phase; *fused_chebyshev = 1 when the Chebyshev /
