@@ -144,8 +144,8 @@ bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, c
         tet_local.assign(n_tets, 0);
         std::fill(stamp.begin(), stamp.end(), NONE);
         for (auto& r : readers) r.clear();
-        bool fits = true;
-        for (uint32_t q = 0; q < parts; q++) {
+        bool fits = true;   // the LDS and the 16-bit local indices
+        for (uint32_t q = 0; q < parts && fits; q++) {
             if (own[q].empty()) continue;
             auto colour_of = [&](uint32_t v) { return plan.item_kind[lo + v] == 1 ? plan.color[lo + v] : colors; };
             std::stable_sort(own[q].begin(), own[q].end(),
@@ -168,7 +168,8 @@ bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, c
                 if (plan.item_kind[lo + v] != 1) break;
                 const VItem& it = plan.item_of[lo + v];
                 const uint32_t begin = (uint32_t)out.inc.size() / 4 - p.inc_off;
-                if (begin + it.inc_count > 0xFFFFu) return false;
+                fits = begin + it.inc_count <= 0xFFFFu && tets.size() + it.inc_count <= 0x4000u;
+                if (!fits) break;
                 out.item.push_back(begin | it.inc_count << 16);
                 out.item.push_back(0);
                 p.items++;
@@ -185,7 +186,6 @@ bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, c
                             halo.push_back(u);
                         }
                     }
-                    if (tet_local[t - t0] > 0x3FFFu) return false;
                     // the particles' local indices are known once the halo is complete
                     for (int j = 0; j < 3; j++) out.inc.push_back(0);
                     out.inc.push_back((uint16_t)(tet_local[t - t0] << 2 | (code & 3u)));
@@ -198,7 +198,8 @@ bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, c
             p.local = p.own + (uint32_t)halo.size();
             p.tets = (uint32_t)tets.size();
             p.inc = (uint32_t)out.inc.size() / 4 - p.inc_off;
-            if (p.local > 0xFFFFu) return false;
+            if (p.local > 0xFFFFu) fits = false;
+            if (!fits) break;
             for (uint32_t k = 0; k < halo.size(); k++) {
                 local[halo[k]] = p.own + k;
                 if (colour_of(halo[k]) < colors) readers[halo[k]].push_back(p.slot + k);
@@ -229,11 +230,13 @@ bool build_scene(const HostModel& m, const ColorPlan& plan, const double* pos, c
             out.patches.push_back(p);
         }
         for (ResidentPatch& p : out.patches) {
+            if (!fits) break;
             p.target_off = (uint32_t)out.target.size();
             for (uint32_t k = 0; k < p.items; k++) {
                 const auto& r = readers[out.gid[p.gid_off + k] - lo];
                 const uint32_t begin = (uint32_t)out.target.size() - p.target_off;
-                if (begin + r.size() > 0xFFFFu) return false;
+                fits = begin + r.size() <= 0xFFFFu;
+                if (!fits) break;
                 out.item[2 * (size_t)(p.item_off + k) + 1] = begin | (uint32_t)r.size() << 16;
                 out.target.insert(out.target.end(), r.begin(), r.end());
             }
