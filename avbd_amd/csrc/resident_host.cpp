@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <future>
 #include <numeric>
 #include <thread>
 
@@ -13,6 +14,8 @@ namespace avbd {
 namespace {
 
 constexpr uint32_t NONE = 0xFFFFFFFFu;
+// a thread of its own, or the caller's at get() when the system has none to give
+constexpr std::launch kThreads = std::launch::async | std::launch::deferred;
 
 // Recursive coordinate bisection: parts [0, parts) of the particles in
 // idx[lo, hi), each cut along the longest side of the box so that the weight
@@ -46,13 +49,14 @@ void bisect(uint32_t* idx, uint32_t lo, uint32_t hi, uint32_t first, uint32_t pa
     uint64_t sum = 0;
     uint32_t cut = lo;
     while (cut < hi && sum + weight[idx[cut]] <= want) sum += weight[idx[cut++]];
-    // the two sides touch different particles
-    std::thread side;
+    // the two sides touch different particles (a failure in either comes out of
+    // get() or of this call, which then waits for the other)
+    std::future<void> side;
     if (hi - lo > 4096 && threads > 1)
-        side = std::thread(bisect, idx, lo, cut, first, left, pos, weight, base, part, threads / 2);
+        side = std::async(kThreads, bisect, idx, lo, cut, first, left, pos, weight, base, part, threads / 2);
     else bisect(idx, lo, cut, first, left, pos, weight, base, part, 1);
     bisect(idx, cut, hi, first + left, parts - left, pos, weight, base, part, threads - threads / 2);
-    if (side.joinable()) side.join();
+    if (side.valid()) side.get();
 }
 
 // Coordinates of the particles [lo, lo + n) along the edges of a tet: the two
@@ -264,15 +268,23 @@ bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos
     const uint32_t cpus = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
     const uint32_t workers = std::min(n_scenes, cpus);
     auto work = [&] {
-        for (uint32_t s; ok && (s = next++) < n_scenes;)
-            if (!build_scene(m, plan, pos, lim, s, std::max(1u, cpus / workers), scenes[s])) ok = false;
+        for (uint32_t s; ok && (s = next++) < n_scenes;) {
+            bool fits = false;
+            try {
+                fits = build_scene(m, plan, pos, lim, s, std::max(1u, cpus / workers), scenes[s]);
+            } catch (...) {
+                ok = false;   // the other threads stop
+                throw;
+            }
+            if (!fits) ok = false;
+        }
     };
-    if (workers <= 1) {
+    {
+        std::vector<std::future<void>> pool;
+        pool.reserve(workers);
+        for (uint32_t w = 1; w < workers; w++) pool.push_back(std::async(kThreads, work));
         work();
-    } else {
-        std::vector<std::thread> pool;
-        for (uint32_t w = 0; w < workers; w++) pool.emplace_back(work);
-        for (auto& t : pool) t.join();
+        for (auto& t : pool) t.get();
     }
     if (!ok) return false;
     out = ResidentPlan{};

@@ -3,15 +3,32 @@
 // builds Kuhn cubes of the given cells per edge as one batch, partitions it and
 // checks every table the kernel reads against the tets and colours; prints
 // "fits PATCHES LDS" or "does not fit".
+//   partition_check memory
+// lets the n-th allocation of a partition fail, for n = 1, 2, 4, ..., in whichever
+// thread makes it: each must come out as std::bad_alloc.
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <set>
 #include <string>
 
 #include "resident.hpp"
 
 using namespace avbd;
+
+static std::atomic<long> allocations_left{-1};   // < 0: no limit
+void* operator new(size_t n) {
+    if (allocations_left.load() >= 0 && allocations_left.fetch_sub(1) <= 0) {
+        allocations_left = 0;
+        throw std::bad_alloc();
+    }
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 #define CHECK(c)                                              \
     do {                                                      \
@@ -155,6 +172,26 @@ static void check(const Batch& b, const ResidentLimits& lim, const ResidentPlan&
 }
 
 int main(int argc, char** argv) {
+    if (argc == 2 && !std::strcmp(argv[1], "memory")) {
+        for (const std::vector<int>& cells : {std::vector<int>{24}, std::vector<int>(24, 6)}) {
+            const Batch b(cells, false);
+            const ResidentLimits lim{4, false, true, 160 * 1024 - 1024, 256, 1000};
+            ResidentPlan out;
+            bool done = false;
+            for (long n = 1; !done; n *= 2) {
+                allocations_left = n;
+                try {
+                    CHECK(build_resident(b.model, b.plan, b.x.data(), lim, out));
+                    done = allocations_left > 0;   // (a failure that a thread start met is made up for)
+                } catch (const std::bad_alloc&) {
+                }
+                allocations_left = -1;
+            }
+            check(b, lim, out);
+        }
+        std::puts("every failure came out");
+        return 0;
+    }
     CHECK(argc == 9 && !std::strcmp(argv[1], "scenes"));
     std::vector<int> cells;
     for (const char* s = argv[2]; s; s = std::strchr(s, ',') ? std::strchr(s, ',') + 1 : nullptr) cells.push_back(std::atoi(s));

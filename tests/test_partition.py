@@ -52,3 +52,7 @@ def test_a_first_cut_beyond_16_bits_is_refined(checker, cells):
     assert 24 * cells ** 3 > 0xFFFF
     out = scenes(checker, [cells, 5], target=10 ** 6)
     assert out[0] == "fits" and int(out[1]) > 2
+
+
+def test_a_failed_allocation_comes_out_as_an_error(checker):
+    assert checker("memory")[:2] == ["every", "failure"]
