@@ -8,7 +8,9 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -86,6 +88,11 @@ struct avbd_ctx {
     bool bundled = false;      // static scenes of oriented particles only, each component small enough
     BundleDev bundles;
     ResidentCheck res_check;   // residual mode: the check intervals of a resident launch
+    // among the contexts of the device whose patches wait for each other (DeviceTurns)
+    bool takes_turns = false;
+    bool in_flight = false;        // resident launches enqueued and not yet seen to have ended
+    hipEvent_t ev_turn = nullptr;  // after them, once another context has asked
+    bool turn_marked = false;      // ev_turn is behind the last of them
 
     bool timing = false;
     std::vector<hipEvent_t> events;
@@ -581,6 +588,86 @@ F64State f64_state(const avbd_ctx* c) {
 // partitioned at set-up, and with dynamic contacts the step is the static one.
 bool uses_resident(const avbd_ctx* c) { return c->resident && (!c->dynamic || dyn_quiet(c)); }
 
+// Patches that wait for each other have to run at once, so two resident launches
+// that together do not fit the device must not start side by side: each could
+// hold a part of it and wait for the rest (three 20^3 FP64 contexts on three
+// threads took 125 us per iteration, most of it in clusters that gave up; 11 in
+// turn).  Contexts launch under the lock of their device and one that would not fit
+// beside those in flight first waits, on its stream, until they have ended.  A
+// context that is alone pays for the lock only.
+struct DeviceTurns {
+    std::mutex m;
+    std::vector<avbd_ctx*> live;
+};
+DeviceTurns& turns_of(int device) {
+    static std::mutex m;
+    static auto* all = new std::map<int, DeviceTurns>;   // (outlives every context)
+    std::lock_guard<std::mutex> hold(m);
+    return (*all)[device];
+}
+
+// Held around the launch of a step or interval that may hold resident launches,
+// and while the stream is capturing (no other context may record on it then).
+class ResidentTurn {
+public:
+    ResidentTurn(avbd_ctx* c, bool launches) {
+        if (!c->takes_turns) return;
+        DeviceTurns& t = turns_of(c->device);
+        hold_ = std::unique_lock<std::mutex>(t.m);
+        if (!launches || !uses_resident(c)) return;
+        // A grid needs room on each of the eight dies its workgroups go to in turn.
+        // With fewer than k workgroups on a CU there is room for one more when k of the
+        // largest fit, so n workgroups all run if n <= k x CUs.
+        constexpr uint32_t kDies = 8;
+        auto share = [](const avbd_ctx* o) { return (o->res.n_patches + kDies - 1) / kDies; };
+        uint64_t wanted = share(c);
+        uint32_t k = c->res.per_cu;
+        for (avbd_ctx* o : t.live) {
+            if (o == c || !o->in_flight) continue;
+            if (o->turn_marked ? ended(hipEventQuery(o->ev_turn)) : ended(hipStreamQuery(o->stream))) {
+                o->in_flight = false;
+                continue;
+            }
+            wanted += share(o);
+            k = std::min(k, o->res.per_cu);
+        }
+        if (wanted > (uint64_t)k * (c->res.cus / kDies))
+            for (avbd_ctx* o : t.live) {
+                if (o == c || !o->in_flight) continue;
+                if (!o->turn_marked) hip_check(hipEventRecord(o->ev_turn, o->stream), "hipEventRecord");
+                o->turn_marked = true;
+                hip_check(hipStreamWaitEvent(c->stream, o->ev_turn, 0), "hipStreamWaitEvent");
+            }
+        c->in_flight = true;
+        c->turn_marked = false;
+    }
+
+private:
+    static bool ended(hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();   // not ready is no error of a launch
+        return e == hipSuccess;
+    }
+    std::unique_lock<std::mutex> hold_;
+};
+
+void join_turns(avbd_ctx* c) {
+    hip_check(hipEventCreateWithFlags(&c->ev_turn, hipEventDisableTiming), "hipEventCreate");
+    DeviceTurns& t = turns_of(c->device);
+    std::lock_guard<std::mutex> hold(t.m);
+    t.live.push_back(c);
+    c->takes_turns = true;
+}
+void leave_turns(avbd_ctx* c) {
+    if (c->takes_turns) {
+        DeviceTurns& t = turns_of(c->device);
+        std::lock_guard<std::mutex> hold(t.m);
+        t.live.erase(std::remove(t.live.begin(), t.live.end(), c), t.live.end());
+        c->takes_turns = false;
+    }
+    if (c->ev_turn) (void)hipEventDestroy(c->ev_turn);
+    c->ev_turn = nullptr;
+}
+
 void enqueue_head(avbd_ctx* c, bool with_events) {
     const float dt = (float)c->desc.dt, g = (float)c->desc.g_accel;
     hipStream_t s = c->stream;
@@ -796,6 +883,7 @@ void destroy_graph(avbd_ctx* c) {
 
 template <class F>
 hipGraphExec_t capture(avbd_ctx* c, F&& body) {
+    const ResidentTurn hold(c, false);
     hip_check(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     try {
         body();
@@ -882,6 +970,7 @@ void run_residual_step(avbd_ctx* c, bool graphs) {
             hip_check(hipEventSynchronize(c->part_ev[k - kAhead]), "hipEventSynchronize");
             if (c->h_conv[k - kAhead]) break;
         }
+        const ResidentTurn turn(c, true);
         if (k == 0) {
             if (graphs) hip_check(hipGraphLaunch(c->head_exec, s), "hipGraphLaunch");
             else {
@@ -1306,8 +1395,11 @@ void setup_resident(avbd_ctx* c) {
     // 32^3), so that waiting for another stream's work costs less than giving up
     r.gather_ticks = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 5000000u;
     r.has_ground = lim.ground;
+    r.cus = lim.max_cluster;
+    r.per_cu = resident_per_cu(r, c->fp64, c->damping);
     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     c->resident = true;
+    if (r.max_cluster > 1) join_turns(c);
 }
 
 // The same for scenes of oriented particles only (rods, jointed bodies)
@@ -1398,6 +1490,7 @@ int avbd_create(const avbd_scene_desc* desc, avbd_ctx** out) {
 void avbd_destroy(avbd_ctx* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    leave_turns(c);
     destroy_graph(c);
     c->mlp.reset();
     for (void* p : c->allocations) (void)hipFree(p);
@@ -2318,7 +2411,10 @@ int avbd_step(avbd_ctx* c, uint32_t n_steps) {
                     run_residual_step(c, graphs);
                     continue;
                 }
-                enqueue_step(c, c->timing);
+                {
+                    const ResidentTurn turn(c, !c->timing);
+                    enqueue_step(c, c->timing);
+                }
                 c->vertex_updates += (uint64_t)c->desc.solver_iters * (c->d.n_items + c->d.n_oitems);
                 if (c->timing) {
                     hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
@@ -2363,9 +2459,15 @@ int avbd_step(avbd_ctx* c, uint32_t n_steps) {
             c->lbvh_avg_ms = lbvh_total / std::max(1u, n_steps);
             c->solve_launches = launches;
         } else if (c->graph_exec) {
-            for (uint32_t s = 0; s < n_steps; s++) hip_check(hipGraphLaunch(c->graph_exec, c->stream), "hipGraphLaunch");
+            for (uint32_t s = 0; s < n_steps; s++) {
+                const ResidentTurn turn(c, true);
+                hip_check(hipGraphLaunch(c->graph_exec, c->stream), "hipGraphLaunch");
+            }
         } else {
-            for (uint32_t s = 0; s < n_steps; s++) enqueue_step(c, false);
+            for (uint32_t s = 0; s < n_steps; s++) {
+                const ResidentTurn turn(c, true);
+                enqueue_step(c, false);
+            }
         }
         hip_check(hipEventRecord(c->ev_b, c->stream), "hipEventRecord");
         c->steps_taken += n_steps;

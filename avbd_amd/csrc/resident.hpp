@@ -138,6 +138,7 @@ struct ResidentDev {
     uint32_t* sync = nullptr;            // per patch (the cluster's first one): arrivals, decision word
     uint32_t* status = nullptr;          // = DevState::status
     uint32_t n_patches = 0, n_colors = 0, lds_bytes = 0, max_cluster = 0, lanes = 8, block = 512;
+    uint32_t cus = 0, per_cu = 0;        // of the device; workgroups of this launch that fit on one of them
     uint32_t gather_ticks = 0;           // 100 MHz ticks a patch waits for its cluster to be resident
     bool has_ground = false;
 };
@@ -147,6 +148,8 @@ void launch_resident(hipStream_t s, const ResidentDev& r, const DevState& d, boo
                      const float* omega_tab, const ResidentCheck& chk);
 void launch_resident_f64(hipStream_t s, const ResidentDev& r, const F64State& f, bool damping, double dt,
                          const ResCtl* rc, const float* omega_tab, const ResidentCheck& chk);
+// Workgroups of the context's launch that fit on one CU at once.
+uint32_t resident_per_cu(const ResidentDev& r, bool fp64, bool damping);
 // After a launch with checks: the step's residual record, counters and frozen scenes.
 void launch_residual_collect(hipStream_t s, ResCtl* rc, const ResidentCheck& chk, double* acc_scene, uint32_t n_scenes,
                              const SceneFreeze& fz);

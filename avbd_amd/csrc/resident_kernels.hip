@@ -751,27 +751,36 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
     if (tid == 0 && p.count > 1) a.r.epoch[blockIdx.x] = tag;
 }
 
+// Launches, or with per_cu set asks how many workgroups fit on a CU.
 template <class R, int L, bool DAMP, int B>
-void dispatch_block(hipStream_t s, const Args<R>& a) {
+void dispatch_block(hipStream_t s, const Args<R>& a, uint32_t* per_cu) {
     // more than 64 KB of LDS has to be asked for
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&resident_kernel<R, L, DAMP, B>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)a.r.lds_bytes);
+    if (per_cu) {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &n, reinterpret_cast<const void*>(&resident_kernel<R, L, DAMP, B>), B, a.r.lds_bytes) != hipSuccess)
+            (void)hipGetLastError();
+        *per_cu = (uint32_t)(n > 1 ? n : 1);
+        return;
+    }
     hipLaunchKernelGGL((resident_kernel<R, L, DAMP, B>), dim3(a.r.n_patches), dim3(B), a.r.lds_bytes, s, a);
 }
 
 template <class R, int L, bool DAMP>
-void dispatch(hipStream_t s, const Args<R>& a) {
+void dispatch(hipStream_t s, const Args<R>& a, uint32_t* per_cu) {
     if constexpr (sizeof(R) == 4)
-        if (a.r.block == 1024) return dispatch_block<R, L, DAMP, 1024>(s, a);
-    dispatch_block<R, L, DAMP, 512>(s, a);
+        if (a.r.block == 1024) return dispatch_block<R, L, DAMP, 1024>(s, a, per_cu);
+    dispatch_block<R, L, DAMP, 512>(s, a, per_cu);
 }
 
 template <class R>
-void launch(hipStream_t s, const Args<R>& a, bool damping) {
-#define AVBD_RES_CASE(LL)                                 \
-    case LL:                                               \
-        if (damping) dispatch<R, LL, true>(s, a);          \
-        else dispatch<R, LL, false>(s, a);                 \
+void launch(hipStream_t s, const Args<R>& a, bool damping, uint32_t* per_cu = nullptr) {
+#define AVBD_RES_CASE(LL)                                     \
+    case LL:                                                   \
+        if (damping) dispatch<R, LL, true>(s, a, per_cu);      \
+        else dispatch<R, LL, false>(s, a, per_cu);             \
         break;
     switch (a.r.lanes) {
         AVBD_RES_CASE(4)
@@ -784,6 +793,20 @@ void launch(hipStream_t s, const Args<R>& a, bool damping) {
 }
 
 }  // namespace
+
+uint32_t resident_per_cu(const ResidentDev& r, bool fp64, bool damping) {
+    uint32_t n = 1;
+    if (fp64) {
+        Args<double> a{};
+        a.r = r;
+        launch<double>(nullptr, a, damping, &n);
+    } else {
+        Args<float> a{};
+        a.r = r;
+        launch<float>(nullptr, a, damping, &n);
+    }
+    return n;
+}
 
 void launch_resident(hipStream_t s, const ResidentDev& r, const DevState& d, bool damping, float dt, const ResCtl* rc,
                      const float* omega_tab, const ResidentCheck& chk) {
