@@ -725,6 +725,13 @@ void enqueue_head(avbd_ctx* c, bool with_events) {
     hip_check(hipGetLastError(), "kernel launch");
 }
 
+// Iterations of a resident launch: one costs some 50 us (loading the patches, the
+// handshake, recording the checks, the gap) against 1.4 ms for 100 iterations at
+// 32^3.  One that runs much longer keeps other streams' work off the CUs, and
+// where a batch has more patches than the device holds, the patches of a scene
+// that begin to run wait as long for the rest (gather_ticks).
+constexpr uint32_t kResidentIters = 100;
+
 // Iterations [i0, i1) of a step.  With `check` (residual mode: i0 = 0,
 // i1 = res_check_every) the Chebyshev weights come from the device table and
 // a residual check follows the last iteration; a resident launch runs up to
@@ -754,11 +761,21 @@ void enqueue_iters(avbd_ctx* c, bool with_events, uint32_t i0, uint32_t i1, bool
     }
     const bool resident = uses_resident(c) && !with_events;
     if (resident) {
+        auto run = [&](uint32_t from, const ResidentCheck& k) {
+            if (c->fp64) launch_resident_f64(s, c->res, f0, c->damping, c->desc.dt, rc, c->omega_tab + from, k);
+            else launch_resident(s, c->res, dz, c->damping, dt, rc, c->omega_tab + from, k);
+        };
+        uint32_t from = i0;
+        for (; i1 - from > kResidentIters; from += kResidentIters) {
+            ResidentCheck plain;
+            plain.every = kResidentIters;
+            run(from, plain);
+        }
         ResidentCheck chk;
         if (check) chk = c->res_check;
+        chk.every = i1 - from;
+        run(from, chk);
         chk.every = i1 - i0;
-        if (c->fp64) launch_resident_f64(s, c->res, f0, c->damping, c->desc.dt, rc, c->omega_tab + i0, chk);
-        else launch_resident(s, c->res, dz, c->damping, dt, rc, c->omega_tab + i0, chk);
         if (check) launch_residual_collect(s, c->rc, chk, c->res_acc_scene, c->n_res_scenes, fz);
     }
     const bool bundled = c->bundled && !c->dynamic && !with_events;
@@ -1365,13 +1382,9 @@ void setup_resident(avbd_ctx* c) {
     r.sums = dev_alloc<unsigned long long>(c, 4 * np);
     hip_check(hipMemsetAsync(r.sums, 0, 4 * np * sizeof(unsigned long long), c->stream), "hipMemsetAsync");
     if (c->rc) {
-        // About 100 iterations per launch: a launch costs some 50 us (loading the
-        // patches, the handshake, recording the checks, the gap) against 1.4 ms for
-        // 100 iterations at 32^3, and one that runs much longer keeps other streams'
-        // work off the CUs.
         ResidentCheck& k = c->res_check;
         k.total = c->res_max_iters / c->res_check_every;
-        k.per_launch = std::max(1u, std::min(k.total, 100u / c->res_check_every));
+        k.per_launch = std::max(1u, std::min(k.total, kResidentIters / c->res_check_every));
         k.per_scene = c->n_res_scenes > 1;
         k.tol2 = c->res_tol * c->res_tol;
         k.mg2 = c->res_mg2_scene;

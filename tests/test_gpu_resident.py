@@ -111,3 +111,29 @@ def test_bundles_of_rods_match_one_launch_per_phase(nx, nz, segments, jointed, o
     print(f"[gpu-test]   off the oracle: per phase {err[0]:.2e}, bundles {err[1]:.2e}", flush=True)
     assert err[1] <= 2 * err[0] + 1e-6
     assert err[1] == err[2]
+
+
+def test_scenes_that_wait_for_a_part_of_the_device_are_not_given_up():
+    """Three scenes whose patches fill 1.4 times the device, many iterations per
+    step: part of the third starts at once and waits for the first two.  A wait
+    as long as their 6,000 iterations (90 ms) made it give up and run on one
+    workgroup (18 s); the stretch is cut into launches instead.  At most three
+    times what one launch per phase takes."""
+    import time
+    from avbd_amd.sim import Simulation
+    print("[gpu-test] three scenes, 6,000 iterations", flush=True)
+    sc = scenes.cube_batch(n_scenes=3, n_min=20, n_max=20)
+    sc.iters = 6000
+    took, x = [], []
+    for f in (0, _lib.FLAG_NO_PERSISTENT):
+        s = Simulation(sc, fp64_state=True, flags=f, lanes_per_vertex=8, block_size=128)
+        s.setup()
+        s.update(1)
+        s.ctx.synchronize()
+        t = time.perf_counter()
+        s.update(1)
+        x.append(s.positions())
+        took.append(time.perf_counter() - t)
+    print(f"[gpu-test]   resident {took[0] * 1e3:.0f} ms, per phase {took[1] * 1e3:.0f} ms", flush=True)
+    assert np.array_equal(x[0], x[1])
+    assert took[0] <= 3 * took[1]
