@@ -729,7 +729,7 @@ void enqueue_head(avbd_ctx* c, bool with_events) {
 // handshake, recording the checks, the gap) against 1.4 ms for 100 iterations at
 // 32^3.  One that runs much longer keeps other streams' work off the CUs, and
 // where a batch has more patches than the device holds, the patches of a scene
-// that begin to run wait as long for the rest (gather_ticks).
+// that begin to run wait as long for the rest (gather_polls).
 constexpr uint32_t kResidentIters = 100;
 
 // Iterations [i0, i1) of a step.  With `check` (residual mode: i0 = 0,
@@ -1404,9 +1404,9 @@ void setup_resident(avbd_ctx* c) {
     r.max_cluster = plan.max_cluster;
     r.lanes = c->cfg.lanes;
     r.block = resident_block(plan, c->plan.num_colors, lim, r.lanes);
-    // 50 ms: half of what 100 iterations of a large scene take alone (1 ms each at
-    // 32^3), so that waiting for another stream's work costs less than giving up
-    r.gather_ticks = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 5000000u;
+    // about 50 ms (0.13 us each): half of what 100 iterations of a large scene take alone (1 ms each
+    // at 32^3), so that waiting for another stream's work costs less than giving up
+    r.gather_polls = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 400000u;
     r.has_ground = lim.ground;
     r.cus = lim.max_cluster;
     r.per_cu = resident_per_cu(r, c->fp64, c->damping);

@@ -46,12 +46,14 @@
 //
 // Waits end: the patches of a scene depend on each other, so they must all be
 // running.  Each announces itself after loading its patch and waits until
-// the cluster is complete (or until `gather_ticks` have passed; the decision is
+// the cluster is complete (or has polled `gather_polls` times; the decision is
 // one compare-and-swap word, the same for all).  A complete cluster's workgroups
 // stay resident, so every later wait is for a running workgroup.  An incomplete
 // cluster gives up before anything is written, and its first patch alone runs
 // the scene from device memory.  Later waits are bounded as well (they set
-// status bit 1 and go on).
+// status bit 1 and go on).  Waits are counted in polls (0.12 us each from an
+// otherwise idle memory) and not by the clock, which runs on while the process is
+// switched out.
 //
 // The arithmetic of an item is that of the per-phase kernels (tet_device.hpp:
 // L lanes per vertex, the same incidence order and butterfly sums), so results
@@ -400,7 +402,7 @@ struct Staged<R, DAMP, true> {
 // words on their way to memory, which no thread of this workgroup reads.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-constexpr uint32_t kWaitTicks = 200000000u;   // 2 s of the 100 MHz clock: the bound of an exchange wait
+constexpr uint32_t kWaitPolls = 1u << 24;   // about 2 s: the bound of an exchange wait
 
 template <class R, int L, bool DAMP, int B>
 __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
@@ -520,10 +522,10 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
                 __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.count - 1u;
             if (full)   // everyone has arrived: ready for the next launch
                 __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint64_t t0 = wall_clock64();
+            uint32_t polls = 0;
             uint32_t now = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             while ((int32_t)(now - want) < 0) {
-                if (full || wall_clock64() - t0 >= a.r.gather_ticks) {
+                if (full || polls++ >= a.r.gather_polls) {
                     uint32_t seen = now;
                     const uint32_t next = full ? want : want + 1u;
                     now = __hip_atomic_compare_exchange_strong(word, &seen, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -548,12 +550,10 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
     constexpr uint32_t groups = B / L;
     // the payload of an exchange word, once it carries `tag`
     auto wait_word = [&](const word_t* src, uint32_t tag) {
-        uint64_t t0 = 0;
-        while (true) {
+        for (uint32_t polls = 0;; polls++) {
             const word_t u = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if ((uint32_t)(u >> 32) == tag) return (uint32_t)u;
-            if (t0 == 0) t0 = wall_clock64();
-            if (*(volatile uint32_t*)&dead || wall_clock64() - t0 > kWaitTicks) {
+            if (*(volatile uint32_t*)&dead || polls > kWaitPolls) {
                 *(volatile uint32_t*)&dead = 1;
                 atomicOr(a.r.status, 2u);
                 return 0u;
