@@ -481,6 +481,7 @@ class SimulationContext:
         return st
 
     def persistent_grid(self) -> int:
+        """Workgroups of the launch that runs a step's iterations; 0: one launch per phase."""
         g = C.c_uint32()
         self._chk(lib.avbd_get_step_mode(self.handle, C.byref(g), None))
         return g.value

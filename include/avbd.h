@@ -367,10 +367,14 @@ uint32_t avbd_num_energies(avbd_ctx* ctx, int type);
  * incidences one lane gathers at once: 1, 2 or 4) of the per-phase launches, after
  * autotuning; neither changes a result. Any pointer may be null. */
 int avbd_get_launch_config(avbd_ctx* ctx, uint32_t* lanes_per_vertex, uint32_t* block_size, uint32_t* gather_batch);
-/* *persistent_grid = blocks of the persistent step kernel, or 0 when the
- * step runs as one launch per phase; *fused_chebyshev = 1 when the Chebyshev /
- * dual update runs inside each iteration's last colour phase
- * (AVBD_FLAG_SEPARATE_CHEBYSHEV). Either pointer may be null. */
+/* *persistent_grid = workgroups of the launch that runs a whole stretch of a
+ * step's iterations (patches of the resident solve, or bundles of oriented
+ * particles), or 0 when the step runs as one launch per phase: scenes that do not
+ * fit (one tet mesh: about 37^3 cells in FP32, 32^3 in FP64, with damping 32^3 and 30^3)
+ * or are mixed, dynamic contacts in play, AVBD_FLAG_NO_PERSISTENT,
+ * AVBD_FLAG_SEPARATE_CHEBYSHEV, timing. *fused_chebyshev = 1 when a per-phase step
+ * runs the Chebyshev / dual update inside each iteration's last colour phase.
+ * Either pointer may be null. */
 int avbd_get_step_mode(avbd_ctx* ctx, uint32_t* persistent_grid, uint32_t* fused_chebyshev);
 /* Kernel timing: while enabled, avbd_step() launches eagerly and brackets
  * every per-colour vertex-solve launch with HIP events on the ctx stream.

@@ -75,3 +75,33 @@ def test_quiet_and_touching_steps_equal_one_launch_per_phase(fp64):
             s.ctx.load_checkpoint(c)
     print(f"[gpu-test]   contacts per step {touched}", flush=True)
     assert touched[0] == 0 and touched[11] > 0
+
+
+def test_step_mode_names_the_path_of_the_next_step():
+    from avbd_amd.sim import Simulation
+    print("[gpu-test] step mode", flush=True)
+    cube, rods = scenes.dropped_cube(n=9, height=0.004), scenes.rod_grid(2, 2, 8, iters=5)
+    grid = {}
+    for name, sc, kw in (("cube", cube, {}), ("cube64", cube, dict(fp64_state=True)), ("rods", rods, {}),
+                         ("phases", cube, dict(flags=_lib.FLAG_NO_PERSISTENT)),
+                         ("rod phases", rods, dict(flags=_lib.FLAG_NO_PERSISTENT)),
+                         ("separate", cube, dict(separate_chebyshev=True)),
+                         ("contacts", two_cubes(), {}), ("mixed", scenes.rod_on_block(), {})):
+        s = Simulation(sc, **kw)
+        s.setup()
+        grid[name] = s.ctx.persistent_grid()
+        s.ctx.set_timing(True)
+        assert s.ctx.persistent_grid() == 0
+        s.ctx.set_timing(False)
+        if name == "contacts":
+            s.update(1)
+            grid["quiet"] = s.ctx.persistent_grid()
+            s.update(12)
+            grid["touching"] = s.ctx.persistent_grid()
+        s.ctx.close()
+    print(f"[gpu-test]   {grid}", flush=True)
+    # 9^3 cells: (24 * 729 incidences + 8 * 1000 particles) / 1000 = 26 patches
+    assert grid["cube"] == grid["cube64"] == 26
+    assert 0 < grid["rods"] <= 4
+    assert grid["quiet"] > 0
+    assert all(grid[k] == 0 for k in ("phases", "rod phases", "separate", "touching", "mixed"))
