@@ -2365,8 +2365,9 @@ int avbd_build_graph(avbd_ctx* c) {
         // without oriented particles or conflicted vertices)
         // (residual mode: with an even check interval, so that every interval
         // starts on the same buffer and one interval graph serves them all)
-        const bool positional = !(c->desc.flags & AVBD_FLAG_SEPARATE_CHEBYSHEV) && c->d.n_rot == 0 &&
-                                c->d.n_oitems == 0 && c->plan.num_colors > 0 && c->plan.conflict_list.empty();
+        const bool separate = (c->desc.flags & AVBD_FLAG_SEPARATE_CHEBYSHEV) != 0;
+        const bool positional = !separate && c->d.n_rot == 0 && c->d.n_oitems == 0 && c->plan.num_colors > 0 &&
+                                c->plan.conflict_list.empty();
         if (positional && (!c->rc || c->res_check_every % 2 == 0)) {
             const uint32_t last = c->plan.num_colors - 1;
             std::vector<uint8_t> in_last(n, 0);
@@ -2383,7 +2384,7 @@ int avbd_build_graph(avbd_ctx* c) {
             c->fuse_cheb = true;
         }
         if (positional) setup_resident(c);
-        else if (c->d.n_rot == n && c->plan.conflict_list.empty()) setup_bundles(c);
+        else if (!separate && c->d.n_rot == n && c->plan.conflict_list.empty()) setup_bundles(c);
         c->built = true;
 
         // timing events bracket the solve launches of a fixed-count step

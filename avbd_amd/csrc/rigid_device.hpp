@@ -499,7 +499,8 @@ __device__ __forceinline__ Element read_element(const DevState& d, const OItem& 
 // the reference's StaticEnergyType order: Cosserat, ground (positional block),
 // rigid-ground, joint (simulation/VBDSolver.hpp:297-397).
 // W lanes (1 or 2) share the rod elements of the particle; every lane ends with
-// the whole sum, which for two elements is the sum of one lane bit for bit.
+// the whole sum, which differs from one lane's by rounding (one lane's second
+// element is contracted into the sum of the first).
 // `read`: the lane's first element, when the caller has read it already.  D
 // lanes (a power of two, `contact` of them this one) share its dynamic contacts;
 // again every lane ends with the whole sum.

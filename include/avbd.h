@@ -63,8 +63,11 @@ typedef enum {
 #define AVBD_FLAG_NO_GRAPH 1u    /* launch kernels eagerly instead of replaying a hipGraph */
 #define AVBD_FLAG_NO_PERSISTENT 4u  /* one kernel launch per solver phase also where the resident solve
                                        (all iterations of a stretch in one launch, each patch of the mesh
-                                       in one workgroup's LDS) would run; the results are identical for the
-                                       same lanes_per_vertex */
+                                       in one workgroup's LDS) or the bundles of oriented particles would
+                                       run.  Meshes: the same positions bit for bit for the same
+                                       lanes_per_vertex (residual sums add in another order: 1e-12).
+                                       Oriented particles: the two elements of a node are summed in
+                                       another order, so results differ by that rounding */
 #define AVBD_FLAG_RESIDENT_ALONE 128u /* for tests: the resident solve takes its path for a device that
                                          cannot hold all patches of a scene at once (one workgroup per
                                          scene runs all of its patches; identical results) */
@@ -88,10 +91,12 @@ typedef enum {
 #define AVBD_FLAG_HOST_COLORING 64u /* run the DSATUR colouring of avbd_build_graph on the host
                                        instead of the device (same colours; without a device the
                                        host colours anyway) */
-#define AVBD_FLAG_SEPARATE_CHEBYSHEV 16u /* run the Chebyshev / dual update of every iteration as
-                                            its own launch.  By default, in scenes without oriented
-                                            particles, it is fused into the iteration's last colour
-                                            phase over two position buffers (identical results) */
+#define AVBD_FLAG_SEPARATE_CHEBYSHEV 16u /* one launch per solver phase, and the Chebyshev / dual update of
+                                            every iteration as its own launch.  By default, in per-phase
+                                            steps without oriented particles, it is fused into the
+                                            iteration's last colour phase over two position buffers
+                                            (identical results; for bundles of oriented particles see
+                                            AVBD_FLAG_NO_PERSISTENT) */
 
 /* SimulationContext capacities + SimulationParams + VBDSolver arguments.
  * Reference: simulation/SimulationContext.hpp:46-59, simulation/SimulationParams.hpp:8-15,

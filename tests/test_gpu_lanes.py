@@ -86,6 +86,7 @@ def test_step_mode_names_the_path_of_the_next_step():
                          ("phases", cube, dict(flags=_lib.FLAG_NO_PERSISTENT)),
                          ("rod phases", rods, dict(flags=_lib.FLAG_NO_PERSISTENT)),
                          ("separate", cube, dict(separate_chebyshev=True)),
+                         ("rods separate", rods, dict(separate_chebyshev=True)),
                          ("contacts", two_cubes(), {}), ("mixed", scenes.rod_on_block(), {})):
         s = Simulation(sc, **kw)
         s.setup()
@@ -104,4 +105,4 @@ def test_step_mode_names_the_path_of_the_next_step():
     assert grid["cube"] == grid["cube64"] == 26
     assert 0 < grid["rods"] <= 4
     assert grid["quiet"] > 0
-    assert all(grid[k] == 0 for k in ("phases", "rod phases", "separate", "touching", "mixed"))
+    assert all(grid[k] == 0 for k in ("phases", "rod phases", "separate", "rods separate", "touching", "mixed"))
