@@ -1072,7 +1072,7 @@ void detect_round(avbd_ctx* c) {
               "D2H");
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     const uint32_t* st = reinterpret_cast<const uint32_t*>(c->h_det);
-    if (st[2] > c->lbd.pair_cap || (st[3] & 1u))
+    if (st[2] > c->lbd.pair_cap)
         throw CodeError(AVBD_E_CAPACITY, "broad phase: candidate pairs exceeded capacity");
     if (st[0] & NARROW_UNSUPPORTED) throw CodeError(AVBD_E_UNSUPPORTED_CONTACT, "Unsupported collision!");
     if (st[1] > c->det_cap) throw CodeError(AVBD_E_CAPACITY, "narrow phase: detected contacts exceeded capacity");
@@ -3587,7 +3587,6 @@ int avbd_download_candidates(avbd_ctx* c, uint32_t* pairs, uint32_t cap, uint32_
         uint32_t ctr[2] = {0, 0};
         hip_check(hipMemcpyAsync(ctr, b.counters, sizeof(ctr), hipMemcpyDeviceToHost, c->stream), "D2H");
         hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-        if (ctr[1] & 1u) throw CodeError(AVBD_E_CAPACITY, "LBVH traversal stack overflow");
         const uint32_t stored = std::min(ctr[0], b.pair_cap);
         const uint32_t m = std::min(stored, cap);
         if (pairs && m)

@@ -40,7 +40,7 @@ struct LbvhDev {
     TravNode* trav = nullptr;       // n - 1 internal nodes (record g - n of node g)
     uint32_t* pairs = nullptr;      // candidate leaf pairs (a < b)
     uint32_t pair_cap = 0;
-    uint32_t* counters = nullptr;   // [0] pair count, [1] status (unused: the stack holds any tree)
+    uint32_t* counters = nullptr;   // [0] pair count; [1] is cleared with it
 };
 
 uint32_t lbvh_table_entries(uint32_t n);

@@ -94,8 +94,8 @@ __device__ __forceinline__ void wave_union(double b[6]) {
 }
 
 // One block: scene box = union of the primitive boxes (in registers, then one
-// exchange between the wavefronts); also resets the pair counter, the status
-// word and the bucket counts of this build.
+// exchange between the wavefronts); also resets the pair counter
+// and the bucket counts of this build.
 __global__ __launch_bounds__(1024) void scene_box_kernel(const double* __restrict__ aabb, uint32_t n,
                                                          double* __restrict__ sbox, uint32_t* __restrict__ counters,
                                                          uint32_t* __restrict__ bucket_count) {
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(1024) void scene_box_kernel(const double* __restric
     }
     if (threadIdx.x == 0) {
         counters[0] = 0;   // pair count
-        counters[1] = 0;   // status bits
+        counters[1] = 0;
     }
 }
 

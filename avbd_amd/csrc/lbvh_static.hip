@@ -90,7 +90,7 @@ hipError_t scratch_address(int dev, unsigned char** out) {
     return hipSuccess;
 }
 
-// counters[0] = pairs found, counters[1] = status bits (an empty input never
+// counters[0] = pairs found, counters[1] = 0 (an empty input never
 // reaches the build kernels, which clear them otherwise).
 __global__ void clear_counters_kernel(uint32_t* counters) {
     if (threadIdx.x < 2) counters[threadIdx.x] = 0u;

@@ -575,11 +575,11 @@ int avbd_calibrate_copy(avbd_ctx* ctx, uint64_t bytes, uint32_t iters, double* a
  *   pairs     device output of up to pair_cap candidate leaf pairs (a < b,
  *             sorted-order leaf indices, 2 uint32 each, order unspecified);
  *   counters  device output of 2 uint32: [0] pairs found (> pair_cap means
- *             truncated), [1] status (bit 0: traversal stack overflow);
+ *             truncated), [1] cleared (the traversal stack holds any tree);
  *   stream    hipStream_t to launch on (NULL = the null stream).
  * Asynchronous: outputs are valid once the stream has reached this point.
  * Every intermediate array lives in one static device array of the library
- * (about 6.7 MiB per GPU, held from the first call on a device until the
+ * (about 6.8 MiB per GPU, held from the first call on a device until the
  * process ends), so a call allocates nothing and never synchronises.  At most
  * AVBD_NOALLOC_MAX_TRIANGLES triangles (AVBD_E_CAPACITY beyond).  Calls on one
  * GPU share that array: calls that overlap in time on one GPU race.  Errors
