@@ -2853,10 +2853,10 @@ int avbd_get_launch_config(avbd_ctx* c, uint32_t* lanes, uint32_t* block, uint32
 int avbd_get_step_mode(avbd_ctx* c, uint32_t* persistent_grid, uint32_t* fused_chebyshev) {
     if (!c) return AVBD_E_ARG;
     if (persistent_grid)
-        *persistent_grid = c->timing                      ? 0u
-                           : uses_resident(c)             ? c->res.n_patches
-                           : c->bundled && !c->dynamic    ? c->bundles.n_bundles
-                                                          : 0u;
+        *persistent_grid = c->timing && !c->rc         ? 0u   // (only fixed-count steps are timed per phase)
+                           : uses_resident(c)          ? c->res.n_patches
+                           : c->bundled && !c->dynamic ? c->bundles.n_bundles
+                                                       : 0u;
     if (fused_chebyshev) *fused_chebyshev = (c->fuse_cheb && (!c->dynamic || dyn_quiet(c))) ? 1u : 0u;
     return AVBD_OK;
 }

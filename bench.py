@@ -12,9 +12,11 @@ launch to its completion, inputs resident in HBM; `steps` steps are timed
 after `warmup` untimed ones.
 
 Also reported: the reference's fixed count of 10 iterations per step with an
-FP32 state (`fixed_iterations`), the roofline of the dominant kernel (the
-per-colour vertex-block solve of the headline leg: algorithmic bytes per
-launch over its average duration, measured with HIP events on the
+FP32 state (`fixed_iterations`), the roofline of the kernel that the headline
+leg's steps spend their time in (the resident solve: bytes an iteration reads
+from LDS over its duration, the slope of step time over iterations; or, where a
+step is one launch per phase, the per-colour vertex-block solve: algorithmic
+bytes per launch over its average duration, measured with HIP events on the
 library's stream), and the CPU baseline: the FP64 C++ restatement of the
 reference's multithreaded CPU path on this machine's host cores, fixed-count
 and residual-targeted, with the thread count and a one-thread figure.
@@ -38,6 +40,7 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "sim steps/sec at fixed force residual, warm-start vs plain; vertex-updates/sec"
 HBM_PEAK_GBS = 8000.0
+LDS_PEAK_GBS = 256 * 128 * 2.4   # CUs x bytes per clock x GHz
 CPU_SHARE = 16   # host CPUs allotted to one GPU on the measurement machines
 
 
@@ -90,6 +93,35 @@ def solve_bytes_per_launch(sc, n_colors: int, fp64: bool) -> float:
     else:
         total = 40 * n_items + 100 * n_inc + 48 * n_g
     return total / n_colors
+
+
+def resident_roofline(sim, sc, fp64: bool, us_per_iteration: float, measured: str):
+    """The resident solve (avbd_get_step_mode): what one iteration reads from LDS
+    for the vertex solves, over the duration of an iteration.  Per incidence
+    FP64 undamped 120 B (8 B of indices, five constants, three positions), FP32
+    106 B (indices, rest shape and material, four positions), with damping 32 B
+    more (FP64: 154 + 32); per vertex its position, target, mass and ground
+    force; Chebyshev and dual update not counted.  The rate is far from the LDS
+    peak: a phase is one chain of latencies (gather, sum, solve, exchange)."""
+    n_items, n_inc, n_g = free_counts(sc)
+    damp = any(m.kd > 0 for m in sc.meshes)
+    real = 8 if fp64 else 4
+    inc = (120 if fp64 and not damp else 58 + 12 * real) + (32 if damp else 0)
+    lds = n_inc * inc + n_items * (7 * real + 8) + n_g * (3 * real + 16)
+    achieved = lds / (us_per_iteration * 1e-6) / 1e9
+    return {"kernel": "resident_kernel", "bound": "lds", "achieved": round(achieved, 1), "peak": LDS_PEAK_GBS,
+            "unit": "GB/s", "frac": round(achieved / LDS_PEAK_GBS, 4), "traffic": None,
+            "us_per_iteration": round(us_per_iteration, 3), "measured": measured, "lds_bytes_per_iteration": int(lds),
+            "workgroups": sim.ctx.persistent_grid(), "lanes_per_vertex": sim.ctx.launch_config()[0]}
+
+
+def iteration_slope(leg) -> float:
+    """us per iteration of a leg's steps: the slope of step time over iterations
+    (the detection round, warm start and velocity of a step drop out)."""
+    its, ms = np.array(leg["iterations_per_step"], float), np.array(leg["ms_per_step_each"])
+    if len(its) < 3 or its.max() < 2 * max(its.min(), 1):
+        return 1e3 * ms.sum() / its.sum()
+    return 1e3 * float(np.polyfit(its, ms, 1)[0])
 
 
 def residual_leg(workload: str, args, launch: dict, params=None, budget=None):
@@ -151,7 +183,8 @@ def residual_leg(workload: str, args, launch: dict, params=None, budget=None):
         out["fallbacks_to_inertial_start"] = int(s1.warm_start_fallbacks - s0.warm_start_fallbacks)
     lanes, block, batch = sim.ctx.launch_config()
     out["launch_config"] = {"lanes_per_vertex": lanes, "block_size": block, "gather_batch": batch,
-                            "fused_chebyshev": sim.ctx.fused_chebyshev()}
+                            "fused_chebyshev": sim.ctx.fused_chebyshev(),
+                            "resident_workgroups": sim.ctx.persistent_grid()}
     return sim, out
 
 
@@ -314,7 +347,7 @@ def main():
     ap.add_argument("--fixed-steps", type=int, default=200, help="timed steps of the fixed-iteration leg")
     ap.add_argument("--no-fixed", action="store_true", help="skip the fixed-iteration leg")
     ap.add_argument("--no-residual", action="store_true", help="skip the residual-targeted legs of the workload")
-    ap.add_argument("--lanes-per-vertex", type=int, default=0, help="0: autotuned at set-up")
+    ap.add_argument("--lanes-per-vertex", type=int, default=0, help="0: by the size of the scene")
     ap.add_argument("--block-size", type=int, default=0, help="0: autotuned at set-up")
     ap.add_argument("--gather-batch", type=int, default=0, help="0: autotuned at set-up")
     ap.add_argument("--res-eager", action="store_true",
@@ -373,9 +406,12 @@ def main():
                "speedup_warm_vs_plain": round(warm["steps_per_s"] / plain["steps_per_s"], 3) if warm else None,
                "steps_per_s": best["steps_per_s"], "ms_per_step": best["ms_per_step"],
                "vertex_updates_per_s": best["vertex_updates_per_s"]}
-        # dominant kernel of the headline leg: the per-colour vertex solve
+        # dominant kernel of the headline leg
         ksim = sim_w
-        if ksim is not None:
+        if ksim is not None and ksim.ctx.persistent_grid():
+            roof = resident_roofline(ksim, sc, fp64, iteration_slope(warm), "slope of step time over iterations")
+            ksim.ctx.close()
+        elif ksim is not None:
             avg_ms, launches = ksim.ctx.time_solve_launches(20)
             _, n_colors = ksim.ctx.coloring()
             bytes_launch = solve_bytes_per_launch(sc, n_colors, fp64)
@@ -387,7 +423,7 @@ def main():
                     "launches_timed": launches}
             # measured HBM bytes per launch (rocprofv3 FETCH_SIZE / WRITE_SIZE
             # runs, profiles/), used only when they were taken on the variant
-            # timed here
+            # timed here, reading the same records
             lanes, _, batch = ksim.ctx.launch_config()
             damp = any(m.kd > 0 for m in sc.meshes)
             if dynamic and contact_aware_step(ksim):   # one incidence gathered per lane in FP64
@@ -397,12 +433,13 @@ def main():
                 variant = (f"solve_color_f64_kernel<{lanes}, {str(damp).lower()}, {batch}, false>" if fp64 else
                            f"solve_color_kernel<{lanes}, {str(damp).lower()}, false, {batch}>")
             roof["variant"] = variant
+            record = "EdgeRec64" if fp64 and not damp else "TetRec"
             # the workload's own profile, else the one of its scene (the same
             # cube without the self-collision pass runs the same static kernel)
             for stem in (args.workload, sc.name):
                 prof = ROOT / "profiles" / f"{kernel}_{stem}_traffic.json"
                 t = json.loads(prof.read_text()) if prof.exists() else {}
-                if t.get("variant") == variant:
+                if t.get("variant") == variant and t.get("record") == record:
                     roof["traffic"] = t.get("bytes_per_launch")
                     roof["traffic_source"] = t.get("source")
                     break
@@ -425,30 +462,39 @@ def main():
         n_detected = len(sim.ctx.detected()[0]) if dynamic else None
         fixed_rate = args.fixed_steps / el
         vups = st.vertex_updates / max(st.steps_taken, 1) * fixed_rate
+        resident = sim.ctx.persistent_grid() > 0
         sim.ctx.set_timing(True)
         sim.ctx.step(2)
         lbvh_ms = sim.ctx.broadphase_timing()
         sim.ctx.set_timing(False)
-        f_avg_ms, f_launches = sim.ctx.time_solve_launches(20)
-        _, n_colors = sim.ctx.coloring()
-        f_bytes = solve_bytes_per_launch(sc, n_colors, False)
+        meshes = not (sc.rods or sc.spheres)
+        if resident and meshes:
+            solve = resident_roofline(sim, sc, False, el / args.fixed_steps / sc.iters * 1e6,
+                                      "step time over its iterations, the rest of the step included")
+        elif resident:
+            solve = {"kernel": "bundle_kernel", "workgroups": sim.ctx.persistent_grid()}
+        else:
+            f_avg_ms, f_launches = sim.ctx.time_solve_launches(20)
+            _, n_colors = sim.ctx.coloring()
+            f_bytes = solve_bytes_per_launch(sc, n_colors, False)
+            achieved = round(f_bytes / (f_avg_ms * 1e-3) / 1e9, 1) if f_avg_ms > 0 else 0
+            solve = {"kernel": "solve_color_kernel", "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
+                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
+                     "avg_launch_us": round(f_avg_ms * 1e3, 3), "algorithmic_bytes_per_launch": int(f_bytes),
+                     "launches_timed": f_launches}
         lanes, block, batch = sim.ctx.launch_config()
         fixed = {"iterations": sc.iters, "state": "fp32", "steps": args.fixed_steps,
                  "steps_per_s": round(fixed_rate, 3), "ms_per_step": round(el / args.fixed_steps * 1e3, 4),
                  "vertex_updates_per_s": round(vups, 1), "final_residual_rel": st.residual_rel,
                  "setup_s": round(t_setup, 2),
                  "contacts_detected_last_step": n_detected,
-                 "solve_kernel": {"kernel": "solve_color_kernel", "avg_launch_us": round(f_avg_ms * 1e3, 3),
-                                  "algorithmic_bytes_per_launch": int(f_bytes),
-                                  "achieved_GBps": round(f_bytes / (f_avg_ms * 1e-3) / 1e9, 1) if f_avg_ms > 0 else 0},
+                 "solve_kernel": solve,
                  "launch_config": {"lanes_per_vertex": lanes, "block_size": block, "gather_batch": batch,
-                                   "fused_chebyshev": sim.ctx.fused_chebyshev()}}
+                                   "fused_chebyshev": sim.ctx.fused_chebyshev(),
+                                   "resident_workgroups": sim.ctx.persistent_grid()}}
         log(f"fixed-count leg: {fixed_rate:.1f} steps/s, residual_rel {st.residual_rel:.3e}")
-        if roof is None and f_launches:
-            roof = {"kernel": "solve_color_kernel", "bound": "hbm", "achieved": fixed["solve_kernel"]["achieved_GBps"],
-                    "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(fixed["solve_kernel"]["achieved_GBps"] / HBM_PEAK_GBS, 4),
-                    "traffic": None, "avg_launch_us": round(f_avg_ms * 1e3, 3),
-                    "algorithmic_bytes_per_launch": int(f_bytes), "launches_timed": f_launches}
+        if roof is None and "achieved" in solve:
+            roof = solve
         calib = None
         if args.calibrate:
             ms = sim.ctx.calibrate_copy(args.calibrate, 10)

@@ -377,7 +377,7 @@ int avbd_get_launch_config(avbd_ctx* ctx, uint32_t* lanes_per_vertex, uint32_t* 
  * particles), or 0 when the step runs as one launch per phase: scenes that do not
  * fit (one tet mesh: about 37^3 cells in FP32, 32^3 in FP64, with damping 32^3 and 30^3)
  * or are mixed, dynamic contacts in play, AVBD_FLAG_NO_PERSISTENT,
- * AVBD_FLAG_SEPARATE_CHEBYSHEV, timing. *fused_chebyshev = 1 when a per-phase step
+ * AVBD_FLAG_SEPARATE_CHEBYSHEV, timed fixed-count steps. *fused_chebyshev = 1 when a per-phase step
  * runs the Chebyshev / dual update inside each iteration's last colour phase.
  * Either pointer may be null. */
 int avbd_get_step_mode(avbd_ctx* ctx, uint32_t* persistent_grid, uint32_t* fused_chebyshev);

@@ -83,6 +83,7 @@ def test_step_mode_names_the_path_of_the_next_step():
     cube, rods = scenes.dropped_cube(n=9, height=0.004), scenes.rod_grid(2, 2, 8, iters=5)
     grid = {}
     for name, sc, kw in (("cube", cube, {}), ("cube64", cube, dict(fp64_state=True)), ("rods", rods, {}),
+                         ("target", cube, dict(residual_target=(1e-3, 100, 10))),
                          ("phases", cube, dict(flags=_lib.FLAG_NO_PERSISTENT)),
                          ("rod phases", rods, dict(flags=_lib.FLAG_NO_PERSISTENT)),
                          ("separate", cube, dict(separate_chebyshev=True)),
@@ -92,7 +93,7 @@ def test_step_mode_names_the_path_of_the_next_step():
         s.setup()
         grid[name] = s.ctx.persistent_grid()
         s.ctx.set_timing(True)
-        assert s.ctx.persistent_grid() == 0
+        assert s.ctx.persistent_grid() == (grid[name] if name == "target" else 0)
         s.ctx.set_timing(False)
         if name == "contacts":
             s.update(1)
@@ -102,7 +103,7 @@ def test_step_mode_names_the_path_of_the_next_step():
         s.ctx.close()
     print(f"[gpu-test]   {grid}", flush=True)
     # 9^3 cells: (24 * 729 incidences + 8 * 1000 particles) / 1000 = 26 patches
-    assert grid["cube"] == grid["cube64"] == 26
+    assert grid["cube"] == grid["cube64"] == grid["target"] == 26
     assert 0 < grid["rods"] <= 4
     assert grid["quiet"] > 0
     assert all(grid[k] == 0 for k in ("phases", "rod phases", "separate", "rods separate", "touching", "mixed"))
