@@ -1406,7 +1406,8 @@ void setup_resident(avbd_ctx* c) {
     r.block = resident_block(plan, c->plan.num_colors, lim, r.lanes);
     // about 50 ms (0.13 us each): half of what 100 iterations of a large scene take alone (1 ms each
     // at 32^3), so that waiting for another stream's work costs less than giving up
-    r.gather_polls = c->desc.flags & AVBD_FLAG_RESIDENT_ALONE ? 0u : 400000u;
+    r.gather_polls = 400000u;
+    r.alternate = (c->desc.flags & AVBD_FLAG_RESIDENT_ALONE) != 0;
     r.has_ground = lim.ground;
     r.cus = lim.max_cluster;
     r.per_cu = resident_per_cu(r, c->fp64, c->damping);

@@ -140,6 +140,7 @@ struct ResidentDev {
     uint32_t n_patches = 0, n_colors = 0, lds_bytes = 0, max_cluster = 0, lanes = 8, block = 512;
     uint32_t cus = 0, per_cu = 0;        // of the device; workgroups of this launch that fit on one of them
     uint32_t gather_polls = 0;           // polls after which a patch no longer waits for its cluster to be resident
+    bool alternate = false;              // for tests: odd launches do not wait for it
     bool has_ground = false;
 };
 

@@ -522,10 +522,11 @@ __global__ __launch_bounds__(B) void resident_kernel(Args<R> a) {
                 __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.count - 1u;
             if (full)   // everyone has arrived: ready for the next launch
                 __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t patience = a.r.alternate && (launch & 1u) ? 0u : a.r.gather_polls;
             uint32_t polls = 0;
             uint32_t now = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             while ((int32_t)(now - want) < 0) {
-                if (full || polls++ >= a.r.gather_polls) {
+                if (full || polls++ >= patience) {
                     uint32_t seen = now;
                     const uint32_t next = full ? want : want + 1u;
                     now = __hip_atomic_compare_exchange_strong(word, &seen, next, __ATOMIC_RELAXED, __ATOMIC_RELAXED,

@@ -68,9 +68,10 @@ typedef enum {
                                        lanes_per_vertex (residual sums add in another order: 1e-12).
                                        Oriented particles: the two elements of a node are summed in
                                        another order, so results differ by that rounding */
-#define AVBD_FLAG_RESIDENT_ALONE 128u /* for tests: the resident solve takes its path for a device that
-                                         cannot hold all patches of a scene at once (one workgroup per
-                                         scene runs all of its patches; identical results) */
+#define AVBD_FLAG_RESIDENT_ALONE 128u /* for tests: every other launch of the resident solve takes its
+                                         path for a device that cannot hold all patches of a scene at
+                                         once (one workgroup per scene runs all of its patches;
+                                         identical results) */
 #define AVBD_FLAG_PERSISTENT 8u     /* rejected by avbd_create (AVBD_E_ARG): a step kernel
                                        with grid barriers was removed.  Every barrier needed agent-scope
                                        release / acquire fences, which write back and invalidate

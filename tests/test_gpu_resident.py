@@ -3,8 +3,8 @@ of a scene in the LDS of workgroups that exchange boundary positions) equals
 one launch per phase bit for bit at the same lanes per vertex, whatever the
 partition: scenes of one patch and of many, patches of odd sizes, particles
 without a free neighbour, damping, ground contacts, batches of scenes of
-different sizes, odd iteration counts, and the path for a device that cannot
-hold a scene's patches at once."""
+different sizes, odd iteration counts, and launches that alternate between the
+exchange and the path for a device that cannot hold a scene's patches at once."""
 import numpy as np
 import pytest
 
@@ -20,8 +20,8 @@ def scene_of(kind, n):
         sc = scenes.dropped_cube(n=n, height=0.01)
         for m in sc.meshes:
             m.kd = 1e-3
-    elif kind == "batch":
-        sc = scenes.cube_batch(n_scenes=n, n_min=1, n_max=9)
+    elif kind in ("batch", "crowd"):
+        sc = scenes.cube_batch(n_scenes=n, n_min=1, n_max=9 if kind == "batch" else 14)
         for m in sc.meshes:
             m.rest[:, 1] += 0.01 - m.rest[:, 1].min()
     else:
@@ -30,9 +30,13 @@ def scene_of(kind, n):
 
 
 # a single cell, a cube below one patch, just above it, tens of patches, ragged
-# ones; lanes below and above the number of 32-bit pieces of a position
+# ones; lanes below and above the number of 32-bit pieces of a position; patches that fill
+# the LDS and have more items in a phase than 512 threads hold groups (FP32: 1,024 threads,
+# FP64: a group takes a second item), one scene and many, damped and not; a crowd's
+# larger cubes do not fit as they are first cut
 CASES = [("hang", 1, 8), ("hang", 2, 4), ("drop", 5, 16), ("drop", 6, 32), ("drop", 13, 8), ("damped", 3, 8),
-         ("damped", 9, 32), ("batch", 7, 8), ("batch", 40, 4)]
+         ("damped", 9, 32), ("batch", 7, 8), ("batch", 40, 4), ("drop", 32, 16), ("drop", 32, 32), ("damped", 28, 32),
+         ("crowd", 400, 8), ("crowd", 400, 32)]
 
 
 @pytest.mark.parametrize("fp64", [False, True])
@@ -47,6 +51,7 @@ def test_resident_equals_one_launch_per_phase(kind, n, lanes, fp64):
             for f in (_lib.FLAG_NO_PERSISTENT, 0, _lib.FLAG_RESIDENT_ALONE, _lib.FLAG_NO_GRAPH)]
     for r in runs:
         r.setup()
+        assert (r.ctx.persistent_grid() > 0) == (r is not runs[0])
     for k in range(3):
         for r in runs:
             r.update(3)
