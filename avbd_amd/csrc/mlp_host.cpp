@@ -157,7 +157,7 @@ void MlpModel::ensure_batch(int rows) {
     if (pad <= cap_rows) return;
     for (void* p : batch_owned) (void)hipFree(p);
     batch_owned.clear();
-    cap_rows = pad;
+    cap_rows = 0;   // until every buffer is there: an allocation may fail
     x16 = dalloc<uint16_t>(batch_owned, (size_t)pad * kMlpInPad);
     for (int l = 0; l < kMlpLayers; l++) {
         z32[l] = dalloc<float>(batch_owned, (size_t)pad * mlp_layer_out(l));
@@ -167,6 +167,7 @@ void MlpModel::ensure_batch(int rows) {
     t32 = dalloc<float>(batch_owned, (size_t)pad * kMlpOut);
     raw_x = dalloc<float>(batch_owned, (size_t)pad * kMlpIn);
     raw_t = dalloc<float>(batch_owned, (size_t)pad * kMlpOut);
+    cap_rows = pad;
 }
 
 // Workspace of the backward pass: partial gradients per row chunk (at most 64
@@ -174,12 +175,14 @@ void MlpModel::ensure_batch(int rows) {
 void MlpModel::ensure_grad_parts(int rows_pad) {
     const int chunks = mlp_grad_chunks(rows_pad), losses = mlp_loss_parts(rows_pad);
     if (chunks <= part_chunks && losses <= loss_parts) return;
+    const int most = std::max(part_chunks, chunks), parts = std::max(loss_parts, losses);
     for (void* p : part_owned) (void)hipFree(p);
     part_owned.clear();
-    part_chunks = std::max(part_chunks, chunks);
-    loss_parts = std::max(loss_parts, losses);
-    part = dalloc<float>(part_owned, (size_t)part_chunks * weight_count());
-    loss_part = dalloc<float>(part_owned, loss_parts);
+    part_chunks = loss_parts = 0;
+    part = dalloc<float>(part_owned, (size_t)most * weight_count());
+    loss_part = dalloc<float>(part_owned, parts);
+    part_chunks = most;
+    loss_parts = parts;
 }
 
 // Forward pass of rows_pad rows of x16 (bf16, normalised, padded): with
