@@ -1153,17 +1153,20 @@ void detect_round(avbd_ctx* c) {
 // the colour phases changed its choice: undamped FP32 32 lanes up to 22^3 cells
 // (3,042 items in the largest colour) and 8 from 3,479 (16 cubes) and 24^3 (3,907) on; FP64
 // 32 up to 14^3 (844), 8 from 16^3 (1,229) on; damped, whose incidence is twice the
-// work, 32 up to 24^3 (3,907), 16 at 32^3 (8,985).  The resident solve agrees but
+// work, 32 up to 24^3 (3,907), 16 at 32^3 (8,985); without ground records 32 up to
+// 23^3 (3,312), 16 at 24^3 (3,750) and 28^3 (5,887), 8 from 30^3 (7,208) on.  The resident solve agrees but
 // for a few per cent between the lines; step of 10 iterations at 8 / 16 / 32 lanes in
 // us: FP32 15^3 151 / 134 / 125, 22^3 160 / 142 / 137, 28^3 168 / 159 / 170, 32^3 189 /
 // 179 / 205; FP64 14^3 132 / 123 / 125, 32^3 177 / 192 / 251; damped 16^3 180 / 155 /
 // 137, 24^3 192 / 170 / 165, 32^3 226 / 217 / 236.
-uint32_t default_lanes(const ColorPlan& plan, bool fp64, bool damping) {
+uint32_t default_lanes(const ColorPlan& plan, bool fp64, bool damping, bool ground) {
     uint32_t most = 0;
     for (uint32_t c = 0; c < plan.num_colors; c++)
         most = std::max(most, plan.item_offsets[c + 1] - plan.item_offsets[c]);
     if (damping) return most <= 4608 ? 32u : (most <= 9216 ? 16u : 8u);
-    return most <= (fp64 ? 1024u : 3072u) ? 32u : 8u;
+    if (fp64) return most <= 1024 ? 32u : 8u;
+    if (!ground) return most <= 3500 ? 32u : (most <= 6500 ? 16u : 8u);
+    return most <= 3072 ? 32u : 8u;
 }
 
 // Temporary device buffers, freed when the holder goes out of scope.
@@ -2068,7 +2071,7 @@ int avbd_build_graph(avbd_ctx* c) {
         c->damping = false;
         for (const auto& t : c->nh)
             if (t.kd != 0.0) c->damping = true;
-        if (!c->desc.lanes_per_vertex) c->cfg.lanes = default_lanes(c->plan, c->fp64, c->damping);
+        if (!c->desc.lanes_per_vertex) c->cfg.lanes = default_lanes(c->plan, c->fp64, c->damping, !c->ground.empty());
 
         DevState& d = c->d;
         d.n = n;

@@ -8,7 +8,6 @@
 #include "dyn_device.hpp"
 #include "internal.hpp"
 #include "rot_math.hpp"
-#include "tet_device.hpp"
 
 namespace avbd {
 namespace rigid {
@@ -501,13 +500,10 @@ __device__ __forceinline__ Element read_element(const DevState& d, const OItem& 
 // W lanes (1 or 2) share the rod elements of the particle; every lane ends with
 // the whole sum, which differs from one lane's by rounding (one lane's second
 // element is contracted into the sum of the first).
-// `read`: the lane's first element, when the caller has read it already.  D
-// lanes (a power of two, `contact` of them this one) share its dynamic contacts;
-// again every lane ends with the whole sum.
-template <bool DYN = false, int W = 1, int D = 1>
+// `read`: the lane's first element, when the caller has read it already.
+template <bool DYN = false, int W = 1>
 __device__ __forceinline__ void accumulate6(const DevState& d, const OItem& it, float3 pos, float4 q, Vec6& G,
-                                            Sym6& H, uint32_t lane = 0, const Element* read = nullptr,
-                                            uint32_t contact = 0) {
+                                            Sym6& H, uint32_t lane = 0, const Element* read = nullptr) {
     const uint32_t ncos = it.n_cos & ~VITEM_CONFLICT;
     uint32_t k = it.inc_begin + ncos;
     for (uint32_t e = lane; e < ncos; e += W) {
@@ -560,32 +556,19 @@ __device__ __forceinline__ void accumulate6(const DevState& d, const OItem& it, 
     if constexpr (DYN) {
         const dyn::View view = dyn::view_of(d);
         const uint32_t e1 = d.dyn_off[it.v + 1];
-        Vec6 g;
-        Sym6 h;
-        if constexpr (D > 1) {
-            vec6_zero(g);
-            sym6_zero(h);
-        }
-        for (uint32_t e = d.dyn_off[it.v] + contact; e < e1; e += D) {
+        for (uint32_t e = d.dyn_off[it.v]; e < e1; e++) {
             const uint32_t code = d.dyn_ent[e];
             const DynRec c = d.dyn[code >> 3];
-            if constexpr (D > 1) dyn::accumulate6(view, c, code & 7u, g, h);
-            else dyn::accumulate6(view, c, code & 7u, G, H);
-        }
-        if constexpr (D > 1) {
-#pragma unroll
-            for (int i = 0; i < 6; i++) G.v[i] += group_sum<D>(g.v[i]);
-#pragma unroll
-            for (int i = 0; i < 21; i++) H.a[i] += group_sum<D>(h.a[i]);
+            dyn::accumulate6(view, c, code & 7u, G, H);
         }
     }
 }
 
 // _solveParticle<6> (simulation/VBDSolver.hpp:450-486): W lanes per oriented vertex
-// (lane W - 1 writes), or D lanes (lane 0 writes).
-template <bool DYN = false, int W = 1, int D = 1>
+// (lane W - 1 writes).
+template <bool DYN = false, int W = 1>
 __device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, float inv_dt2, uint32_t lane = 0,
-                                            const Element* read = nullptr, uint32_t contact = 0) {
+                                            const Element* read = nullptr) {
     const float4 xv = d.x[it.v];
     const float3 pos = xyz(xv);
     const float4 q = d.q[it.rot];
@@ -593,7 +576,7 @@ __device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, 
     Sym6 H;
     vec6_zero(G);
     sym6_zero(H);
-    accumulate6<DYN, W, D>(d, it, pos, q, G, H, lane, read, contact);
+    accumulate6<DYN, W>(d, it, pos, q, G, H, lane, read);
     const float md = xv.w * inv_dt2;
     const float3 I = xyz(d.inertia[it.rot]);
     const float3 yv = xyz(d.y[it.v]);
@@ -611,7 +594,7 @@ __device__ __forceinline__ void solve_oitem(const DevState& d, const OItem& it, 
     lu6(H, b, dx);
     const float4 nx = make_float4(pos.x + dx[0], pos.y + dx[1], pos.z + dx[2], xv.w);
     const float4 nq = plus_s3(q, v3(dx[3], dx[4], dx[5]));
-    if (lane != W - 1 || contact != 0) return;
+    if (lane != W - 1) return;
     if (it.n_cos & VITEM_CONFLICT) {
         d.x_buf[it.v] = nx;
         d.q_buf[it.rot] = nq;

@@ -206,7 +206,7 @@ __device__ __forceinline__ void sym6_outer(Sym6& h, const float a[6], float s) {
 // pivot is the first row of largest magnitude in the column; the row swaps
 // are register selects, so every index stays compile-time.
 __device__ __forceinline__ void lu6(const Sym6& S, const float b[6], float x[6]) {
-    float A[6][6], r[6], inv[6];   // inv: one division per pivot
+    float A[6][6], r[6];
 #pragma unroll
     for (int i = 0; i < 6; i++) {
         r[i] = b[i];
@@ -238,10 +238,10 @@ __device__ __forceinline__ void lu6(const Sym6& S, const float b[6], float x[6])
             r[k] = sw ? r[i] : t;
             r[i] = sw ? t : r[i];
         }
-        inv[k] = 1.f / A[k][k];
+        const float inv = 1.f / A[k][k];
 #pragma unroll
         for (int i = k + 1; i < 6; i++) {
-            const float f = A[i][k] * inv[k];
+            const float f = A[i][k] * inv;
 #pragma unroll
             for (int j = k + 1; j < 6; j++) A[i][j] -= f * A[k][j];
             r[i] -= f * r[k];
@@ -252,7 +252,7 @@ __device__ __forceinline__ void lu6(const Sym6& S, const float b[6], float x[6])
         float t = r[i];
 #pragma unroll
         for (int j = i + 1; j < 6; j++) t -= A[i][j] * x[j];
-        x[i] = t * inv[i];
+        x[i] = t / A[i][i];
     }
 }
 

@@ -59,17 +59,39 @@ struct DynArgs {
 __host__ __device__ __forceinline__ DynArgs dyn_args(const DevState& d) {
     return DynArgs{d.dyn_off, d.dyn_ent, d.dyn, d.q, d.rot_of};
 }
-// Contacts `lane`, lane + L, ... of particle v.
+// The contacts of particle v added in list order to g and h, as one lane would:
+// the lanes of its group form the terms of up to L contacts side by side (each a
+// chain of loads through the record to its vertices) and every lane then adds
+// them one after the other.  8.3 -> 5.9 us per colour phase of 24^3 cells under 36
+// spheres against the leader alone; a sum across the lanes took 5.2, but in another
+// order, and the friction of a contact branches on the last bit.
 template <int L>
 __device__ __forceinline__ void dyn_add3(const DynArgs& a, const float4* x, uint32_t v, uint32_t lane, float3& g,
                                          Sym3& h) {
     if (!a.off) return;
     const dyn::View view{x, a.q, a.rot_of};
     const uint32_t e1 = a.off[v + 1];
-    for (uint32_t e = a.off[v] + lane; e < e1; e += L) {
-        const uint32_t code = a.ent[e];
-        const DynRec c = a.rec[code >> 3];
-        dyn::accumulate3(view, c, code & 7u, g, h);
+    for (uint32_t e0 = a.off[v]; e0 < e1; e0 += L) {
+        float3 cg = make_float3(0.f, 0.f, 0.f);
+        Sym3 ch = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (e0 + lane < e1) {
+            const uint32_t code = a.ent[e0 + lane];
+            const DynRec c = a.rec[code >> 3];
+            dyn::accumulate3(view, c, code & 7u, cg, ch);
+        }
+        const uint32_t n = min((uint32_t)L, e1 - e0);
+        for (uint32_t k = 0; k < n; k++) {
+            auto of = [&](float t) { return L == 1 ? t : __shfl(t, (int)k, L); };
+            g.x += of(cg.x);
+            g.y += of(cg.y);
+            g.z += of(cg.z);
+            h.a00 += of(ch.a00);
+            h.a11 += of(ch.a11);
+            h.a22 += of(ch.a22);
+            h.a01 += of(ch.a01);
+            h.a02 += of(ch.a02);
+            h.a12 += of(ch.a12);
+        }
     }
 }
 
@@ -90,14 +112,10 @@ __device__ __forceinline__ uint32_t xcd_logical_block() {
 // are loaded together, then its vertex positions together with the next
 // batch's records, then its terms are added in incidence order -- the same
 // order and arithmetic as one at a time, with fewer dependent memory round trips.
-// With `da` the lanes share the item's dynamic contacts as well, ahead of the sum
-// (the leader alone took them one after the other behind it: 8.3 -> 5.1 us per
-// colour phase of 24^3 cells under 36 spheres).
 template <int L, bool DAMP, int U>
 __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, const uint32_t* __restrict__ inc,
                                               const TetRec* __restrict__ irec, const TetDamp* __restrict__ damp,
-                                              const float4* x, float inv_dt, float3& g, Sym3& h,
-                                              const DynArgs* da = nullptr) {
+                                              const float4* x, float inv_dt, float3& g, Sym3& h) {
     using Inc = TetInc<DAMP>;
     const uint32_t place = sum_place<L>(lane);
     const uint32_t cnt = it.inc_count & ~VITEM_CONFLICT, base = it.inc_begin;
@@ -122,7 +140,6 @@ __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, co
 #pragma unroll
         for (int u = 0; u < U; u++) cur[u] = next[u];
     }
-    if (da) dyn_add3<L>(*da, x, it.v, lane, g, h);
     g.x = group_sum<L>(g.x);
     g.y = group_sum<L>(g.y);
     g.z = group_sum<L>(g.z);
@@ -138,8 +155,7 @@ __device__ __forceinline__ void item_gradient(const VItem& it, uint32_t lane, co
 // and the 3x3 solve; returns the new position.
 __device__ __forceinline__ float4 item_solve(const VItem& it, float4 xv, float4 yv, const GroundRec& gr, float3 g,
                                              Sym3 h, float inv_dt2) {
-    const float3 p = f3(xv);
-    if (it.ground >= 0) ground_accumulate(gr, p, g, h);
+    if (it.ground >= 0) ground_accumulate(gr, f3(xv), g, h);
     return block_step(xv, yv, g, h, inv_dt2);
 }
 
@@ -163,9 +179,18 @@ __device__ __forceinline__ void solve_item(const VItem& it, uint32_t lane, const
     }
     float3 g;
     Sym3 h;
-    item_gradient<L, DAMP, U>(it, lane, inc, irec, damp, x, inv_dt, g, h, DYN ? &da : nullptr);
-    if (!lead) return;
-    const float4 nx = item_solve(it, xv, yv, gr, g, h, inv_dt2);
+    item_gradient<L, DAMP, U>(it, lane, inc, irec, damp, x, inv_dt, g, h);
+    float4 nx;
+    if constexpr (DYN) {
+        // the contacts follow the ground terms
+        if (lead && it.ground >= 0) ground_accumulate(gr, f3(xv), g, h);
+        dyn_add3<L>(da, x, it.v, lane, g, h);
+        if (!lead) return;
+        nx = block_step(xv, yv, g, h, inv_dt2);
+    } else {
+        if (!lead) return;
+        nx = item_solve(it, xv, yv, gr, g, h, inv_dt2);
+    }
     if (it.inc_count & VITEM_CONFLICT) x_buf[it.v] = nx;
     else x_out[it.v] = nx;
 }
@@ -575,23 +600,6 @@ __global__ __launch_bounds__(256) void solve_ocolor_kernel(DevState d, uint32_t 
     const OItem it = d.oitems[begin + k];
     if (d.frozen && d.frozen[d.scene_of[it.v]]) return;
     rigid::solve_oitem<DYN>(d, it, inv_dt2);
-}
-
-// The same with the dynamic contacts of a particle shared by kContactLanes
-// lanes: a sphere on a mesh has ten and more, and one thread takes them one after
-// the other, each a chain of loads.  36 spheres on a block: 13.9 -> 6.8 us per
-// launch.  The other terms are repeated by every lane, so this is for launches
-// whose lanes would else be idle: up to kContactItems particles, one wavefront
-// for each of the 1,024 SIMDs.
-constexpr uint32_t kContactLanes = 16, kContactItems = 4096;
-__global__ __launch_bounds__(256) void solve_ocontact_kernel(DevState d, uint32_t begin, uint32_t count, float inv_dt2,
-                                                             const uint32_t* __restrict__ done) {
-    if (done && *done) return;
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, k = t / kContactLanes;
-    if (k >= count) return;   // a particle's lanes leave together
-    const OItem it = d.oitems[begin + k];
-    if (d.frozen && d.frozen[d.scene_of[it.v]]) return;
-    rigid::solve_oitem<true, 1, kContactLanes>(d, it, inv_dt2, 0, nullptr, t % kContactLanes);
 }
 
 // Resident solve of oriented particles: one workgroup runs all iterations of a
@@ -1273,10 +1281,7 @@ void launch_step_begin(hipStream_t s, const DevState& d, float dt, float g) {
 void launch_solve_ocolor(hipStream_t s, const DevState& d, uint32_t begin, uint32_t count, float dt,
                          const uint32_t* done) {
     if (count == 0) return;
-    if (d.dyn_off && count <= kContactItems)
-        hipLaunchKernelGGL(solve_ocontact_kernel, dim3(blocks_for(count * kContactLanes, 256)), dim3(256), 0, s, d,
-                           begin, count, 1.0f / (dt * dt), done);
-    else if (d.dyn_off)
+    if (d.dyn_off)
         hipLaunchKernelGGL(solve_ocolor_kernel<true>, dim3(blocks_for(count, 256)), dim3(256), 0, s, d, begin, count,
                            1.0f / (dt * dt), done);
     else
