@@ -1332,8 +1332,8 @@ void tune_fusion(avbd_ctx* c) {
 // Partition the scenes for the resident solve and put the plan on the device.
 // A scene takes it when every patch fits a workgroup's LDS and, since the
 // patches of a scene have to run at once, there are at most as many as CUs
-// (a single tet mesh up to about 36^3 cells in FP64); otherwise, and with
-// AVBD_FLAG_NO_PERSISTENT or AVBD_FLAG_SEPARATE_CHEBYSHEV, every colour phase is
+// (a single Kuhn cube up to 37^3 cells in FP32, 32^3 in FP64, with damping 32^3 and
+// 30^3); otherwise, and with AVBD_FLAG_NO_PERSISTENT or AVBD_FLAG_SEPARATE_CHEBYSHEV, every colour phase is
 // a launch of its own.
 void setup_resident(avbd_ctx* c) {
     if (c->desc.flags & AVBD_FLAG_NO_PERSISTENT) return;
@@ -1353,9 +1353,9 @@ void setup_resident(avbd_ctx* c) {
     lim.ground = c->d.n_ground != 0;
     lim.max_cluster = (uint32_t)prop.multiProcessorCount;
     lim.lds_bytes = (uint32_t)prop.maxSharedMemoryPerMultiProcessor - 1024u;
-    // a patch below 1000 (about 42 free vertices) costs more in exchange than it
-    // saves in arithmetic: 8^3 and 15^3 steps of 20 iterations take 326 us and 2.27
-    // ms with 1000, 352 us and 2.37 ms with 500
+    // below 1000 (about 30 free vertices) a patch gains little in arithmetic for what it
+    // adds in exchange: 10 steps of 20 iterations at 15^3 take 2.56 ms with 1000 and
+    // 2.46 with 500, 8^3 and 32^3 the same with both
     lim.target = (uint32_t)std::max<uint64_t>(1000, (inc + lim.max_cluster - 1) / lim.max_cluster);
     ResidentPlan plan;
     if (!build_resident(m, c->plan, c->x.data(), lim, plan)) return;

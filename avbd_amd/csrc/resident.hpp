@@ -104,8 +104,8 @@ bool build_resident(const HostModel& m, const ColorPlan& plan, const double* pos
                     ResidentPlan& out);
 
 // Threads of a patch's workgroup: 1024 where one phase has more items than 512
-// threads hold groups of `lanes` (512 scenes: 38.0 -> 34.4 ms; idle wavefronts cost
-// 2.4 -> 3.3 ms at 32^3); FP64 stays at 512, where its registers fit.
+// threads hold groups of `lanes` (512 scenes: 45.2 -> 40.8 ms; where all fit, idle
+// wavefronts cost 2.45 -> 2.71 ms at 32^3); FP64 stays at 512, where its registers fit.
 uint32_t resident_block(const ResidentPlan& plan, uint32_t colors, const ResidentLimits& lim, uint32_t lanes);
 
 // What a launch runs: check intervals of `every` iterations until the scene has

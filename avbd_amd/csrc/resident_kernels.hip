@@ -20,13 +20,15 @@
 // three incidences (2,400 cycles for wavefront 0 in FP64 at 8 lanes: nine
 // positions and five constants each, by all wavefronts of the CU), their sum over
 // the lanes and the 3x3 solve (600), sending (1,000), then waiting for the
-// neighbours' words (2,100); 4 times per iteration.  Loading the patch and the
-// handshake take 45,000 cycles per launch, a residual check 17,000.
+// neighbours' words (2,100); 4 times per iteration.  Wavefronts wait two thirds of
+// their cycles; the LDS pipe is active in 20 % of the CU's and a quarter of that
+// is bank conflicts.  Loading the patch and the handshake take 45,000 cycles per
+// launch, a residual check 17,000.
 // One launch per phase before -> now: FP64 32^3 to a residual target 36.6 ->
 // 14.4 us per iteration, checks every 10 included (18.8 with one launch per
-// check); 64 FP64 cubes 48.5 -> 25.4 ms; FP32 32^3 step of 10 iterations 365 ->
-// 240 us (then bound by the broad phase beside it), 15^3 of 20 440 -> 237 us, 512
-// cubes of 4 to 16 cells 49.1 -> 33.9 ms per 10 steps with the read-back.
+// check); 64 FP64 cubes 48.5 -> 27.3 ms; FP32 32^3 step of 10 iterations 365 ->
+// 215 us, 15^3 of 20 430 -> 242 us, 512 cubes of 4 to 16 cells 49.4 -> 39.7 ms per 10
+// steps with the read-back.
 //
 // Exchange: every 32-bit piece of a position travels in an 8-byte word next
 // to a 32-bit tag (the number of the exchange), written and read with relaxed
@@ -56,7 +58,7 @@
 // switched out.
 //
 // The arithmetic of an item is that of the per-phase kernels (tet_device.hpp:
-// L lanes per vertex, the same incidence order and butterfly sums), so results
+// L lanes per vertex, the same incidence order and lane sums), so results
 // do not depend on the partition and equal the per-phase kernels' bit for bit
 // at the same L.
 #include "resident.hpp"

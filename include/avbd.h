@@ -113,7 +113,7 @@ typedef struct {
     uint32_t flags;
     int32_t device;                /* HIP device ordinal */
     uint32_t lanes_per_vertex;     /* 4, 8, 16 or 32, or 0 = 8 to 32 by the size of the largest colour,
-                                      precision and damping of the context.  The lanes fix the order of a
+                                      ground records, precision and damping of the context.  The lanes fix the order of a
                                       vertex's sum: give them where a scene in a batch and the same scene
                                       in a context of its own have to agree bit for bit */
     uint32_t block_size;           /* 0 = autotuned; else 64..1024, multiple of 64 */
