@@ -591,7 +591,7 @@ bool uses_resident(const avbd_ctx* c) { return c->resident && (!c->dynamic || dy
 // Patches that wait for each other have to run at once, so two resident launches
 // that together do not fit the device must not start side by side: each could
 // hold a part of it and wait for the rest (three 20^3 FP64 contexts on three
-// threads took 125 us per iteration, most of it in clusters that gave up; 11 in
+// threads took 125 us per iteration, most of it in clusters that gave up; 12 in
 // turn).  Contexts launch under the lock of their device and one that would not fit
 // beside those in flight first waits, on its stream, until they have ended.  A
 // context that is alone pays for the lock only.
@@ -1149,16 +1149,18 @@ void detect_round(avbd_ctx* c) {
 // sum and with it the roundings of a step, so they follow from the scene alone
 // (timing them chose 8 or 16 by chance at 28^3 cells, and a context rebuilt from a
 // checkpoint could go on with other roundings), and every path of the context uses
-// the same: resident, per phase, timed, warm start.  The lines lie where timing
-// the colour phases changed its choice: undamped FP32 32 lanes up to 22^3 cells
-// (3,042 items in the largest colour) and 8 from 3,479 (16 cubes) and 24^3 (3,907) on; FP64
-// 32 up to 14^3 (844), 8 from 16^3 (1,229) on; damped, whose incidence is twice the
-// work, 32 up to 24^3 (3,907), 16 at 32^3 (8,985); without ground records 32 up to
-// 23^3 (3,312), 16 at 24^3 (3,750) and 28^3 (5,887), 8 from 30^3 (7,208) on.  The resident solve agrees but
-// for a few per cent between the lines; step of 10 iterations at 8 / 16 / 32 lanes in
-// us: FP32 15^3 151 / 134 / 125, 22^3 160 / 142 / 137, 28^3 168 / 159 / 170, 32^3 189 /
-// 179 / 205; FP64 14^3 132 / 123 / 125, 32^3 177 / 192 / 251; damped 16^3 180 / 155 /
-// 137, 24^3 192 / 170 / 165, 32^3 226 / 217 / 236.
+// the same: resident, per phase, timed, warm start.  The lines lie where timing the
+// colour phases changed its choice, in items of the largest colour:
+//   FP32 on the ground    32 up to 22^3 cells (3,042), 8 from 23^3 (3,456) on
+//   FP32 without ground   32 up to 23^3 (3,312), 16 at 24^3 (3,750) and 28^3 (5,887),
+//                         8 from 30^3 (7,208) on
+//   FP64                  32 up to 14^3 (844), 8 from 16^3 (1,229) on
+//   damped (twice the work of an incidence)
+//                         32 up to 24^3 (3,907), 16 at 32^3 (8,985)
+// The resident solve agrees but for a few per cent between the lines; step of 10
+// iterations at 8 / 16 / 32 lanes in us: FP32 15^3 151 / 134 / 125, 22^3 160 / 142 / 137,
+// 28^3 168 / 159 / 170, 32^3 189 / 179 / 205; FP64 14^3 132 / 123 / 125, 32^3 177 / 192 /
+// 251; damped 16^3 180 / 155 / 137, 24^3 192 / 170 / 165, 32^3 226 / 217 / 236.
 uint32_t default_lanes(const ColorPlan& plan, bool fp64, bool damping, bool ground) {
     uint32_t most = 0;
     for (uint32_t c = 0; c < plan.num_colors; c++)
@@ -1333,8 +1335,9 @@ void tune_fusion(avbd_ctx* c) {
 // A scene takes it when every patch fits a workgroup's LDS and, since the
 // patches of a scene have to run at once, there are at most as many as CUs
 // (a single Kuhn cube up to 37^3 cells in FP32, 32^3 in FP64, with damping 32^3 and
-// 30^3); otherwise, and with AVBD_FLAG_NO_PERSISTENT or AVBD_FLAG_SEPARATE_CHEBYSHEV, every colour phase is
-// a launch of its own.
+// 30^3).  With a scene that does not, and with AVBD_FLAG_NO_PERSISTENT or
+// AVBD_FLAG_SEPARATE_CHEBYSHEV, every colour phase of the context is a launch of
+// its own.
 void setup_resident(avbd_ctx* c) {
     if (c->desc.flags & AVBD_FLAG_NO_PERSISTENT) return;
     hipDeviceProp_t prop;
@@ -1407,8 +1410,9 @@ void setup_resident(avbd_ctx* c) {
     r.max_cluster = plan.max_cluster;
     r.lanes = c->cfg.lanes;
     r.block = resident_block(plan, c->plan.num_colors, lim, r.lanes);
-    // about 50 ms (0.13 us each): half of what 100 iterations of a large scene take alone (1 ms each
-    // at 32^3), so that waiting for another stream's work costs less than giving up
+    // about 50 ms (0.13 us each): half of what 100 iterations of a large scene take
+    // alone (1 ms each at 32^3), so that waiting for another stream's work costs less
+    // than giving up
     r.gather_polls = 400000u;
     r.alternate = (c->desc.flags & AVBD_FLAG_RESIDENT_ALONE) != 0;
     r.has_ground = lim.ground;
